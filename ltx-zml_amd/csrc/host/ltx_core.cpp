@@ -2,6 +2,8 @@
 // (ltx/scheduler.zig) and the denoising loop that drives a stack of resident
 // blocks (ltx/e2e_denoise.zig:218-336). Everything here is f32, as in the
 // reference; the linear layers use the f32 GEMM kernel with bf16 weights.
+#include <algorithm>
+#include <cstdio>
 #include <cstring>
 #include <vector>
 
@@ -66,6 +68,10 @@ static void sinusoid(ltx_ctx* c, const float* t, int rows, float* out, hipStream
     c->launch("ltx_core_sinusoid", rows, 1, 1, 128, &a, st);
 }
 
+// Timestep rows up to which the conditioning MLPs run on the few-row kernels
+// (eight rows a pass over the weights) instead of the f32 GEMM.
+constexpr int kCoreRows = 32;
+
 // Scratch of the conditioning MLPs for K timestep rows, carved from one
 // context buffer: sin [K+1][256], h [K][D], silu(emb) [K][D], and the prompt
 // branch's own rows.
@@ -73,6 +79,26 @@ static float* core_scratch(ltx_ctx* c, int K) {
     const size_t need = ((size_t)(K + 1) * 256 + (size_t)(3 * K + 4) * LTX_DIM + 64) * sizeof(float);
     if (c->core_ws.bytes < need) c->core_ws.alloc(need);
     return (float*)c->core_ws.p;
+}
+
+// One launch of the layer pair (job 0: the timestep branch's r rows, job 1:
+// the prompt branch's one row, or NULL) on the few-row kernels.
+static void rows_pair(ltx_ctx* c, const ltx_core_weights* cw, bool sin, int r, int wi, const float* a, float* out,
+                      float* act, int pwi, const float* pa, float* pout, float* pact, hipStream_t st) {
+    auto job = [&](int w, const float* in, float* y, float* ya, int rows) {
+        return LtxRowsJob{in, (const uint16_t*)cw->t[w].p, (const float*)cw->t[w + 1].p, y, ya, rows, kCore[w].o};
+    };
+    LtxRowsArgs g{};
+    g.j[0] = job(wi, a, out, act, r);
+    if (pa) g.j[1] = job(pwi, pa, pout, pact, 1);
+    static const int kR[] = {1, 2, 3, 4, 6, 8};
+    int R = 8;
+    for (int i = 5; i >= 0; i--)
+        if (kR[i] >= r) R = kR[i];
+    char name[32];
+    std::snprintf(name, sizeof(name), sin ? "ltx_core_rows_sin_%d" : "ltx_core_rows_%d", R);
+    // two workgroups a CU while their rows (16 KB each, and the prompt's) fit its LDS
+    c->launch(name, c->num_cu * (R <= 4 ? 2 : 1), 1, 1, 512, &g, st);
 }
 
 // ts9r, embedded_timestep and pts2r (ltx/core_parts.zig:112-141).
@@ -86,6 +112,20 @@ static void conditioning(ltx_ctx* c, const ltx_core_weights* cw, const float* t,
     float* ph = se + (size_t)K * LTX_DIM;             // [1][D]
     float* pe = ph + LTX_DIM;                         // [1][D]
     float* pse = pe + LTX_DIM;                        // [1][D]
+    if (K <= kCoreRows) {
+        for (int r0 = 0; r0 < K; r0 += 8) {
+            const int r = std::min(8, K - r0);
+            const bool p = r0 == 0;  // the prompt branch goes with the first rows
+            const size_t o = (size_t)r0 * LTX_DIM;
+            rows_pair(c, cw, true, r, LTX_C_ADA_L1_W, t + r0, nullptr, h + o, LTX_C_PADA_L1_W, p ? sigma_dev : nullptr,
+                      nullptr, ph, st);
+            rows_pair(c, cw, false, r, LTX_C_ADA_L2_W, h + o, emb + o, se + o, LTX_C_PADA_L2_W, p ? ph : nullptr,
+                      nullptr, pse, st);
+            rows_pair(c, cw, false, r, LTX_C_ADA_OUT_W, se + o, tstab + 9 * o, nullptr, LTX_C_PADA_OUT_W,
+                      p ? pse : nullptr, pts2, nullptr, st);
+        }
+        return;
+    }
     // emb = lin2(silu(lin1(sinusoid(t))));  ts9 = lin_out(silu(emb))
     sinusoid(c, t, K, sn, st);
     lin32(c, cw, LTX_C_ADA_L1_W, sn, K, h, st);

@@ -1,18 +1,24 @@
 // Kernels of the parts around the blocks (ltx/core_parts.zig) and of the
-// distilled scheduler (ltx/scheduler.zig). All f32; the linear layers run on
-// the f32 GEMM (k_f32.hip).
+// distilled scheduler (ltx/scheduler.zig). All f32; the linear layers of a few
+// rows run here, the others on the f32 GEMM (k_f32.hip).
 #include "ltx_device.h"
 
 // DDPM/PixArt sinusoid of t * 1000, cos half first, divisor HALF = 128
 // (ltx/core_parts.zig:36-49): freq[k] = exp(k * (-ln(1e4) / 128)) in f32,
 // arg = (t * 1000) * freq, out = [cos(arg) | sin(arg)].
+__device__ __forceinline__ void core_sinusoid(float t, int k, float& c, float& s) {
+    const float freq = expf((float)k * (-9.210340371976184f / 128.0f));
+    const float arg = (t * 1000.0f) * freq;
+    c = cosf(arg);
+    s = sinf(arg);
+}
 extern "C" __global__ void __launch_bounds__(128) ltx_core_sinusoid(const LtxSinArgs a) {
     const int r = blockIdx.x, k = threadIdx.x;
     if (r >= a.rows) return;
-    const float freq = expf((float)k * (-9.210340371976184f / 128.0f));
-    const float arg = (a.t[r] * 1000.0f) * freq;
-    a.out[(size_t)r * 256 + k] = cosf(arg);
-    a.out[(size_t)r * 256 + 128 + k] = sinf(arg);
+    float c, s;
+    core_sinusoid(a.t[r], k, c, s);
+    a.out[(size_t)r * 256 + k] = c;
+    a.out[(size_t)r * 256 + 128 + k] = s;
 }
 
 // y = x * sigmoid(x) (ltx/core_parts.zig:22-24), elementwise.
@@ -22,6 +28,165 @@ extern "C" __global__ void __launch_bounds__(256) ltx_core_silu(const LtxEltArgs
     const float x = a.x[i];
     a.y[i] = x * (1.0f / (1.0f + expf(-x)));
 }
+
+// Linear layers of up to R rows in f32 on the VALU: y[r][n] = a[r] . w[n] +
+// bias[n], w bf16. Bound by the weights' bytes: a weight is read once, for all
+// rows, 16 bytes a lane. A wave takes two consecutive columns n at a time and
+// all of K = 4,096 (eight chunks of 512, 8 weights a lane and column); each
+// chunk's registers are refilled for the wave's next columns as soon as they
+// are used, so 16 KB a wave are in flight. The rows lie in LDS, the 8 values of
+// a lane as two float4 512 floats' half apart (a lane stride of 16 B: no bank
+// conflicts). The grid is persistent and runs two layers of the same K: the
+// timestep branch (job 0, up to R rows) and the prompt branch (job 1, one
+// row). Two workgroups a CU up to 4 rows (128 registers a lane): the out
+// layers at 3 rows, 369 MB of weights, take 70 us = 5.3 TB/s; with three waves
+// a SIMD and the LDS reads lifted out of the loop, the conditioning took 162
+// instead of 94 us.
+template <int R>
+struct RowsDot {
+    // acc[r][c] += the chunk's products of rows r and columns c
+    static __device__ __forceinline__ void fma8(const float* sa, const u32x4 (&w)[2], float (&acc)[R][2]) {
+        float wf[2][8];
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                wf[c][2 * e] = __builtin_bit_cast(float, w[c][e] << 16);
+                wf[c][2 * e + 1] = __builtin_bit_cast(float, w[c][e] & 0xffff0000u);
+            }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const f32x4 a0 = *(const f32x4*)(sa + r * LTX_D), a1 = *(const f32x4*)(sa + r * LTX_D + 256);
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    acc[r][c] = __builtin_fmaf(a0[e], wf[c][e], acc[r][c]);
+                    acc[r][c] = __builtin_fmaf(a1[e], wf[c][4 + e], acc[r][c]);
+                }
+        }
+    }
+};
+
+// the layer's outputs from the finished dot product of row r, column n
+__device__ __forceinline__ void rows_store(const LtxRowsJob& j, int r, int n, float v) {
+    if (r >= j.rows || n >= j.N) return;
+    v += j.bias[n];
+    const size_t o = (size_t)r * j.N + n;
+    if (j.out) j.out[o] = v;
+    if (j.act) j.act[o] = v * (1.0f / (1.0f + expf(-v)));
+}
+
+template <int R>
+__device__ __forceinline__ void rows_job(const LtxRowsJob& j, const float* sa, int g, int step) {
+    const int lane = threadIdx.x & 63, ng = j.N / 2;
+    if (g >= ng) return;
+    const uint16_t* w = j.w + 8 * lane;
+    u32x4 buf[8][2];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) buf[k][c] = *(const u32x4*)(w + (size_t)(2 * g + c) * LTX_D + 512 * k);
+    for (; g < ng; g += step) {
+        const int gn = min(g + step, ng - 1);  // past the end: the last columns again
+        // the lane's place in the rows, opaque: or the compiler lifts the LDS
+        // reads of all chunks out of this loop and spills them (288 B a lane
+        // at 3 rows, 1,780 B at 8)
+        int lo = 4 * lane;
+        asm volatile("" : "+v"(lo));
+        float acc[R][2];
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r][0] = acc[r][1] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            RowsDot<R>::fma8(sa + 512 * k + lo, buf[k], acc);
+#pragma unroll
+            for (int c = 0; c < 2; c++) buf[k][c] = *(const u32x4*)(w + (size_t)(2 * gn + c) * LTX_D + 512 * k);
+        }
+        float mine = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                float v = acc[r][c];
+                for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+                if (lane == 2 * r + c) mine = v;
+            }
+        if (lane < 2 * R) rows_store(j, lane >> 1, 2 * g + (lane & 1), mine);
+    }
+}
+
+template <int R>
+__device__ __forceinline__ void rows_body(const LtxRowsArgs& a) {
+    __shared__ __attribute__((aligned(16))) float sa[(R + 1) * LTX_D];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < (R + 1) * (LTX_D / 4); i += 512) {
+        const int r = i / (LTX_D / 4), q = i % (LTX_D / 4);  // float4 q of row r
+        const LtxRowsJob& j = a.j[r == R];
+        const int rr = r == R ? 0 : r;
+        const f32x4 v = rr < j.rows ? *(const f32x4*)(j.a + (size_t)rr * LTX_D + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+        *(f32x4*)(sa + r * LTX_D + (q >> 7) * 512 + (q & 1) * 256 + ((q >> 1) & 63) * 4) = v;
+    }
+    __syncthreads();
+    // columns pairs of job 0, then of job 1, dealt to the grid's waves in turn
+    const int nw = gridDim.x * 8, g0 = a.j[0].N / 2;
+    int g = blockIdx.x * 8 + (tid >> 6);
+    rows_job<R>(a.j[0], sa, g, nw);
+    if (g < g0) g += (g0 - g + nw - 1) / nw * nw;
+    rows_job<1>(a.j[1], sa + R * LTX_D, g - g0, nw);
+}
+
+// The first layers (K = 256) on the sinusoid of t * 1000, which each workgroup
+// forms for itself (as ltx_core_sinusoid). A half-wave takes one column.
+template <int R>
+__device__ __forceinline__ void rows_sin_body(const LtxRowsArgs& a) {
+    __shared__ __attribute__((aligned(16))) float sa[(R + 1) * 256];
+    const int tid = threadIdx.x;
+    for (int i = tid; i < (R + 1) * 128; i += 512) {
+        const int r = i >> 7, k = i & 127;
+        const LtxRowsJob& j = a.j[r == R];
+        const int rr = r == R ? 0 : r;
+        float c = 0.f, s = 0.f;
+        if (rr < j.rows) core_sinusoid(j.a[rr], k, c, s);
+        sa[r * 256 + k] = c;
+        sa[r * 256 + 128 + k] = s;
+    }
+    __syncthreads();
+    const int l = tid & 31, n0 = a.j[0].N, nt = n0 + a.j[1].N;
+    for (int n = (blockIdx.x * 512 + tid) >> 5; n < nt; n += gridDim.x * 16) {
+        const bool one = n >= n0;  // job 1: its single row
+        const LtxRowsJob& j = a.j[one];
+        const int nn = one ? n - n0 : n;
+        const u32x4 w = *(const u32x4*)(j.w + (size_t)nn * 256 + 8 * l);
+        float wf[8];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            wf[2 * e] = __builtin_bit_cast(float, w[e] << 16);
+            wf[2 * e + 1] = __builtin_bit_cast(float, w[e] & 0xffff0000u);
+        }
+        const int nr = one ? 1 : R;
+        for (int r = 0; r < nr; r++) {
+            const float* p = sa + (one ? R : r) * 256 + 8 * l;
+            float v = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) v = __builtin_fmaf(p[e], wf[e], v);
+            for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 32);
+            if (l == 0) rows_store(j, r, nn, v);
+        }
+    }
+}
+
+#define CORE_ROWS_KERNEL(R)                                                                                            \
+    extern "C" __global__ void __launch_bounds__(512, R <= 4 ? 4 : 2) ltx_core_rows_##R(const LtxRowsArgs a) {        \
+        rows_body<R>(a);                                                                                              \
+    }                                                                                                                  \
+    extern "C" __global__ void __launch_bounds__(512) ltx_core_rows_sin_##R(const LtxRowsArgs a) { rows_sin_body<R>(a); }
+CORE_ROWS_KERNEL(1)
+CORE_ROWS_KERNEL(2)
+CORE_ROWS_KERNEL(3)
+CORE_ROWS_KERNEL(4)
+CORE_ROWS_KERNEL(6)
+CORE_ROWS_KERNEL(8)
 
 // Output tail norm (ltx/core_parts.zig:26-35, 143-147): mean-subtracting
 // LayerNorm without weight, biased variance, eps 1e-6, then

@@ -251,6 +251,20 @@ typedef struct {
     size_t n;
 } LtxEltArgs;
 
+// Linear layers of a few rows: y[r][n] = a[r] . w[n] + bias[n], two layers of
+// the same K in one launch (job 1 has one row, or N = 0: none).
+typedef struct {
+    const float* a;     // [rows][K], or [rows] timesteps (ltx_core_rows_sin_*)
+    const uint16_t* w;  // [N][K] bf16
+    const float* bias;  // [N]
+    float* out;         // [rows][N] or NULL
+    float* act;         // [rows][N] silu(y) or NULL
+    int rows, N;        // N even
+} LtxRowsJob;
+typedef struct {
+    LtxRowsJob j[2];
+} LtxRowsArgs;
+
 typedef struct {
     const float* x;       // [T][D]
     const float* fsst;    // [2][D] (shift row, scale row)

@@ -110,6 +110,23 @@ def test_conditioning(ctx, core_np, core_dev, sigma, striped):
     assert all(v <= 1e-4 for v in r.values()), r
 
 
+@pytest.mark.parametrize("K", [1, 2, 5, 8, 9, 32, 33])
+def test_conditioning_rows(ctx, core_np, core_dev, K):
+    """Row counts at both ends of the few-row kernels (1 to 8 rows a pass, up
+    to four passes) and one past them (the f32 GEMM)."""
+    say(f"core conditioning rows K={K}")
+    t = np.linspace(0.0, 0.003, K + 1, dtype=np.float32)[1:]
+    tstab = torch.full((K, 9, 4096), float("nan"), device="cuda")
+    emb = torch.full((K, 4096), float("nan"), device="cuda")
+    pts2 = torch.full((2, 4096), float("nan"), device="cuda")
+    ctx.conditioning(core_dev, dev(t), dev(np.array([0.002], np.float32)), tstab, emb, pts2)
+    # phases up to 3 rad, so the sinusoids agree to a few ulp; then three f32
+    # layers whose sums are at most 4,096 terms long: 1e-5
+    assert oracle.rel_rms(host(tstab), oracle.core_ts9r(core_np, t)) <= 1e-5
+    assert oracle.rel_rms(host(emb), oracle.core_emb(core_np, t)) <= 1e-5
+    assert oracle.rel_rms(host(pts2), oracle.core_pts2r(core_np, 0.002)) <= 1e-5
+
+
 @pytest.mark.parametrize("T", [1024, 1000])
 def test_patchify_and_tail(ctx, core_np, core_dev, T):
     say(f"core patchify + tail T={T}")
