@@ -73,6 +73,22 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
     return q8 && M < 4096 && K <= 4096 && gemm_ksplit(c->num_cu, M, N, K) > 1;
 }
 
+// Whether the f32 GEMM on bf16 MFMAs takes an M x N x K product (shape and
+// 31-bit buffer offsets; gemm32 checks the alignment of the operands). It does
+// wherever it can: at 1,024 rows it takes a third of the f32 MFMA kernel's time
+// and below that its split-K fills the chip where the other has N / 128
+// workgroups a row tile.
+bool f3_shape(const ltx_ctx* c, int M, int N, int K) {
+    return c->gemm_f3 && M > 0 && N % 128 == 0 && K % 128 == 0 && (uint64_t)M * K * 2 < (1ull << 31) &&
+           (uint64_t)N * K * 2 < (1ull << 31);
+}
+// Its scratch: the three planes of A, and the split-K partial sums (0: no split).
+size_t f3_planes_bytes(int M, int K) { return 3 * al((size_t)M * K * 2); }
+size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K) {
+    const int s = gemm_ksplit(c->num_cu, M, N, K, 128, 128);
+    return s > 1 ? (size_t)s * M * N * 4 : 0;
+}
+
 // The small-T schedule of the block forward (side stream from the first
 // RMSNorm + modulate on).
 static bool side_early(const ltx_ctx* c, size_t T) {
@@ -127,9 +143,10 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
 
 struct Ws32 {
     void *n_msa, *q, *k, *v, *glog1, *o1, *x_sa, *attn_in, *q2, *enc, *k2, *v2, *glog2, *o2, *x_ca, *ff_in, *h;
+    void *planes, *part;  // the f3 GEMMs' split of the current A (three bf16 planes) and split-K partial sums
 };
 
-static void carve32(Carve& c, Ws32& w, size_t T, size_t S) {
+static void carve32(Carve& c, Ws32& w, size_t T, size_t S, const ltx_ctx* ctx) {
     const size_t D = LTX_D;
     w.n_msa = c.take(T * D * 4);
     w.q = c.take(T * D * 4);
@@ -148,13 +165,24 @@ static void carve32(Carve& c, Ws32& w, size_t T, size_t S) {
     w.x_ca = c.take(T * D * 4);
     w.ff_in = c.take(T * D * 4);
     w.h = c.take(T * LTX_FF * 4);
+    w.planes = w.part = nullptr;
+    size_t planes = 0, part = 0;
+    const int shapes[4][3] = {{(int)T, LTX_D, LTX_D}, {(int)S, LTX_D, LTX_D}, {(int)T, LTX_FF, LTX_D},
+                              {(int)T, LTX_D, LTX_FF}};
+    for (const auto& sh : shapes) {
+        if (!f3_shape(ctx, sh[0], sh[1], sh[2])) continue;
+        planes = std::max(planes, f3_planes_bytes(sh[0], sh[2]));
+        part = std::max(part, f3_part_bytes(ctx, sh[0], sh[1], sh[2]));
+    }
+    if (planes) w.planes = c.take(planes);
+    if (part) w.part = c.take(part);
 }
 
 static void ensure_ws(ltx_ctx* c, size_t T, size_t S, int mode) {
     Carve cv{nullptr, 0, 0, true};
     if (mode == LTX_MODE_F32) {
         Ws32 w;
-        carve32(cv, w, T, S);
+        carve32(cv, w, T, S, c);
     } else {
         Ws16 w;
         carve16(cv, w, T, S, c, mode);
@@ -407,23 +435,77 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
     c->launch(name, a.q_tiles * LTX_H, 1, 1, 512, &a, st, label);
 }
 
+// Splits A [M][K] into the three bf16 planes at `planes` (f3_planes_bytes).
+static void split3(ltx_ctx* c, const float* A, int M, int K, void* planes, hipStream_t st) {
+    const size_t n = (size_t)M * K, ps = al(n * 2);
+    char* p = (char*)planes;
+    LtxSplit3Args a{A, (uint16_t*)p, (uint16_t*)(p + ps), (uint16_t*)(p + 2 * ps), n};
+    c->launch("ltx_split3", (unsigned)((n / 8 + 255) / 256), 1, 1, 256, &a, st, "split3");
+}
+
 // f32-mode GEMM over rows [r0, r0 + N) of a (possibly fused) projection.
+// planes: A's split by split3, or NULL (the f32 MFMA kernel); part: split-K
+// partial sums (f3_part_bytes) or NULL.
 static void gemm32(ltx_ctx* c, const LtxProj& p, int r0, int N, const float* A, int M, float* out, int epi,
-                   const float* resid, LtxAda ada, int igate, int gelu, hipStream_t st,
-                   const char* label = nullptr) {
+                   const float* resid, LtxAda ada, int igate, int gelu, hipStream_t st, const char* label = nullptr,
+                   const void* planes = nullptr, void* part = nullptr) {
+    const size_t G = p.K / LTX_GROUP;
+    const void *wb, *ws = nullptr;
+    if (p.q8) {
+        wb = (const int8_t*)p.q.p + (size_t)r0 * p.K;
+        ws = (const char*)p.s.p + (size_t)r0 * G * (p.scale_f16 ? 2 : 4);
+    } else {
+        wb = (const uint16_t*)p.w_bf16.p + (size_t)r0 * p.K;
+    }
+    const float* bias = p.bias.p ? (const float*)p.bias.p + r0 : nullptr;
+    const uint32_t qxor = p.qflip ? 0u : 0x80808080u;
+    auto al16 = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
+    if (planes && f3_shape(c, M, N, p.K) && al16(wb) && al16(out) && al16(bias) && al16(resid) && al16(ada.tstab) &&
+        al16(ada.sst)) {
+        LtxGemmF3Args f{};
+        LtxGemmArgs& g = f.g;
+        const size_t ps = al((size_t)M * p.K * 2);
+        g.a = planes;
+        f.a1 = (const char*)planes + ps;
+        f.a2 = (const char*)planes + 2 * ps;
+        g.b = wb;
+        g.scales = ws;
+        g.bias = bias;
+        g.out = out;
+        g.resid = resid;
+        g.ada = ada;
+        g.M = M;
+        g.N = N;
+        g.K = p.K;
+        g.lda = p.K;
+        g.ldo = N;
+        g.igate = igate;
+        g.gelu = gelu;
+        g.out_f32 = 1;
+        g.qxor = qxor;
+        g.tiles_m = (M + 127) / 128;
+        g.tiles_n = N / 128;
+        g.ksplit = part ? gemm_ksplit(c->num_cu, M, N, p.K, 128, 128) : 1;
+        g.part = (float*)part;
+        const char* es = epi == LTX_EPI_RESID_GATE ? "resid" : "store";
+        char name[48];
+        std::snprintf(name, sizeof(name), "ltx_gemm_f3_%s_%s%s", !p.q8 ? "w16" : p.scale_f16 ? "i8f16" : "i8f32", es,
+                      epi == LTX_EPI_STORE && gelu ? "_gelu" : "");
+        const int nitems = g.tiles_m * g.tiles_n * g.ksplit;
+        c->launch(name, std::min(nitems, c->num_cu), 1, 1, 256, &f, st, label);
+        if (g.ksplit > 1) {
+            std::snprintf(name, sizeof(name), "ltx_gemm_reduce_bf16_%s", es);
+            c->launch(name, N / 64, (M + 63) / 64, 1, 256, &g, st, "splitk_reduce");
+        }
+        return;
+    }
     LtxGemm32Args g{};
     g.a = A;
-    const size_t G = p.K / LTX_GROUP;
-    if (p.q8) {
-        g.bkind = p.scale_f16 ? 1 : 0;
-        g.qxor = p.qflip ? 0u : 0x80808080u;
-        g.b = (const int8_t*)p.q.p + (size_t)r0 * p.K;
-        g.scales = (const char*)p.s.p + (size_t)r0 * G * (p.scale_f16 ? 2 : 4);
-    } else {
-        g.bkind = 2;
-        g.b = (const uint16_t*)p.w_bf16.p + (size_t)r0 * p.K;
-    }
-    g.bias = p.bias.p ? (const float*)p.bias.p + r0 : nullptr;
+    g.b = wb;
+    g.scales = ws;
+    g.bkind = !p.q8 ? 2 : p.scale_f16 ? 1 : 0;
+    g.qxor = qxor;
+    g.bias = bias;
     g.out = out;
     g.resid = resid;
     g.ada = ada;
@@ -479,34 +561,47 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
 
     if (mode == LTX_MODE_F32) {
         Ws32 b;
-        carve32(cv, b, T, S);
+        carve32(cv, b, T, S, c);
         // self-attention (ltx/block.zig:546-547, qAttn1 520-530)
         norm_mod(c, mode, x, b.n_msa, ada, T, 0, 1, st,
              mode == LTX_MODE_F16 ? (const unsigned long long*)w->f16_over.p : nullptr);
-        gemm32(c, w->qkv1, 0, LTX_D, (const float*)b.n_msa, T, (float*)b.q, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1");
-        gemm32(c, w->qkv1, LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.k, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1");
-        gemm32(c, w->qkv1, 2 * LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.v, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1");
+        // the GEMMs' A operands are split into bf16 planes as they are formed
+        const void* pl = nullptr;
+        auto split = [&](const void* A, int rows, int K) {
+            pl = b.planes;
+            if (pl) split3(c, (const float*)A, rows, K, b.planes, st);
+        };
+        split(b.n_msa, T, LTX_D);
+        gemm32(c, w->qkv1, 0, LTX_D, (const float*)b.n_msa, T, (float*)b.q, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
+        gemm32(c, w->qkv1, LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.k, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
+        gemm32(c, w->qkv1, 2 * LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.v, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
         gemm32(c, w->g1, 0, LTX_H, (const float*)b.n_msa, T, (float*)b.glog1, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "ltx_gate:1");
         qknorm32(c, (float*)b.q, w->qn1.p, cs, sn, T, st);
         qknorm32(c, (float*)b.k, w->kn1.p, cs, sn, T, st);
         attn32(c, (const float*)b.q, (const float*)b.k, (const float*)b.v, (const float*)b.glog1, (float*)b.o1, T, T, st, "attn:self");
-        gemm32(c, w->o1, 0, LTX_D, (const float*)b.o1, T, (float*)b.x_sa, LTX_EPI_RESID_GATE, x, ada, 2, 0, st, "gemm:o1");
+        split(b.o1, T, LTX_D);
+        gemm32(c, w->o1, 0, LTX_D, (const float*)b.o1, T, (float*)b.x_sa, LTX_EPI_RESID_GATE, x, ada, 2, 0, st, "gemm:o1", pl, b.part);
         // cross-attention (ltx/block.zig:548-568)
         norm_mod(c, mode, (const float*)b.x_sa, b.attn_in, ada, T, 6, 7, st);
         LtxEncArgs ea{ctxv, (const float*)w->psst.p, pts2, b.enc, S};
         c->launch("ltx_enc_f32", S, 1, 1, 256, &ea, st);
-        gemm32(c, w->q2, 0, LTX_D, (const float*)b.attn_in, T, (float*)b.q2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:q2");
-        gemm32(c, w->kv2, 0, LTX_D, (const float*)b.enc, S, (float*)b.k2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2");
-        gemm32(c, w->kv2, LTX_D, LTX_D, (const float*)b.enc, S, (float*)b.v2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2");
+        split(b.attn_in, T, LTX_D);
+        gemm32(c, w->q2, 0, LTX_D, (const float*)b.attn_in, T, (float*)b.q2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:q2", pl, b.part);
+        split(b.enc, S, LTX_D);
+        gemm32(c, w->kv2, 0, LTX_D, (const float*)b.enc, S, (float*)b.k2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
+        gemm32(c, w->kv2, LTX_D, LTX_D, (const float*)b.enc, S, (float*)b.v2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
         gemm32(c, w->g2, 0, LTX_H, (const float*)b.attn_in, T, (float*)b.glog2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "ltx_gate:2");
         qknorm32(c, (float*)b.q2, w->qn2.p, nullptr, nullptr, T, st);
         qknorm32(c, (float*)b.k2, w->kn2.p, nullptr, nullptr, S, st);
         attn32(c, (const float*)b.q2, (const float*)b.k2, (const float*)b.v2, (const float*)b.glog2, (float*)b.o2, T, S, st, "attn:cross");
-        gemm32(c, w->o2, 0, LTX_D, (const float*)b.o2, T, (float*)b.x_ca, LTX_EPI_RESID_GATE, (const float*)b.x_sa, ada, 8, 0, st, "gemm:o2");
+        split(b.o2, T, LTX_D);
+        gemm32(c, w->o2, 0, LTX_D, (const float*)b.o2, T, (float*)b.x_ca, LTX_EPI_RESID_GATE, (const float*)b.x_sa, ada, 8, 0, st, "gemm:o2", pl, b.part);
         // feed-forward (ltx/block.zig:569-573)
         norm_mod(c, mode, (const float*)b.x_ca, b.ff_in, ada, T, 3, 4, st);
-        gemm32(c, w->f1, 0, LTX_FF, (const float*)b.ff_in, T, (float*)b.h, LTX_EPI_STORE, nullptr, ada, 0, 1, st, "gemm:ff1");
-        gemm32(c, w->f2, 0, LTX_D, (const float*)b.h, T, y, LTX_EPI_RESID_GATE, (const float*)b.x_ca, ada, 5, 0, st, "gemm:ff2");
+        split(b.ff_in, T, LTX_D);
+        gemm32(c, w->f1, 0, LTX_FF, (const float*)b.ff_in, T, (float*)b.h, LTX_EPI_STORE, nullptr, ada, 0, 1, st, "gemm:ff1", pl, b.part);
+        split(b.h, T, LTX_FF);
+        gemm32(c, w->f2, 0, LTX_D, (const float*)b.h, T, y, LTX_EPI_RESID_GATE, (const float*)b.x_ca, ada, 5, 0, st, "gemm:ff2", pl, b.part);
         set_stage(c, LTX_ST_NORM_MSA, b.n_msa, TD * 4);
         set_stage(c, LTX_ST_Q1, b.q, TD * 4);
         set_stage(c, LTX_ST_K1, b.k, TD * 4);
@@ -718,7 +813,10 @@ void linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, i
         if (mode == LTX_MODE_F32) {
             if (!out_f32) throw Error("mode F32 writes f32 output");
             LtxAda ada{};
-            gemm32(c, p, 0, N, (const float*)a, M, (float*)y, LTX_EPI_STORE, nullptr, ada, 0, gelu, st);
+            const bool f3 = sc.planes && ((uintptr_t)a & 15) == 0;
+            if (f3) split3(c, (const float*)a, M, K, sc.planes, st);
+            gemm32(c, p, 0, N, (const float*)a, M, (float*)y, LTX_EPI_STORE, nullptr, ada, 0, gelu, st, nullptr,
+                   f3 ? sc.planes : nullptr, sc.part);
         } else {
             if (linear_q8_needs_scratch(c, N, K, mode)) {
                 if (!sc.q || !sc.pairs) throw Error("linear_q8: no scratch");
@@ -872,6 +970,21 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         ltx::check_linear_q8(M, N, K, mode);  // before N and K size the scratch
         HIPC(hipSetDevice(c->device));
         ltx::LinearScratch sc{};
+        hipStream_t st = (hipStream_t)stream;
+        // Mode F32 splits A into planes in a buffer of the context. A call on
+        // another stream than the last waits for that one's use of it; a call
+        // being captured (whose replays nothing could order, and which may not
+        // allocate) takes the f32 MFMA kernel, which needs none.
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        const bool f3 = mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K) &&
+                        hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
+        if (f3) {
+            const size_t np = ltx::f3_planes_bytes(M, K), need = np + ltx::f3_part_bytes(c, M, N, K);
+            if (c->op_f3.bytes < need) c->op_f3.alloc(need);  // (frees the old one after the device has finished with it)
+            sc.planes = c->op_f3.p;
+            sc.part = need > np ? (char*)c->op_f3.p + np : nullptr;
+            if (c->op_f3_used && c->op_f3_stream != st) HIPC(hipStreamWaitEvent(st, c->op_f3_ev, 0));
+        }
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
             // scratch owned by the context, grown as needed
             const size_t nq = (size_t)N * K, np = (size_t)N * (K / LTX_GROUP) * 4;
@@ -884,7 +997,12 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
                 sc.w16 = c->op_w16.p;
             }
         }
-        ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, (hipStream_t)stream);
+        ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, st);
+        if (f3) {
+            HIPC(hipEventRecord(c->op_f3_ev, st));
+            c->op_f3_stream = st;
+            c->op_f3_used = true;
+        }
     })
 }
 

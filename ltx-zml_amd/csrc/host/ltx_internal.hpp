@@ -96,6 +96,9 @@ struct ltx_ctx {
     // where the 256 x 256 kernels would split K over at most 4,096 (M below
     // 4,096), 2 wherever the shape allows (tests)
     int gemm_s4 = 1;
+    // mode F32's GEMM on bf16 MFMAs (three exact planes of A) where the shape
+    // allows, or the f32 MFMA kernel everywhere (false: tests)
+    bool gemm_f3 = true;
     int num_cu = 256;             // compute units: the persistent GEMM's grid bound
     bool gemm_persistent = true;  // LDS-DMA GEMM: at most one workgroup per CU, looping over tiles
     bool attn_pp = true;
@@ -121,6 +124,12 @@ struct ltx_ctx {
     ltx::DevBuf op_pairs;  // scale pairs of the last ltx_op_linear_q8 call (f16 scales)
     ltx::DevBuf op_q;      // its weights as bytes q + 128
     ltx::DevBuf op_w16;    // and dequantised to 16 bits (four-wave GEMM)
+    // ltx_op_linear_q8 in mode F32: the planes and partial sums of the last
+    // call, the event after that call and the stream it ran on
+    ltx::DevBuf op_f3;
+    hipEvent_t op_f3_ev = nullptr;
+    hipStream_t op_f3_stream = nullptr;
+    bool op_f3_used = false;
     ltx::DevBuf blob_stage;  // device copy of the blob image of the last streaming upload
     ltx::DevBuf core_ws;   // conditioning MLP rows
     ltx::DevBuf tail_ws;   // normed rows of ltx_core_tail
@@ -170,6 +179,8 @@ float f16_bits_to_f32(uint16_t h);
 struct LinearScratch {
     uint32_t* q;
     uint32_t* pairs;
+    void* planes = nullptr;  // mode F32: f3_planes_bytes and f3_part_bytes, or NULL (the f32 MFMA kernel)
+    void* part = nullptr;
     void* w16 = nullptr;  // N * K 16-bit weights for the four-wave GEMM, or NULL (the W8A16 kernel)
 };
 // Whether the four-wave 16-bit GEMM takes an M x N x K product with A rows of
@@ -177,6 +188,11 @@ struct LinearScratch {
 bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda);
 // Whether the small-grid GEMM takes it (q8: int8 weights, else 16-bit).
 bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8);
+// The f32 GEMM on bf16 MFMAs: whether it takes an M x N x K product, and the
+// bytes of its scratch.
+bool f3_shape(const ltx_ctx* c, int M, int N, int K);
+size_t f3_planes_bytes(int M, int K);
+size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K);
 // Shape and mode checks of the isolated int8 GEMM (throws Error), made before
 // any scratch is sized from N and K.
 void check_linear_q8(int M, int N, int K, int mode);

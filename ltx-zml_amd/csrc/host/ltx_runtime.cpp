@@ -9,7 +9,8 @@
 
 // gfx950 code objects, embedded at build time (ltx_codeobjects.S).
 extern "C" {
-extern const unsigned char ltx_co_k_gemm[], ltx_co_k_gemm_s4[], ltx_co_k_attn[], ltx_co_k_norm[], ltx_co_k_f32[],
+extern const unsigned char ltx_co_k_gemm[], ltx_co_k_gemm_s4[], ltx_co_k_gemm_f3[],
+    ltx_co_k_attn[], ltx_co_k_norm[], ltx_co_k_f32[],
     ltx_co_k_core[];
 }
 
@@ -192,6 +193,7 @@ int ltx_init(int device, ltx_ctx** out) {
             c->gemm_x4 = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
         if (const char* e = std::getenv("LTX_GEMM_S4"))
             c->gemm_s4 = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
+        if (const char* e = std::getenv("LTX_GEMM_F3")) c->gemm_f3 = std::strcmp(e, "off") != 0;
         if (const char* e = std::getenv("LTX_SIDE_EARLY"))
             c->side_early = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
         if (const char* e = std::getenv("LTX_ATTN_VARIANT")) {
@@ -200,9 +202,11 @@ int ltx_init(int device, ltx_ctx** out) {
         }
         HIPC(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));  // default priority
         for (auto& e : c->side_ev) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPC(hipEventCreateWithFlags(&c->op_f3_ev, hipEventDisableTiming));
         for (auto& e : c->marks) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence));
         for (const unsigned char* co :
-             {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_attn, ltx_co_k_norm, ltx_co_k_f32, ltx_co_k_core}) {
+             {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_gemm_f3, ltx_co_k_attn, ltx_co_k_norm, ltx_co_k_f32,
+              ltx_co_k_core}) {
             hipModule_t m;
             HIPC(hipModuleLoadData(&m, co));
             c->modules.push_back(m);
@@ -229,6 +233,7 @@ void ltx_destroy(ltx_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     for (auto e : c->marks)
         if (e) (void)hipEventDestroy(e);
+    if (c->op_f3_ev) (void)hipEventDestroy(c->op_f3_ev);
     if (c->side) (void)hipStreamDestroy(c->side);
     c->ws.free_();
     c->op_pairs.free_();

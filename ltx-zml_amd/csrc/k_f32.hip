@@ -1,7 +1,8 @@
 // f32 reference-precision kernels (mode LTX_MODE_F32): a GEMM that dequantises
 // in f32 (f32(q) * s, exactly dq4 at ltx/block.zig:462-471) and an
-// online-softmax attention, both on f32 MFMAs. These carry the <= 1e-5 parity
-// mode.
+// online-softmax attention, both on f32 MFMAs. The GEMM takes the shapes that
+// the faster one on bf16 MFMAs (gemm_f3.h) does not: N or K no multiple of 128,
+// misaligned operands, calls that may use no scratch.
 #include "ltx_device.h"
 
 // y[M][N] = A[M][K] . W[N][K]^T (+ bias, GELU or the gated residual) in f32

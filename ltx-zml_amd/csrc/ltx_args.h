@@ -90,6 +90,24 @@ typedef struct {
     float* part;          // go to part [S][M][N] for ltx_gemm_reduce_* to finish with the epilogue
 } LtxGemmArgs;
 
+// f32 GEMM on bf16 MFMAs: g.a is plane 0 of the activations' exact split into
+// three bf16 planes (ltx_split3), a1 and a2 the other two, each [M][K]; g.b and
+// g.scales the weights as stored ([N][K], [N][K / 128]), the output f32.
+typedef struct {
+    LtxGemmArgs g;
+    const void* a1;
+    const void* a2;
+} LtxGemmF3Args;
+
+// x = p0 + p1 + p2 exactly, each a bf16 (n a multiple of 8).
+typedef struct {
+    const float* x;
+    uint16_t* p0;
+    uint16_t* p1;
+    uint16_t* p2;
+    size_t n;
+} LtxSplit3Args;
+
 // Dequantisation of int8 projections into 16-bit weights for the four-wave
 // 16-bit GEMM: out[j] [N][K] = the W8A16 kernel's operands, from the bytes
 // q + 128 [N][K] and the scale words [K / 128][N]. Workgroups start[j] ..

@@ -245,6 +245,74 @@ def test_linear_q8_f32_mode(ctx, M, N, K, scale_f16, gelu):
     assert oracle.rel_rms(f64(y), want) <= (1e-5 if gelu else 1e-6)
 
 
+# mode F32 where N is a multiple of 128: bf16 MFMAs on three exact planes of A
+# (one K group, an odd number of groups, ragged rows on both sides of a 128-row
+# tile, split K), or the f32 MFMA kernel
+@pytest.mark.parametrize("f3", ["on", "off"])
+@pytest.mark.parametrize("M,N,K,scale_f16,gelu", [(1, 128, 128, True, False), (127, 256, 384, True, False),
+                                                  (129, 384, 384, False, True), (300, 256, 4096, False, False),
+                                                  (2200, 2048, 512, True, True)])
+def test_linear_q8_f32_planes(monkeypatch, M, N, K, scale_f16, gelu, f3):
+    say(f"linear_q8 f32 planes={f3} M={M} N={N} K={K} scale_f16={scale_f16} gelu={gelu}")
+    monkeypatch.setenv("LTX_GEMM_F3", f3)
+    c = rt.Context(0)
+    try:
+        a, q, s, b = _gemm_case(M, N, K, seed=7 + M + N, scale_f16=scale_f16)
+        a *= (10.0 ** np.random.default_rng(M).uniform(-3, 3, size=(M, 1))).astype(np.float32)
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        c.linear_q8(torch.from_numpy(a).cuda(), torch.from_numpy(q).cuda(), torch.from_numpy(s).cuda(),
+                    torch.from_numpy(b).cuda(), y, mode=rt.MODE_F32, gelu=gelu)
+        torch.cuda.synchronize()
+        z = oracle.linear(a, q=q, s=s.astype(np.float32)) + b
+        want = 0.5 * z * (1 + np.tanh(np.sqrt(2 / np.pi) * (z + 0.044715 * z ** 3))) if gelu else z
+        # as test_linear_q8_f32_mode: the products alone 1e-6, GELU 1e-5. The
+        # f32 MFMA kernel (off) adds K / 4 sums of four products one after the
+        # other; each rounds the running sum by at most 2^-24, and as a random
+        # walk they come to at most 2^-24 sqrt(K / 4) of the result: 1.9e-6 at
+        # K = 4,096 (measured 1.1e-6)
+        if f3 == "off" and not gelu:
+            assert oracle.rel_rms(f64(y), want) <= max(1e-6, 2.0 ** -24 * np.sqrt(K / 4))
+            return
+        assert oracle.rel_rms(f64(y), want) <= (1e-5 if gelu else 1e-6)
+    finally:
+        c.close()
+
+
+def test_linear_q8_f32_planes_nonfinite_and_streams(ctx):
+    """An infinity or a NaN in A stays in its own row (inf where the products
+    are; its lower planes must not turn it into NaN); a call on a second
+    stream right behind one on the first gives what each gives alone."""
+    say("linear_q8 f32 planes: inf, NaN, two streams")
+    M, N, K = 200, 128, 256
+    a, q, s, _ = _gemm_case(M, N, K, seed=3, scale_f16=True)
+    q[q == 0] = 1
+    a[5, 7], a[9, 200] = np.inf, np.nan
+    dq, ds = torch.from_numpy(q).cuda(), torch.from_numpy(s).cuda()
+    y = torch.empty((M, N), dtype=torch.float32, device="cuda")
+    ctx.linear_q8(torch.from_numpy(a).cuda(), dq, ds, None, y, mode=rt.MODE_F32)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.array_equal(got[5], np.where(q[:, 7] > 0, np.inf, -np.inf).astype(np.float32))
+    assert np.isnan(got[9]).all()
+    rest = np.delete(np.arange(M), [5, 9])
+    want = oracle.linear(a[rest], q=q, s=s.astype(np.float32))
+    assert oracle.rel_rms(got[rest], want) <= 1e-6
+    das = [torch.randn(M, K, generator=torch.Generator().manual_seed(i)).cuda() for i in range(2)]
+    alone = []
+    for da in das:
+        ctx.linear_q8(da, dq, ds, None, y, mode=rt.MODE_F32)
+        alone.append(y.clone())
+    streams, ys = [torch.cuda.Stream() for _ in das], [torch.empty_like(y) for _ in das]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for st, da, o in zip(streams, das, ys):
+            with torch.cuda.stream(st):
+                ctx.linear_q8(da, dq, ds, None, o, mode=rt.MODE_F32)
+    torch.cuda.synchronize()
+    for o, w in zip(ys, alone):
+        assert torch.equal(o, w)
+
+
 def _heads(x, L):  # [L, D] -> [H, L, 128]
     return np.ascontiguousarray(x.reshape(L, 32, 128).transpose(1, 0, 2))
 
