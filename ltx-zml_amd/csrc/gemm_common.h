@@ -39,7 +39,13 @@ __device__ __forceinline__ void gemm_epilogue(const LtxGemmArgs& a, const f32x16
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int m = rb + 32 * i + 8 * (r >> 2) + (r & 3);
-            if (m >= a.M) continue;
+            if (m >= a.M) {
+                if (EPI == LTX_EPI_QKV && n0 >= a.nsplit && m < a.ldv)  // V^T's padding
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+                        ((uint16_t*)a.out2)[(size_t)(cb + 32 * j - a.nsplit) * a.ldv + m] = 0;
+                continue;
+            }
             const float* gt = nullptr;
             const float* gs = nullptr;
             if (EPI == LTX_EPI_RESID_GATE) {  // ada row of the gate: sst[i] + tstab[tidx[m]][i]
@@ -67,7 +73,7 @@ __device__ __forceinline__ void gemm_epilogue(const LtxGemmArgs& a, const f32x16
                         bad += out_of_range<T>(v);
                     } else {
                         int c = n - a.nsplit;  // = h * 128 + d
-                        ((uint16_t*)a.out2)[(size_t)c * a.M + m] = Op<T>::bits(v);
+                        ((uint16_t*)a.out2)[(size_t)c * a.ldv + m] = Op<T>::bits(v);
                         bad += out_of_range<T>(v);
                     }
                 }
@@ -95,8 +101,7 @@ __device__ __forceinline__ void gemm_epilogue(const LtxGemmArgs& a, const f32x16
 // is the form for NI x NJ blocks of 32 x 32.
 //
 // The body is compiled per output form (OUT: 0 16-bit rows, 1 f32 rows, 2
-// V^T), GELU and whether every row of the wave's tile is inside M (FULL, and M
-// a multiple of 8), and the per-column values (bias, gate shift) are loaded
+// V^T), GELU and whether every row of the wave's tile is inside M (FULL), and the per-column values (bias, gate shift) are loaded
 // once before the blocks. On full tiles the stores are issued in batches
 // from registers that nothing reuses before they have gone out: the 16-bit
 // outputs of HOLD blocks (the whole wave tile where registers allow) are
@@ -179,6 +184,9 @@ __device__ __forceinline__ void gemm_epilogue_body(const LtxGemmArgs& a, Fill fi
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] = patch[(8 * rg + e) * LD + cc] + bn[p];
                 const int m = mb + 8 * rg;
+                if (!FULL)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] = m + e < a.M ? v[e] : 0.0f;  // the padding
                 const u32x4 pk = {pack2<T>(v[0], v[1]), pack2<T>(v[2], v[3]), pack2<T>(v[4], v[5]),
                                   pack2<T>(v[6], v[7])};
                 if (FULL) {
@@ -186,16 +194,10 @@ __device__ __forceinline__ void gemm_epilogue_body(const LtxGemmArgs& a, Fill fi
 #pragma unroll
                     for (int e = 0; e < 8; e++) mx = __builtin_elementwise_maximum(mx, __builtin_fabsf(v[e]));
                 } else {
-                    uint16_t* dst = (uint16_t*)a.out2 + (size_t)c * a.M + m;
 #pragma unroll
-                    for (int e = 0; e < 8; e++) bad += m + e < a.M ? out_of_range<T>(v[e]) : 0u;
-                    if ((a.M & 7) == 0 && m + 8 <= a.M) {
-                        __builtin_nontemporal_store(pk, (u32x4*)dst);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 8; e++)
-                            if (m + e < a.M) dst[e] = Op<T>::bits(v[e]);
-                    }
+                    for (int e = 0; e < 8; e++) bad += out_of_range<T>(v[e]);
+                    if (m < a.ldv)
+                        __builtin_nontemporal_store(pk, (u32x4*)((uint16_t*)a.out2 + (size_t)c * a.ldv + m));
                 }
             }
             if (FULL && !(mx <= RangeMax<T>::v))  // rare: count this block's values from the patch
@@ -277,7 +279,7 @@ __device__ __forceinline__ void gemm_epilogue_body(const LtxGemmArgs& a, Fill fi
                     if (OUT == 2) {
                         const int c = nw + 16 * p + (lane >> 2) - a.nsplit;
                         __builtin_nontemporal_store(
-                            ob[h][p], (u32x4*)((uint16_t*)a.out2 + (size_t)c * a.M + bb + 8 * (lane & 3)));
+                            ob[h][p], (u32x4*)((uint16_t*)a.out2 + (size_t)c * a.ldv + bb + 8 * (lane & 3)));
                     } else {
                         const int m = bb + lane / HLPR + HRPP * p;
                         __builtin_nontemporal_store(
@@ -292,7 +294,7 @@ __device__ __forceinline__ void gemm_epilogue_body(const LtxGemmArgs& a, Fill fi
 
 template <typename T, int EPI, int NI, int NJ, int OUT, bool GELU, int HOLD, typename Fill>
 __device__ __forceinline__ void gemm_epilogue_rows(const LtxGemmArgs& a, Fill fill, float* patch, int mw, int nw) {
-    if (mw + 32 * NI <= a.M && (a.M & 7) == 0)
+    if (mw + 32 * NI <= a.M)
         gemm_epilogue_body<T, EPI, NI, NJ, OUT, GELU, true, HOLD>(a, fill, patch, mw, nw);
     else
         gemm_epilogue_body<T, EPI, NI, NJ, OUT, GELU, false, 1>(a, fill, patch, mw, nw);

@@ -14,6 +14,9 @@ static const char* msuffix(int mode) { return mode == LTX_MODE_BF16 ? "bf16" : "
 
 static size_t al(size_t n) { return (n + 255) & ~(size_t)255; }
 
+// V^T's row stride: the keys in whole 64-key attention tiles.
+static int vt_ld(size_t n) { return (int)((n + 63) & ~(size_t)63); }
+
 // Bump allocator over the context workspace.
 struct Carve {
     char* base;
@@ -100,7 +103,7 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
     const int num_cu = ctx->num_cu;
     w.n_msa = c.take(T * D * 2);
     w.qk16 = c.take(T * 2 * D * 2);
-    w.vt1 = c.take(T * D * 2);
+    w.vt1 = c.take((size_t)vt_ld(T) * D * 2);
     w.qh1 = c.take(T * D * 2);
     w.kh1 = c.take(T * D * 2);
     w.glog1 = c.take(T * LTX_H * 4);
@@ -111,7 +114,7 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
     w.glog2 = c.take(T * LTX_H * 4);
     w.enc = c.take(S * D * 2);
     w.k2_16 = c.take(S * D * 2);
-    w.vt2 = c.take(S * D * 2);
+    w.vt2 = c.take((size_t)vt_ld(S) * D * 2);
     w.qh2 = c.take(T * D * 2);
     w.kh2 = c.take(S * D * 2);
     w.o2 = c.take(T * D * 2);
@@ -381,6 +384,21 @@ static void gate16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
         c->launch(mode == LTX_MODE_BF16 ? "ltx_gate_ks_bf16" : "ltx_gate_ks_f16", (M + 31) / 32, 1, 1, 256, &g, st);
 }
 
+// Whether ltx_op_attention pads V^T (lkv no multiple of 64) for the LDS-DMA
+// kernels. The padding launch costs 7 to 9 us; the any-length kernel takes about
+// twice as long a round of workgroups and key tile, less where 8 divides lkv
+// (it then loads V^T in 16-byte vectors). Measured, padded against any-length,
+// us (lq x lkv): four or more rounds 7,001 x 16 38 : 54, 7,001 x 200 55 : 67;
+// two 2,970 x 50 27 : 22, 2,970 x 77 27 : 27, 2,970 x 129 29 : 33, 2,970 x
+// 2,970 154 : 278; one 1,000 x 200 20 : 15, 1,000 x 255 20 : 21, 1,000 x 500
+// 25 : 30, 1,000 x 1,000 (8 divides) 38 : 34.
+static bool pad_pays(const ltx_ctx* c, int lq, int lkv) {
+    const int nt = (lkv + 63) / 64, rounds = ((lq + 255) / 256 * LTX_H + c->num_cu - 1) / c->num_cu;
+    if (rounds >= 4) return true;
+    if (rounds >= 2) return nt >= 2;
+    return nt >= (lkv % 8 == 0 ? 28 : 5);
+}
+
 // The attention's exponent scale: softmax scale 1/sqrt(128) times log2(e).
 static const float kAttnC = (float)(1.4426950408889634 / 11.313708498984761);
 
@@ -394,9 +412,10 @@ static void qknorm16(ltx_ctx* c, int mode, const void* x, int ldx, const void* w
 
 // q_scaled: Q already carries kAttnC (the block path); else plain Q.
 // qk_rows: Q and K as token rows [L][4096] (the block's qk-norm output);
-// else head-major [32][L][128] (ltx_op_attention).
-static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const void* vt, const float* glog, void* out,
-                   int lq, int lkv, bool q_scaled, hipStream_t st, const char* label = nullptr,
+// else head-major [32][L][128] (ltx_op_attention). vld: V^T's row stride, a
+// multiple of 64 with zeros past lkv for the LDS-DMA kernels.
+static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const void* vt, int vld, const float* glog,
+                   void* out, int lq, int lkv, bool q_scaled, hipStream_t st, const char* label = nullptr,
                    unsigned long long* sat = nullptr, bool qk_rows = false) {
     LtxAttnArgs a{};
     a.sat = sat;
@@ -407,6 +426,7 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
     a.k_hs = qk_rows ? LTX_HD : lkv * LTX_HD;
     a.k_rs = qk_rows ? LTX_D : LTX_HD;
     a.vt = vt;
+    a.v_rs = vld;
     a.glog = glog;
     a.out = out;
     a.lq = lq;
@@ -415,7 +435,9 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
     a.q_tiles = (lq + 255) / 256;  // 256 queries per workgroup
     char name[48];
     const int wph = std::max(1, std::min(c->num_cu / LTX_H, a.q_tiles));  // workgroups per head
-    if (c->attn_kv && lkv % 64 == 0 && lkv >= 64 && lkv <= 256 && (a.q_tiles >= 2 * wph || lkv < 128)) {
+    const int nt = (lkv + 63) / 64;
+    const bool whole = vld == 64 * nt;  // V^T rows of whole key tiles
+    if (c->attn_kv && whole && nt <= 4 && (a.q_tiles >= 2 * wph || nt < 2)) {
         // resident K/V: each workgroup loads one head's K and V^T once and
         // runs every wph-th query tile of that head (with fewer than two
         // tiles per workgroup the streaming kernel, which overlaps the K/V
@@ -424,8 +446,8 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
         c->launch(name, LTX_H * wph, 1, 1, 512, &a, st, label);
         return;
     }
-    if (c->attn_pp && lkv % 64 == 0 && lkv >= 128) {
-        // ping-pong kernel: whole 64-key tiles, at least two
+    if (c->attn_pp && whole && nt >= 2) {
+        // ping-pong kernel: at least two 64-key tiles
         std::snprintf(name, sizeof(name), "ltx_attn_%s_pp%s", msuffix(mode), q_scaled ? "" : "_uq");
         c->launch(name, a.q_tiles * LTX_H, 1, 1, 512, &a, st, label);
         return;
@@ -537,9 +559,12 @@ static void stream_after(hipStream_t to, hipStream_t from, hipEvent_t e) {
     HIPC(hipStreamWaitEvent(to, e, 0));
 }
 
-static void set_stage(ltx_ctx* c, int id, void* p, size_t bytes) {
+// vld: V^T's row stride (ltx_block_stage hands out its rows without the padding)
+static void set_stage(ltx_ctx* c, int id, void* p, size_t bytes, int vld = 0) {
     c->stage_ptr[id] = p;
     c->stage_bytes[id] = bytes;
+    if (id == LTX_ST_V1) c->stage_vld[0] = vld;
+    if (id == LTX_ST_V2) c->stage_vld[1] = vld;
 }
 
 // ---- the block ------------------------------------------------------------
@@ -654,6 +679,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         gk.out = b.k2_16;
         gk.out2 = b.vt2;
         gk.nsplit = LTX_D;
+        gk.ldv = vt_ld(S);
         gk.sat = sat;
         gk.part = (float*)part;
         gemm16(c, mode, w->kv2, b.enc, S, LTX_D, LTX_EPI_QKV, gk, s, "gemm:kv2");
@@ -680,6 +706,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     g.out = b.qk16;
     g.out2 = b.vt1;
     g.nsplit = 2 * LTX_D;
+    g.ldv = vt_ld(T);
     g.sat = sat;
     g.part = (float*)b.part;  // split-K partial sums (small grids)
     gemm16(c, mode, w->qkv1, b.n_msa, T, LTX_D, LTX_EPI_QKV, g, st, "gemm:qkv1", dq[0]);
@@ -697,7 +724,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         c->launch(mode == LTX_MODE_BF16 ? "ltx_qknorm2_bf16" : "ltx_qknorm2_f16", T, 1, 1, 256, &qa, st);
     }
     HIPC(hipStreamWaitEvent(st, c->side_ev[1], 0));
-    attn16(c, mode, b.qh1, b.kh1, b.vt1, (const float*)b.glog1, b.o1, T, T, true, st, "attn:self", sat, true);
+    attn16(c, mode, b.qh1, b.kh1, b.vt1, vt_ld(T), (const float*)b.glog1, b.o1, T, T, true, st, "attn:self", sat, true);
     g = LtxGemmArgs{};
     g.out = b.x_sa;
     g.resid = x;
@@ -736,7 +763,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
             qknorm16(c, mode, b.k2_16, LTX_D, w->kn2.p, nullptr, nullptr, b.kh2, S, 1.0f, st);
         }
         stream_after(st, sd, c->side_ev[3]);  // glog2 (and, early, the context side) ready
-        attn16(c, mode, b.qh2, b.kh2, b.vt2, (const float*)b.glog2, b.o2, T, S, true, st, "attn:cross", sat, true);
+        attn16(c, mode, b.qh2, b.kh2, b.vt2, vt_ld(S), (const float*)b.glog2, b.o2, T, S, true, st, "attn:cross", sat, true);
     }
     g = LtxGemmArgs{};
     g.out = b.x_ca;
@@ -767,7 +794,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     set_stage(c, LTX_ST_NORM_MSA, b.n_msa, TD * 2);
     set_stage(c, LTX_ST_Q1, b.qh1, TD * 2);
     set_stage(c, LTX_ST_K1, b.kh1, TD * 2);
-    set_stage(c, LTX_ST_V1, b.vt1, TD * 2);
+    set_stage(c, LTX_ST_V1, b.vt1, TD * 2, vt_ld(T));
     set_stage(c, LTX_ST_GLOG1, b.glog1, (size_t)T * LTX_H * 4);
     set_stage(c, LTX_ST_ATTN1, b.o1, TD * 2);
     set_stage(c, LTX_ST_X_SA, b.x_sa, TD * 4);
@@ -779,7 +806,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     set_stage(c, LTX_ST_GLOG2, b.glog2, (size_t)T * LTX_H * 4);
     set_stage(c, LTX_ST_Q2, b.qh2, TD * 2);
     set_stage(c, LTX_ST_K2, b.kh2, SD * 2);
-    set_stage(c, LTX_ST_V2, b.vt2, SD * 2);
+    set_stage(c, LTX_ST_V2, b.vt2, SD * 2, vt_ld(S));
 }
 
 bool linear_q8_needs_scratch(const ltx_ctx* c, int N, int K, int mode) {
@@ -876,6 +903,7 @@ struct ltx_block_graph {
     // every launch
     void* stage_ptr[LTX_ST_COUNT] = {};
     uint64_t stage_bytes[LTX_ST_COUNT] = {};
+    int stage_vld[2] = {};
 };
 
 int ltx_block_graph_create(ltx_ctx* c, const ltx_block_weights* w, const float* x, const float* tstab, int K,
@@ -938,6 +966,7 @@ int ltx_block_graph_create(ltx_ctx* c, const ltx_block_weights* w, const float* 
         g->exec = exec;
         std::memcpy(g->stage_ptr, c->stage_ptr, sizeof(g->stage_ptr));
         std::memcpy(g->stage_bytes, c->stage_bytes, sizeof(g->stage_bytes));
+        std::memcpy(g->stage_vld, c->stage_vld, sizeof(g->stage_vld));
         c->ws_pins++;
         *out = g;
     })
@@ -951,6 +980,7 @@ int ltx_block_graph_launch(ltx_block_graph* g, void* stream) {
         HIPC(hipGraphLaunch(g->exec, (hipStream_t)stream));
         std::memcpy(c->stage_ptr, g->stage_ptr, sizeof(c->stage_ptr));
         std::memcpy(c->stage_bytes, g->stage_bytes, sizeof(c->stage_bytes));
+        std::memcpy(c->stage_vld, g->stage_vld, sizeof(c->stage_vld));
     })
 }
 
@@ -971,19 +1001,14 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         HIPC(hipSetDevice(c->device));
         ltx::LinearScratch sc{};
         hipStream_t st = (hipStream_t)stream;
-        // Mode F32 splits A into planes in a buffer of the context. A call on
-        // another stream than the last waits for that one's use of it; a call
-        // being captured (whose replays nothing could order, and which may not
-        // allocate) takes the f32 MFMA kernel, which needs none.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        const bool f3 = mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K) &&
-                        hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone;
-        if (f3) {
+        // mode F32 splits A into planes (not captured: then the f32 MFMA kernel)
+        bool f3 = false;
+        if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
             const size_t np = ltx::f3_planes_bytes(M, K), need = np + ltx::f3_part_bytes(c, M, N, K);
-            if (c->op_f3.bytes < need) c->op_f3.alloc(need);  // (frees the old one after the device has finished with it)
-            sc.planes = c->op_f3.p;
-            sc.part = need > np ? (char*)c->op_f3.p + np : nullptr;
-            if (c->op_f3_used && c->op_f3_stream != st) HIPC(hipStreamWaitEvent(st, c->op_f3_ev, 0));
+            if ((sc.planes = c->op_scratch.take(need, st))) {
+                f3 = true;
+                sc.part = need > np ? (char*)sc.planes + np : nullptr;
+            }
         }
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
             // scratch owned by the context, grown as needed
@@ -998,11 +1023,7 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
             }
         }
         ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, st);
-        if (f3) {
-            HIPC(hipEventRecord(c->op_f3_ev, st));
-            c->op_f3_stream = st;
-            c->op_f3_used = true;
-        }
+        if (f3) c->op_scratch.done(st);
     })
 }
 
@@ -1015,11 +1036,21 @@ int ltx_op_attention(ltx_ctx* c, const void* q, const void* k, const void* v, co
         mode &= ~LTX_ATTN_Q_SCALED;
         if (q_scaled && mode == LTX_MODE_F32) throw ltx::Error("LTX_ATTN_Q_SCALED applies to the 16-bit modes");
         HIPC(hipSetDevice(c->device));
-        if (mode == LTX_MODE_F32)
-            ltx::attn32(c, (const float*)q, (const float*)k, (const float*)v, glog, (float*)out, lq, lkv,
-                        (hipStream_t)stream);
-        else
-            ltx::attn16(c, mode, q, k, v, glog, out, lq, lkv, q_scaled, (hipStream_t)stream);
+        hipStream_t st = (hipStream_t)stream;
+        if (mode == LTX_MODE_F32) {
+            ltx::attn32(c, (const float*)q, (const float*)k, (const float*)v, glog, (float*)out, lq, lkv, st);
+            return LTX_OK;
+        }
+        // V^T's rows padded to whole key tiles for the LDS-DMA kernels (not
+        // captured: then the any-length kernel)
+        const int vld = ltx::vt_ld(lkv);
+        void* pad = nullptr;
+        if (vld != lkv && c->attn_pp && ltx::pad_pays(c, lq, lkv) && (pad = c->op_scratch.take((size_t)LTX_D * vld * 2, st))) {
+            LtxVtPadArgs pa{(const uint16_t*)v, (uint16_t*)pad, lkv, vld};
+            c->launch("ltx_vt_pad", (vld + 511) / 512, LTX_D / 4, 1, 256, &pa, st);
+        }
+        ltx::attn16(c, mode, q, k, pad ? pad : v, pad ? vld : lkv, glog, out, lq, lkv, q_scaled, st);
+        if (pad) c->op_scratch.done(st);
     })
 }
 

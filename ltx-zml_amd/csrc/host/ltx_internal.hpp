@@ -40,6 +40,24 @@ struct DevBuf {
     DevBuf& operator=(const DevBuf&) = delete;
 };
 
+// Scratch of the isolated operators that needed none before they had it: one
+// buffer per context, kept and grown. Calls on different streams stay
+// independent for the caller: take() makes the stream wait for the last use on
+// another one (done()). It returns NULL to a call that is being captured, whose
+// replays nothing here could order and which may not allocate; the caller then
+// runs the kernel that needs no scratch.
+struct StreamScratch {
+    DevBuf buf;
+    hipEvent_t ev = nullptr;
+    hipStream_t last = nullptr;
+    bool used = false;
+    void* take(size_t bytes, hipStream_t st);
+    void done(hipStream_t st);
+    ~StreamScratch() {
+        if (ev) (void)hipEventDestroy(ev);
+    }
+};
+
 struct ProfRec {
     const char* name;
     hipEvent_t a, b;
@@ -124,12 +142,9 @@ struct ltx_ctx {
     ltx::DevBuf op_pairs;  // scale pairs of the last ltx_op_linear_q8 call (f16 scales)
     ltx::DevBuf op_q;      // its weights as bytes q + 128
     ltx::DevBuf op_w16;    // and dequantised to 16 bits (four-wave GEMM)
-    // ltx_op_linear_q8 in mode F32: the planes and partial sums of the last
-    // call, the event after that call and the stream it ran on
-    ltx::DevBuf op_f3;
-    hipEvent_t op_f3_ev = nullptr;
-    hipStream_t op_f3_stream = nullptr;
-    bool op_f3_used = false;
+    // ltx_op_linear_q8 in mode F32 (planes and partial sums) and
+    // ltx_op_attention (padded V^T)
+    ltx::StreamScratch op_scratch;
     ltx::DevBuf blob_stage;  // device copy of the blob image of the last streaming upload
     ltx::DevBuf core_ws;   // conditioning MLP rows
     ltx::DevBuf tail_ws;   // normed rows of ltx_core_tail
@@ -139,6 +154,8 @@ struct ltx_ctx {
     int ws_pins = 0;  // live block graphs: their kernels hold workspace addresses
     void* stage_ptr[LTX_ST_COUNT] = {};
     uint64_t stage_bytes[LTX_ST_COUNT] = {};
+    int stage_vld[2] = {};     // row stride of the V^T stages V1, V2 (0: mode F32)
+    ltx::DevBuf stage_vt[2];   // their rows without the padding (ltx_block_stage)
     // profiling
     bool prof = false;
     std::vector<ltx::ProfRec> prof_recs;

@@ -54,6 +54,21 @@ void DevBuf::free_() {
     bytes = 0;
 }
 
+void* StreamScratch::take(size_t bytes, hipStream_t st) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
+    if (!ev) HIPC(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    if (buf.bytes < bytes) buf.alloc(bytes);  // (hipFree of the old one waits for the device)
+    if (used && last != st) HIPC(hipStreamWaitEvent(st, ev, 0));
+    return buf.p;
+}
+
+void StreamScratch::done(hipStream_t st) {
+    HIPC(hipEventRecord(ev, st));
+    last = st;
+    used = true;
+}
+
 uint16_t f32_to_f16_bits(float f) {  // round to nearest even, IEEE binary16
     uint32_t x;
     std::memcpy(&x, &f, 4);
@@ -202,7 +217,6 @@ int ltx_init(int device, ltx_ctx** out) {
         }
         HIPC(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));  // default priority
         for (auto& e : c->side_ev) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        HIPC(hipEventCreateWithFlags(&c->op_f3_ev, hipEventDisableTiming));
         for (auto& e : c->marks) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence));
         for (const unsigned char* co :
              {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_gemm_f3, ltx_co_k_attn, ltx_co_k_norm, ltx_co_k_f32,
@@ -233,7 +247,6 @@ void ltx_destroy(ltx_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     for (auto e : c->marks)
         if (e) (void)hipEventDestroy(e);
-    if (c->op_f3_ev) (void)hipEventDestroy(c->op_f3_ev);
     if (c->side) (void)hipStreamDestroy(c->side);
     c->ws.free_();
     c->op_pairs.free_();
@@ -303,7 +316,21 @@ int ltx_block_stage(ltx_ctx* c, int stage, void** dev_ptr, uint64_t* bytes) {
         if (!c) throw ltx::Error("NULL context");
         if (stage < 0 || stage >= LTX_ST_COUNT) throw ltx::Error("stage id out of range");
         if (!c->stage_ptr[stage]) throw ltx::Error("stage not available (no forward yet, or not in this mode)");
-        if (dev_ptr) *dev_ptr = c->stage_ptr[stage];
+        void* p = c->stage_ptr[stage];
+        // V^T is kept with rows padded to whole key tiles: hand out [32][128][n]
+        if (stage == LTX_ST_V1 || stage == LTX_ST_V2) {
+            const int i = stage == LTX_ST_V2;
+            const size_t n = c->stage_bytes[stage] / (LTX_D * 2), vld = (size_t)c->stage_vld[i];
+            if (vld && vld != n) {
+                HIPC(hipSetDevice(c->device));
+                HIPC(hipDeviceSynchronize());
+                if (c->stage_vt[i].bytes < c->stage_bytes[stage]) c->stage_vt[i].alloc(c->stage_bytes[stage]);
+                HIPC(hipMemcpy2D(c->stage_vt[i].p, n * 2, p, vld * 2, n * 2, LTX_D, hipMemcpyDeviceToDevice));
+                HIPC(hipDeviceSynchronize());
+                p = c->stage_vt[i].p;
+            }
+        }
+        if (dev_ptr) *dev_ptr = p;
         if (bytes) *bytes = c->stage_bytes[stage];
     })
 }

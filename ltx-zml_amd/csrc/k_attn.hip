@@ -2,11 +2,15 @@
 // ltx/block.zig:105-154, whileSdpaC), fused with the per-(token, head) gate
 // 2*sigmoid(glog) and the head merge (ltx/block.zig:237-242). Two kernels:
 //
-// - ltx_attn_{f16,bf16}_pp (the ping-pong kernel, below): whole 64-key tiles
-//   (lkv % 64 == 0, at least two), K and V^T streamed global -> LDS by DMA;
-//   the block's self- and cross-attention take it;
-// - ltx_attn_{f16,bf16}_w8[_full] (any key count): 8 waves of 32 queries, K
-//   and V^T staged through registers into LDS, keys past lkv masked.
+// - ltx_attn_{f16,bf16}_pp (the ping-pong kernel, below): at least two 64-key
+//   tiles, K and V^T streamed global -> LDS by DMA; the block's self- and
+//   cross-attention take it. Keys past lkv are masked in the last tile, and
+//   V^T's rows are padded with zeros to whole tiles (0 * p stays 0): 2,970
+//   queries and keys 154 us with the padding's launch, 278-308 us on the w8
+//   kernel, which took every ragged key count before;
+// - ltx_attn_{f16,bf16}_w8[_full] (any key count, V^T rows of any stride): 8
+//   waves of 32 queries, K and V^T staged through registers into LDS, keys
+//   past lkv masked.
 //
 // Both compute the scores TRANSPOSED, S^T = K . Q^T, and the output as
 // O^T = V^T . P^T: the query is then the MFMA column index, so a query's
@@ -53,7 +57,7 @@ __device__ void attn_body(const LtxAttnArgs& a) {
 
     const uint16_t* Q = (const uint16_t*)a.q + (size_t)h * a.q_hs;
     const uint16_t* K = (const uint16_t*)a.k + (size_t)h * a.k_hs;
-    const uint16_t* V = (const uint16_t*)a.vt + (size_t)h * LTX_HD * lkv;
+    const uint16_t* V = (const uint16_t*)a.vt + (size_t)h * LTX_HD * a.v_rs;
 
     // Q^T operand: lane holds Q[q][16 c + 8 (lane / 32) .. + 8] for its query.
     const int fr = lane & 31, hi = lane >> 5;
@@ -92,8 +96,8 @@ __device__ void attn_body(const LtxAttnArgs& a) {
         for (int i = 0; i < NCH; i++) {
             int id = tid + NT * i, d = id >> 3, kc = id & 7;
             int key = kv0 + 8 * kc;
-            const uint16_t* src = V + (size_t)d * lkv + key;
-            if (FULL || (key + 8 <= lkv && (lkv & 7) == 0)) {  // 16-byte aligned row chunk
+            const uint16_t* src = V + (size_t)d * a.v_rs + key;
+            if (FULL || (key + 8 <= lkv && (a.v_rs & 7) == 0)) {  // 16-byte aligned row chunk
                 rv[i] = *(const u32x4*)src;
             } else {  // ragged tail / unaligned rows: element loads, zero-fill (0 * p stays finite)
                 uint16_t e[8];
@@ -287,8 +291,8 @@ __device__ __forceinline__ float asp_quad_max(float x) {
 }
 
 // ---------------------------------------------------------------------------
-// Ping-pong kernel for whole 64-key tiles (lkv % 64 == 0, at least two
-// tiles), on v_mfma_f32_16x16x32: 8 waves of 32 queries; waves w and w + 4
+// Ping-pong kernel for 64-key tiles (at least two, the last one masked past
+// lkv), on v_mfma_f32_16x16x32: 8 waves of 32 queries; waves w and w + 4
 // share a SIMD and run one phase apart. A wave alternates an MFMA phase
 // (PV(t-1) then S(t), fragments from LDS) with a softmax phase (softmax(t),
 // the rare output rescale, and the DMA of K(t+2) and V(t+1)), so at any time
@@ -392,7 +396,7 @@ struct AttnPP {
 #pragma unroll
             for (int i = 0; i < 2; i++)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (attn_lds_ptr)(d + 8192 * h + 1024 * i), 16, gv[i],
-                                                         t * 128 + 128 * a.lkv * h, 0, 0);
+                                                         t * 128 + 128 * a.v_rs * h, 0, 0);
     }
 
     // MFMA phase t: PV(t-1) from the V^T tile at sv, then S(t) from the K tile
@@ -485,7 +489,18 @@ struct AttnPP {
     // moved, the output and row sum rescaled (after PV(t-1), before PV(t))
     // and the weights formed again. The first tile always takes that path
     // and sets m to its max.
-    __device__ __forceinline__ void softmax(bool first) {
+    // LAST: this may be the last tile, whose keys past lkv get no weight.
+    template <bool LAST = true>
+    __device__ __forceinline__ void softmax(bool first, bool last) {
+        if (LAST && last && (a.lkv & 63)) {
+            // keys of the lane's values left in the tile, from its first one
+            const int left = (a.lkv & 63) - 8 * ((opaque_tid() >> 4) & 3);
+#pragma unroll
+            for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (32 * (kb >> 1) + 4 * (kb & 1) + r >= left) s[kb][0][r] = s[kb][1][r] = -__builtin_inff();
+        }
         f32x2 ps = exps<false>(f32x2{0.f, 0.f});
         if (first || __builtin_amdgcn_ballot_w64(!(ps[0] <= 256.0f) || !(ps[1] <= 256.0f)) != 0) {
             f32x2 delta;
@@ -497,7 +512,8 @@ struct AttnPP {
 #pragma unroll
                     for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[kb][qb][r]);
                 mx = asp_quad_max(mx);  // tile max relative to m
-                delta[qb] = first ? mx : fmaxf(mx, 0.f);
+                // (a first tile with no finite score keeps m = 0)
+                delta[qb] = first ? (mx == -__builtin_inff() ? 0.f : mx) : fmaxf(mx, 0.f);
                 const float corr = first ? 0.f : __builtin_amdgcn_exp2f(PS ? -delta[qb] : -delta[qb] * C);
                 m[qb] += delta[qb];
                 l[qb] *= corr;
@@ -546,7 +562,7 @@ struct AttnPP {
             dma_v<(T4 + 2) % 4>(t + 2);
         }
         __builtin_amdgcn_sched_barrier(0);
-        softmax(!FULL && t == 0);
+        softmax<!FULL>(!FULL && t == 0, !FULL && t == nt - 1);
         pin_softmax_pre();
         __builtin_amdgcn_sched_barrier(0);
         if (g == 0) {
@@ -561,14 +577,16 @@ struct AttnPP {
     // Buffers, DMA sources and fragment offsets of head h (wave w)
     __device__ __forceinline__ void setup(int h, int w, int lane) {
         const int lkv = a.lkv;
-        nt = lkv / 64;
+        nt = (lkv + 63) / 64;
         C = a.scale_log2;
         // K rows are kr bytes apart (head-major: 256; token rows: 8 KB)
         kr = 2u * (uint32_t)a.k_rs;
         rk = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)a.k + (size_t)h * a.k_hs), 0,
                                                (int)((uint32_t)(lkv - 1) * kr + 2u * LTX_HD), ASP_RSRC_W3);
-        rv = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)a.vt + (size_t)h * LTX_HD * lkv), 0,
-                                               lkv * LTX_HD * 2, ASP_RSRC_W3);
+        // (K rows past lkv lie past this end: the buffer's range check reads
+        // them as zeros, and their scores are masked)
+        rv = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)a.vt + (size_t)h * LTX_HD * a.v_rs), 0,
+                                               a.v_rs * LTX_HD * 2, ASP_RSRC_W3);
         lw = 2048 * w;
         // DMA sources: K instruction i of wave w fills LDS rows 4 (2 w + i) ..
         // +3 (16 lanes a row; row R holds key perm(R), the +32 half likewise);
@@ -581,7 +599,7 @@ struct AttnPP {
             gk[i] = (uint32_t)key * kr + 16u * c;
             const int d = 8 * (2 * w + i) + (lane >> 3);
             const int cv = (lane & 7) ^ ((d >> 1) & 7);
-            gv[i] = (uint32_t)d * (uint32_t)lkv * 2u + 16u * cv;
+            gv[i] = (uint32_t)d * (uint32_t)a.v_rs * 2u + 16u * cv;
         }
         const int j = lane >> 4, r = lane & 15;
 #pragma unroll
@@ -749,7 +767,7 @@ struct AttnPP {
         barrier();
     }
 
-    // Resident K/V (lkv = 64 nt, 1 <= nt <= 4): the workgroup loads head h's
+    // Resident K/V (nt = 1 to 4 tiles of 64 keys): the workgroup loads head h's
     // whole K and V^T into LDS once (kres, vres: nt tiles of 16 KB each, the
     // stage layouts above), then runs query tiles qt0, qt0 + wph, ... of that
     // head with no DMA, as one continuous ping-pong over the (query tile, key
@@ -780,7 +798,7 @@ struct AttnPP {
                             (uint32_t)(64 * t + 32 * hh) * kr, 0, 0);
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(
                             rv, (attn_lds_ptr)(vres + 16384 * t + lw + 8192 * hh + 1024 * i), 16, gv[i],
-                            t * 128 + 128 * a.lkv * hh, 0, 0);
+                            t * 128 + 128 * a.v_rs * hh, 0, 0);
                     }
             }
         }
@@ -812,21 +830,21 @@ struct AttnPP {
                 store_out<32>(patch, h, q0 - 256 * wph, lane, gl, bad);
                 load_glog(gl, h, q0, lane);
             }
-            softmax(true);
+            softmax(true, nt == 1);
             if (nt == 1) next_tile(qn);
             prefetch_v(vres);
             pin_softmax_pre();
             barrier();
             for (int t = 1; t < nt - 1; t++) {
                 rphase<true>(kres + 16384 * t, vres + 16384 * (t - 1), true, true);
-                softmax(false);
+                softmax<false>(false, false);
                 prefetch_v(vres + 16384 * t);
                 pin_softmax_pre();
                 barrier();
             }
             if (nt > 1) {
                 rphase<true>(kres + 16384 * (nt - 1), vres + 16384 * (nt - 2), true, true);
-                softmax(false);
+                softmax(false, true);
                 next_tile(qn);
                 prefetch_v(vres + 16384 * (nt - 1));
                 pin_softmax_pre();
@@ -860,7 +878,7 @@ extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_bf16_pp_uq(const L
     k.run();
 }
 
-// _kv: resident K/V (a multiple of 64 keys, at most 256), persistent over
+// _kv: resident K/V (at most 256 keys), persistent over
 // query tiles: grid = LTX_H x workgroups per head
 __shared__ __attribute__((aligned(1024))) uint8_t arx_k[65536];
 __shared__ __attribute__((aligned(1024))) uint8_t arx_v[65536];
@@ -880,4 +898,21 @@ extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_f16_kv_uq(const Lt
 extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_bf16_kv_uq(const LtxAttnArgs a) {
     AttnPP<__bf16, false> k(a);
     k.run_resident(arx_k, arx_v, arx_patch);
+}
+
+// V^T rows padded to whole key tiles for the kernels above (whose 16-byte DMA
+// needs aligned rows): 8 columns a thread, loaded as one 16-byte vector where
+// they are all inside the row (of any 2-byte alignment).
+extern "C" __global__ void __launch_bounds__(256) ltx_vt_pad(const LtxVtPadArgs a) {
+    const int c = 8 * (blockIdx.x * 64 + (threadIdx.x & 63)), d = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (c >= a.ld) return;
+    const uint16_t* src = a.v + (size_t)d * a.n + c;
+    uint16_t e[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (c + 8 <= a.n)
+        __builtin_memcpy(e, src, 16);
+    else
+        for (int j = 0; j < 8; j++) e[j] = c + j < a.n ? src[j] : (uint16_t)0;
+    u32x4 v;
+    __builtin_memcpy(&v, e, 16);
+    *(u32x4*)(a.y + (size_t)d * a.ld + c) = v;
 }

@@ -365,21 +365,16 @@ __device__ void reduce_body(const LtxGemmArgs& a) {
     } else if (EPI == LTX_EPI_QKV && n0 >= a.nsplit) {
         // V^T [c][m], c = n - nsplit: through LDS, then 64-token rows
 #pragma unroll
-        for (int e = 0; e < 16; e++) tr[cq + e][r] = Op<T>::bits(v[e]);
+        for (int e = 0; e < 16; e++) tr[cq + e][r] = Op<T>::bits(v[e]);  // rows past M: zeros, V^T's padding
         if (row_ok)
 #pragma unroll
             for (int e = 0; e < 16; e++) bad += out_of_range<T>(v[e]);
         __syncthreads();
         const int c = n0 - a.nsplit + r, mm = m0 + cq;  // row r of the transposed block, tokens cq ..
-        uint16_t* dst = (uint16_t*)a.out2 + (size_t)c * a.M + mm;
-        if (mm + 16 <= a.M && (a.M & 7) == 0) {
-            const u32x4* src = (const u32x4*)&tr[r][cq];
-            *(u32x4*)dst = src[0];
-            *(u32x4*)(dst + 8) = src[1];
-        } else {
-            for (int e = 0; e < 16; e++)
-                if (mm + e < a.M) dst[e] = tr[r][cq + e];
-        }
+        uint16_t* dst = (uint16_t*)a.out2 + (size_t)c * a.ldv + mm;
+        const u32x4* src = (const u32x4*)&tr[r][cq];
+        *(u32x4*)dst = src[0];
+        *(u32x4*)(dst + 8) = src[1];
     } else if (row_ok) {  // STORE, or the q | k rows of the QKV split
         const bool gelu = EPI == LTX_EPI_STORE && a.gelu;
         if (gelu)

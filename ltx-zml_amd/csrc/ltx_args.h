@@ -56,7 +56,7 @@ typedef struct {
 enum {
     LTX_EPI_STORE = 0,      // y = acc (+ bias); out f32 or 16-bit; optional GELU
     LTX_EPI_RESID_GATE = 1, // out32 = resid + (acc (+ bias)) * ada[igate]
-    LTX_EPI_QKV = 2,        // cols < nsplit: 16-bit [M][nsplit] (+bias); cols >= nsplit: 16-bit V^T [H][HD][M]
+    LTX_EPI_QKV = 2,        // cols < nsplit: 16-bit [M][nsplit] (+bias); cols >= nsplit: 16-bit V^T [H][HD][ldv]
 };
 
 // B operand kinds.
@@ -79,6 +79,7 @@ typedef struct {
     int lda;
     int ldo;              // output row stride (elements)
     int nsplit;           // QKV: first V column
+    int ldv;              // QKV: V^T row stride, M rounded up to 64 (columns M .. ldv - 1 are written as zeros)
     int igate;            // RESID_GATE ada row
     int gelu;             // STORE: apply GELU-tanh
     int out_f32;          // STORE: 1 = f32 output, 0 = 16-bit output
@@ -156,7 +157,8 @@ typedef struct {
 // Blockwise online-softmax attention with per-(token, head) gate.
 // q, k: 16-bit, element (h, l, d) at h * hs + l * rs + d: head-major
 // [H][L][HD] (hs = L HD, rs = HD) or token rows [L][D] (hs = HD, rs = D);
-// vt: [H][HD][Lkv] 16-bit; glog: [Lq][H] f32 gate logits (gate =
+// vt: [H][HD][v_rs] 16-bit (the LDS-DMA kernels: v_rs a multiple of 64, zeros
+// from column Lkv on); glog: [Lq][H] f32 gate logits (gate =
 // 2*sigmoid); out: [Lq][D] 16-bit merged heads.
 typedef struct {
     const void* q;
@@ -167,10 +169,19 @@ typedef struct {
     int lq, lkv;
     int q_hs, q_rs;     // element strides of q: head, row
     int k_hs, k_rs;     // of k
+    int v_rs;           // element stride of V^T rows
     float scale_log2;   // softmax scale * log2(e)
     int q_tiles;        // ceil(lq / q-tile)
     unsigned long long* sat;  // range guard counter of the 16-bit output or NULL
 } LtxAttnArgs;
+
+// V^T rows [LTX_D][n] -> [LTX_D][ld], ld = n rounded up to 64, zeros from
+// column n on (ltx_op_attention, key counts that are no multiple of 64).
+typedef struct {
+    const uint16_t* v;
+    uint16_t* y;
+    int n, ld;
+} LtxVtPadArgs;
 
 // Gate logits: glog[t][h] = a[t] . gw[h] + gb[h] (N = 32 heads).
 typedef struct {

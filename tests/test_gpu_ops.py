@@ -357,6 +357,59 @@ def test_attention(ctx, mode, lq, lkv, gated, q_scaled):
     assert oracle.rel_rms(f64(out), want) <= (2e-3 if mode == "f16" else 1e-2)
 
 
+# the LDS-DMA kernels on key counts that are no multiple of 64: one key, one
+# short of a tile and one past it, resident K/V (up to 256 keys, one or several
+# query tiles a workgroup) and the streaming form's shortest and longer loops
+@pytest.mark.parametrize("mode,q_scaled", [("f16", False), ("bf16", True)])
+@pytest.mark.parametrize("lq,lkv", [(70, 1), (300, 63), (257, 65), (4100, 100), (2100, 255), (256, 129), (300, 257),
+                                    (513, 449), (130, 706), (8200, 1), (2100, 70)])
+def test_attention_ragged_keys(ctx, mode, q_scaled, lq, lkv):
+    """Everything past the last key is NaN in memory, so a key that is not
+    masked, or a V^T column that is not padded, shows."""
+    say(f"attention ragged keys mode={mode} lq={lq} lkv={lkv}")
+    m, dt = MODES[mode]
+    cq = np.float32(rt.ATTN_C if q_scaled else 1.0)
+    rng = np.random.default_rng(lq + 5 * lkv)
+    q, k, v = (rng.standard_normal((n, 4096)).astype(np.float32) for n in (lq, lkv, lkv))
+
+    def put(a):  # contiguous, with NaN behind it
+        a = to16(a, dt)
+        buf = torch.full((a.numel() + 65536,), float("nan"), dtype=dt)
+        buf[:a.numel()] = a.flatten()
+        return buf.cuda()[:a.numel()].view(a.shape)
+
+    dq, dk = put(_heads(q * cq, lq)), put(_heads(k, lkv))
+    dv = put(np.ascontiguousarray(v.reshape(lkv, 32, 128).transpose(1, 2, 0)))
+    out = torch.full((lq, 4096), float("nan"), dtype=dt, device="cuda")
+    ctx.attention(dq, dk, dv, None, out, lq, lkv, mode=m, q_scaled=q_scaled)
+    torch.cuda.synchronize()
+    want = oracle.sdpa(f64(dq).transpose(1, 0, 2).reshape(lq, 4096) / cq, f64(dk).transpose(1, 0, 2).reshape(lkv, 4096),
+                       f64(dv).transpose(2, 0, 1).reshape(lkv, 4096), chunk=0)
+    # as test_attention: the rounding of P and of the output to 16 bits
+    assert oracle.rel_rms(f64(out), want) <= (2e-3 if mode == "f16" else 1e-2)
+
+
+def test_attention_ragged_keys_captured(ctx):
+    """Under capture no scratch is taken (the any-length kernel runs); eager
+    calls between the replays take the padded path."""
+    say("attention ragged keys under capture")
+    lq, lkv = 300, 450
+    g = torch.Generator(device="cuda").manual_seed(4)
+    q, k, v = (torch.randn(32, n, d, generator=g, device="cuda").half() for n, d in ((lq, 128), (lkv, 128), (128, lkv)))
+    out, eager = (torch.zeros(lq, 4096, dtype=torch.float16, device="cuda") for _ in range(2))
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        ctx.attention(q, k, v, None, out, lq, lkv)
+    for i in range(3):
+        out.zero_()
+        graph.replay()
+        ctx.attention(q, k, v, None, eager, lq, lkv)
+        torch.cuda.synchronize()
+        # two kernels, P and the output each rounded once to f16: 2e-3
+        assert oracle.rel_rms(f64(out), f64(eager)) <= 2e-3, i
+
+
 @pytest.mark.parametrize("lq,lkv", [(130, 70), (1000, 1000), (257, 193), (64, 1)])
 def test_attention_f32_mode(ctx, lq, lkv):
     say(f"attention mode=f32 lq={lq} lkv={lkv}")
