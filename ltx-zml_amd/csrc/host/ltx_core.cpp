@@ -142,11 +142,16 @@ static void conditioning(ltx_ctx* c, const ltx_core_weights* cw, const float* t,
     lin32(c, cw, LTX_C_PADA_OUT_W, pse, 1, pts2, st);
 }
 
+static void patchify(ltx_ctx* c, const ltx_core_weights* cw, const float* latent, int T, float* x, hipStream_t st) {
+    LtxPatchifyArgs a{latent, (const uint16_t*)cw->t[LTX_C_PAT_W].p, (const float*)cw->t[LTX_C_PAT_B].p, x, T};
+    c->launch("ltx_core_patchify", (T + 63) / 64, LTX_DIM / 512, 1, 512, &a, st);
+}
+
 static void tail(ltx_ctx* c, const ltx_core_weights* cw, const float* x, const float* emb, const int32_t* tidx, int T,
-                 float* normed, float* vel, hipStream_t st) {
-    LtxTailNormArgs a{x, (const float*)cw->t[LTX_C_FSST].p, emb, tidx, normed};
-    c->launch("ltx_core_tail_norm", T, 1, 1, 256, &a, st);
-    lin32(c, cw, LTX_C_PO_W, normed, T, vel, st);
+                 float* vel, hipStream_t st) {
+    LtxTailArgs a{x, (const float*)cw->t[LTX_C_FSST].p, emb, tidx, (const uint16_t*)cw->t[LTX_C_PO_W].p,
+                  (const float*)cw->t[LTX_C_PO_B].p, vel, T};
+    c->launch("ltx_core_tail", (T + 31) / 32, 1, 1, 512, &a, st);
 }
 
 }  // namespace ltx
@@ -205,7 +210,7 @@ int ltx_core_patchify(ltx_ctx* c, const ltx_core_weights* cw, const float* laten
         if (!c || !cw || !latent || !x) throw Error("NULL argument");
         if (T <= 0) throw Error("T must be positive");
         HIPC(hipSetDevice(c->device));
-        ltx::lin32(c, cw, LTX_C_PAT_W, latent, T, x, (hipStream_t)stream);
+        ltx::patchify(c, cw, latent, T, x, (hipStream_t)stream);
     })
 }
 
@@ -215,9 +220,7 @@ int ltx_core_tail(ltx_ctx* c, const ltx_core_weights* cw, const float* x, const 
         if (!c || !cw || !x || !emb || !tidx || !vel) throw Error("NULL argument");
         if (T <= 0) throw Error("T must be positive");
         HIPC(hipSetDevice(c->device));
-        const size_t need = (size_t)T * LTX_DIM * 4;
-        if (c->tail_ws.bytes < need) c->tail_ws.alloc(need);
-        ltx::tail(c, cw, x, emb, tidx, T, (float*)c->tail_ws.p, vel, (hipStream_t)stream);
+        ltx::tail(c, cw, x, emb, tidx, T, vel, (hipStream_t)stream);
     })
 }
 
@@ -270,15 +273,14 @@ int ltx_denoise(ltx_ctx* c, const ltx_block_weights* const* blocks, int nblocks,
             if (!blocks[b]) throw Error("NULL block weights");
         HIPC(hipSetDevice(c->device));
         hipStream_t st = (hipStream_t)stream;
-        // workspace: x ping-pong [T][D] x 2, tail norm [T][D], tstab [K][9][D],
-        // emb [K][D], pts2 [2][D], velocity [T][128], tk [K] + sigma
+        // workspace: x ping-pong [T][D] x 2, tstab [K][9][D], emb [K][D], pts2
+        // [2][D], velocity [T][128], tk [K] + sigma
         const size_t xd = (size_t)T * LTX_DIM;
-        const size_t need = (3 * xd + (size_t)K * 10 * LTX_DIM + 2 * LTX_DIM + (size_t)T * 128 + 64) * 4;
+        const size_t need = (2 * xd + (size_t)K * 10 * LTX_DIM + 2 * LTX_DIM + (size_t)T * 128 + 64) * 4;
         if (c->dn_ws.bytes < need) c->dn_ws.alloc(need);
         float* xa = (float*)c->dn_ws.p;
         float* xb = xa + xd;
-        float* normed = xb + xd;
-        float* tstab = normed + xd;
+        float* tstab = xb + xd;
         float* emb = tstab + (size_t)K * 9 * LTX_DIM;
         float* pts2 = emb + (size_t)K * LTX_DIM;
         float* vel = pts2 + 2 * LTX_DIM;
@@ -289,12 +291,12 @@ int ltx_denoise(ltx_ctx* c, const ltx_block_weights* const* blocks, int nblocks,
             LtxTimestepArgs ta{maskk, tk, K, sigma};
             c->launch("ltx_sched_timesteps", 1, 1, 1, 64, &ta, st);
             ltx::conditioning(c, cw, tk, K, tk + K, tstab, emb, pts2, st);
-            ltx::lin32(c, cw, LTX_C_PAT_W, latent, T, xa, st);
+            ltx::patchify(c, cw, latent, T, xa, st);
             for (int b = 0; b < nblocks; b++) {
                 ltx::block_forward(c, blocks[b], xa, tstab, K, tidx, ctx_tokens, S, pts2, cos, sin, T, xb, mode, st);
                 std::swap(xa, xb);
             }
-            ltx::tail(c, cw, xa, emb, tidx, T, normed, vel, st);
+            ltx::tail(c, cw, xa, emb, tidx, T, vel, st);
             // elementwise, so the latent is updated in place
             LtxSchedArgs sa{latent, vel, clean, tk, maskk, tidx, latent, n, LTX_IN_CH, sigma, sigma_next};
             c->launch("ltx_sched_step", (unsigned)((n + 255) / 256), 1, 1, 256, &sa, st);

@@ -541,6 +541,11 @@ static void gemm32(ltx_ctx* c, const LtxProj& p, int r0, int N, const float* A, 
     c->launch("ltx_gemm_f32", (N + 127) / 128, (M + 127) / 128, 1, 256, &g, st, label);
 }
 
+static void gate32(ltx_ctx* c, const LtxProj& p, const float* A, int M, float* out, hipStream_t st, const char* label) {
+    LtxGate32Args g{A, (const uint16_t*)p.w_bf16.p, (const float*)p.bias.p, out, M};
+    c->launch("ltx_gate_f32", (M + 15) / 16, 1, 1, 512, &g, st, label);
+}
+
 static void qknorm32(ltx_ctx* c, float* x, const void* w, const float* cs, const float* sn, int rows, hipStream_t st) {
     LtxQkNorm32Args a{x, (const float*)w, cs, sn, rows, LTX_D};
     c->launch("ltx_qknorm_f32", rows, 1, 1, 256, &a, st);
@@ -600,7 +605,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         gemm32(c, w->qkv1, 0, LTX_D, (const float*)b.n_msa, T, (float*)b.q, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
         gemm32(c, w->qkv1, LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.k, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
         gemm32(c, w->qkv1, 2 * LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.v, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
-        gemm32(c, w->g1, 0, LTX_H, (const float*)b.n_msa, T, (float*)b.glog1, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "ltx_gate:1");
+        gate32(c, w->g1, (const float*)b.n_msa, T, (float*)b.glog1, st, "ltx_gate:1");
         qknorm32(c, (float*)b.q, w->qn1.p, cs, sn, T, st);
         qknorm32(c, (float*)b.k, w->kn1.p, cs, sn, T, st);
         attn32(c, (const float*)b.q, (const float*)b.k, (const float*)b.v, (const float*)b.glog1, (float*)b.o1, T, T, st, "attn:self");
@@ -615,7 +620,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         split(b.enc, S, LTX_D);
         gemm32(c, w->kv2, 0, LTX_D, (const float*)b.enc, S, (float*)b.k2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
         gemm32(c, w->kv2, LTX_D, LTX_D, (const float*)b.enc, S, (float*)b.v2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
-        gemm32(c, w->g2, 0, LTX_H, (const float*)b.attn_in, T, (float*)b.glog2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "ltx_gate:2");
+        gate32(c, w->g2, (const float*)b.attn_in, T, (float*)b.glog2, st, "ltx_gate:2");
         qknorm32(c, (float*)b.q2, w->qn2.p, nullptr, nullptr, T, st);
         qknorm32(c, (float*)b.k2, w->kn2.p, nullptr, nullptr, S, st);
         attn32(c, (const float*)b.q2, (const float*)b.k2, (const float*)b.v2, (const float*)b.glog2, (float*)b.o2, T, S, st, "attn:cross");

@@ -147,7 +147,6 @@ struct ltx_ctx {
     ltx::StreamScratch op_scratch;
     ltx::DevBuf blob_stage;  // device copy of the blob image of the last streaming upload
     ltx::DevBuf core_ws;   // conditioning MLP rows
-    ltx::DevBuf tail_ws;   // normed rows of ltx_core_tail
     ltx::DevBuf dn_ws;     // the denoising loop's activations
     size_t ws_T = 0, ws_S = 0;
     int ws_mode = -1;

@@ -253,7 +253,6 @@ void ltx_destroy(ltx_ctx* c) {
     c->op_q.free_();
     c->blob_stage.free_();
     c->core_ws.free_();
-    c->tail_ws.free_();
     c->dn_ws.free_();
     for (hipModule_t m : c->modules) (void)hipModuleUnload(m);
     delete c;

@@ -188,37 +188,237 @@ CORE_ROWS_KERNEL(4)
 CORE_ROWS_KERNEL(6)
 CORE_ROWS_KERNEL(8)
 
-// Output tail norm (ltx/core_parts.zig:26-35, 143-147): mean-subtracting
-// LayerNorm without weight, biased variance, eps 1e-6, then
-// n * (1 + (fsst[1] + e)) + (fsst[0] + e) with e = emb[tidx[t]]. One
-// workgroup of 256 threads per row.
-extern "C" __global__ void __launch_bounds__(256) ltx_core_tail_norm(const LtxTailNormArgs a) {
-    __shared__ float red[4];
-    const int t = blockIdx.x;
-    const float* x = a.x + (size_t)t * LTX_D;
-    float v[16];
-    float s = 0.f;
+// Output tail (ltx/core_parts.zig:26-35, 143-166): mean-subtracting LayerNorm
+// without weight, biased variance, eps 1e-6, then n * (1 + (fsst[1] + e)) +
+// (fsst[0] + e) with e = emb[tidx[t]], times w^T [4096 -> 128] + bias.
+// Bound by reading x. A workgroup of 8 waves takes 32 tokens: their statistics
+// first, four whole rows a wave; then 256 channels of all of them a step, 32 a
+// wave (x a second time, out of the last-level cache: the 32 rows in registers
+// would fill them all), normalised, split into three bf16 planes (exact) and
+// multiplied with w on bf16 MFMAs, two steps' w and x in flight; the waves'
+// partial sums are added in LDS, 16 tokens at a time.
+// The modulation rows of a tile whose tokens share one timestep row (all but
+// the tiles where the mask changes) are formed once, in LDS. (With the norm a
+// launch of its own and the product on the f32 GEMM's T / 128 workgroups, 7,920
+// tokens took 57 + 288 us; now 84.)
+__shared__ __attribute__((aligned(16))) float tail_mod[2 * LTX_D];  // 1 + scale, shift
+__shared__ __attribute__((aligned(16))) float tail_part[8][16][LTX_IN_CH + 4];
+__shared__ float tail_mean[32], tail_rstd[32];
+
+template <bool ONE>  // one timestep row in the tile
+__device__ __forceinline__ void tail_product(const LtxTailArgs& a, int t0, f32x4 (&acc)[2][8]) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int c0 = 32 * w + 8 * lg;  // the lane's channels: c0 + 256 ks + 0 .. 7
+    const float* x[2];
+    const float* e[2];
+    float mean[2], r[2];
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        v[i] = x[threadIdx.x + 256 * i];
-        s += v[i];
+    for (int tb = 0; tb < 2; tb++) {
+        const int t = min(t0 + 16 * tb + lr, a.T - 1);
+        x[tb] = a.x + (size_t)t * LTX_D + c0;
+        e[tb] = a.emb + (size_t)a.tidx[t] * LTX_D + c0;
+        mean[tb] = tail_mean[16 * tb + lr];
+        r[tb] = tail_rstd[16 * tb + lr];
     }
-    const float mean = block_sum256(s, red) / (float)LTX_D;
-    float q = 0.f;
+    const uint16_t* pw = a.w + (size_t)lr * LTX_D + c0;  // row 16 nb + lr of w
+    // two steps of x and w in flight: a step's x is reloaded as soon as its
+    // planes are formed, its w after its MFMAs
+    u32x4 wf[2][8];
+    f32x4 xr[2][2][2];
+    auto load_w = [&](int b, int ks) {
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        v[i] -= mean;
-        q += v[i] * v[i];
+        for (int nb = 0; nb < 8; nb++) wf[b][nb] = *(const u32x4*)(pw + (size_t)16 * nb * LTX_D + 256 * ks);
+    };
+    auto load_x = [&](int b, int ks) {
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) xr[b][tb][h] = *(const f32x4*)(x[tb] + 256 * ks + 4 * h);
+    };
+    auto step = [&](int b, int ks) {
+        u32x4 p[2][3];
+        f32x4 m1[2], m0[2];
+        if (ONE)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                m1[h] = *(const f32x4*)(tail_mod + c0 + 256 * ks + 4 * h);
+                m0[h] = *(const f32x4*)(tail_mod + LTX_D + c0 + 256 * ks + 4 * h);
+            }
+#pragma unroll
+        for (int tb = 0; tb < 2; tb++) {
+            float y[8];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                if (!ONE) {
+                    const f32x4 ev = *(const f32x4*)(e[tb] + 256 * ks + 4 * h);
+                    m1[h] = 1.0f + (*(const f32x4*)(a.fsst + LTX_D + c0 + 256 * ks + 4 * h) + ev);
+                    m0[h] = *(const f32x4*)(a.fsst + c0 + 256 * ks + 4 * h) + ev;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; i++) y[4 * h + i] = (xr[b][tb][h][i] - mean[tb]) * r[tb] * m1[h][i] + m0[h][i];
+            }
+            split3(y, p[tb]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_x(b, min(ks + 2, 15));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+                for (int nb = 0; nb < 8; nb++)
+                    acc[tb][nb] = Op<__bf16>::mfma16(__builtin_bit_cast(bf16x8, p[tb][q]),
+                                                     __builtin_bit_cast(bf16x8, wf[b][nb]), acc[tb][nb]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(b, min(ks + 2, 15));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load_x(0, 0);
+    load_w(0, 0);
+    load_x(1, 1);
+    load_w(1, 1);
+    for (int ks = 0; ks < 16; ks += 2) {
+        step(0, ks);
+        step(1, ks + 1);
     }
-    const float var = block_sum256(q, red) / (float)LTX_D;
-    const float r = 1.0f / sqrtf(var + 1e-6f);
-    const float* e = a.emb + (size_t)a.tidx[t] * LTX_D;
-    float* y = a.y + (size_t)t * LTX_D;
+}
+
+extern "C" __global__ void __launch_bounds__(512, 2) ltx_core_tail(const LtxTailArgs a) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int t0 = blockIdx.x * 32;
+    // statistics of rows 4 w .. 4 w + 3, two at a time
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int c = threadIdx.x + 256 * i;
-        const float scl = a.fsst[LTX_D + c] + e[c], shift = a.fsst[c] + e[c];
-        y[c] = v[i] * r * (1.0f + scl) + shift;
+    for (int g = 0; g < 2; g++) {
+        f32x4 v[2][16];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const float* x = a.x + (size_t)min(t0 + 4 * w + 2 * g + k, a.T - 1) * LTX_D + 4 * lane;
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[k][i] = *(const f32x4*)(x + 256 * i);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            auto sum = [](f32x4 s4) {
+                float s = (s4[0] + s4[1]) + (s4[2] + s4[3]);
+                for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+                return s;
+            };
+            f32x4 s4 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 16; i++) s4 += v[k][i];
+            const float mean = sum(s4) / (float)LTX_D;
+            s4 = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const f32x4 d = v[k][i] - mean;
+                s4 += d * d;
+            }
+            const float var = sum(s4) / (float)LTX_D;
+            if (lane == 0) {
+                tail_mean[4 * w + 2 * g + k] = mean;
+                tail_rstd[4 * w + 2 * g + k] = 1.0f / sqrtf(var + 1e-6f);
+            }
+        }
+    }
+    const int k0 = a.tidx[t0];
+    const bool one = __builtin_amdgcn_ballot_w64(a.tidx[min(t0 + (lane & 31), a.T - 1)] != k0) == 0;  // the same in every wave
+    if (one) {
+        const float* e = a.emb + (size_t)k0 * LTX_D;
+        for (int c = 4 * tid; c < LTX_D; c += 2048) {
+            const f32x4 ev = *(const f32x4*)(e + c);
+            *(f32x4*)(tail_mod + c) = 1.0f + (*(const f32x4*)(a.fsst + LTX_D + c) + ev);
+            *(f32x4*)(tail_mod + LTX_D + c) = *(const f32x4*)(a.fsst + c) + ev;
+        }
+    }
+    __syncthreads();
+    f32x4 acc[2][8];
+#pragma unroll
+    for (int tb = 0; tb < 2; tb++)
+#pragma unroll
+        for (int nb = 0; nb < 8; nb++) acc[tb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (one)
+        tail_product<true>(a, t0, acc);
+    else
+        tail_product<false>(a, t0, acc);
+    // acc[tb][nb][i]: token 16 tb + 4 lg + i, column 16 nb + lr
+    const int row = tid >> 5, c = 4 * (tid & 31);
+#pragma unroll
+    for (int tb = 0; tb < 2; tb++) {
+        if (tb) __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < 8; nb++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) tail_part[w][4 * lg + i][16 * nb + lr] = acc[tb][nb][i];
+        __syncthreads();
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; i++) o += *(const f32x4*)&tail_part[i][row][c];
+        const int t = t0 + 16 * tb + row;
+        if (t < a.T) {
+            float* dst = a.vel + (size_t)t * LTX_IN_CH + c;  // (of any 4-byte alignment)
+#pragma unroll
+            for (int i = 0; i < 4; i++) dst[i] = o[i] + a.bias[c + i];
+        }
+    }
+}
+
+// Patchify (ltx/core_parts.zig:112-121): x = lat . w^T + bias, 128 -> 4096.
+// Bound by writing x. A workgroup of 8 waves takes 64 tokens and 512 columns:
+// the latents go to LDS once as three bf16 planes (exact), each wave holds the
+// weights of its 64 columns in registers, and the loop over the token blocks
+// then reads LDS only. (With weights loaded in a loop over the columns, each
+// load's wait also waited for the stores before it: 59 us against 41 at 7,920
+// tokens; on the f32 GEMM 95.) w's rows are the MFMA's A operand, so a lane's results are four
+// consecutive columns of one token.
+// LDS rows of 256 B a token and plane, 16-byte chunk c of token t in slot
+// c ^ (t & 15): the 16 tokens of a fragment read cover all banks.
+extern "C" __global__ void __launch_bounds__(512, 4) ltx_core_patchify(const LtxPatchifyArgs a) {
+    __shared__ __attribute__((aligned(16))) uint8_t planes[3][64 * 256];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int t0 = blockIdx.x * 64, n0 = 512 * blockIdx.y + 64 * w;
+    u32x4 wf[4][4];  // [16 columns][32 channels]
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++)
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+            wf[nb][ks] = *(const u32x4*)(a.w + (size_t)(n0 + 16 * nb + lr) * LTX_IN_CH + 32 * ks + 8 * lg);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int id = tid + 512 * i, t = id >> 4, c = id & 15;  // chunk c (8 channels) of token t0 + t
+        const float* l = a.lat + (size_t)min(t0 + t, a.T - 1) * LTX_IN_CH + 8 * c;
+        const f32x4 l0 = *(const f32x4*)l, l1 = *(const f32x4*)(l + 4);
+        u32x4 p[3];
+        split3({l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]}, p);
+#pragma unroll
+        for (int q = 0; q < 3; q++) *(u32x4*)(planes[q] + 256 * t + 16 * (c ^ (t & 15))) = p[q];
+    }
+    f32x4 b[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++) b[nb] = *(const f32x4*)(a.bias + n0 + 16 * nb + 4 * lg);
+    __syncthreads();
+#pragma unroll
+    for (int tb = 0; tb < 4; tb++) {
+        f32x4 acc[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; nb++) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) {
+                const u32x4 f = *(const u32x4*)(planes[q] + 256 * (16 * tb + lr) + 16 * ((4 * ks + lg) ^ lr));
+#pragma unroll
+                for (int nb = 0; nb < 4; nb++)
+                    acc[nb] = Op<__bf16>::mfma16(__builtin_bit_cast(bf16x8, wf[nb][ks]), __builtin_bit_cast(bf16x8, f),
+                                                 acc[nb]);
+            }
+        const int t = t0 + 16 * tb + lr;
+        if (t < a.T)
+#pragma unroll
+            for (int nb = 0; nb < 4; nb++) *(f32x4*)(a.x + (size_t)t * LTX_D + n0 + 16 * nb + 4 * lg) = acc[nb] + b[nb];
     }
 }
 

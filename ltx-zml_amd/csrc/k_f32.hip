@@ -324,3 +324,42 @@ extern "C" __global__ void __launch_bounds__(512) ltx_attn_f32(const LtxAttn32Ar
             f32x4{o[4][r] / lsum * g, o[5][r] / lsum * g, o[6][r] / lsum * g, o[7][r] / lsum * g};
     }
 }
+
+// Gate logits in mode F32: glog[t][h] = a[t] . gw[h] + gb[h], 32 heads, gw
+// bf16. Bound by reading a. A workgroup of 8 waves takes 16 rows, each wave
+// 512 of the 4,096 channels: a's values are split into three bf16 planes (exact)
+// in the layout of the MFMA's A operand, and the waves' sums meet in LDS. (As
+// one 128-column tile of the f32 GEMM above it had rows / 128 workgroups: at
+// 1,024 rows 283 us, now 17.)
+extern "C" __global__ void __launch_bounds__(512) ltx_gate_f32(const LtxGate32Args a) {
+    __shared__ float part[8][16][LTX_H + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int m0 = blockIdx.x * 16, c0 = 512 * w + 8 * lg;
+    const float* x = a.a + (size_t)min(m0 + lr, a.M - 1) * LTX_D + c0;
+    const uint16_t* g = a.gw + (size_t)lr * LTX_D + c0;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll 8
+    for (int ks = 0; ks < 16; ks++) {
+        const f32x4 x0 = *(const f32x4*)(x + 32 * ks), x1 = *(const f32x4*)(x + 32 * ks + 4);
+        u32x4 wf[2], p[3];
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++) wf[nb] = *(const u32x4*)(g + 16 * nb * LTX_D + 32 * ks);
+        split3({x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]}, p);
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+                acc[nb] = Op<__bf16>::mfma16(__builtin_bit_cast(bf16x8, p[q]), __builtin_bit_cast(bf16x8, wf[nb]), acc[nb]);
+    }
+#pragma unroll
+    for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) part[w][4 * lg + i][16 * nb + lr] = acc[nb][i];
+    __syncthreads();
+    const int row = tid >> 5, h = tid & 31;
+    float o = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; i++) o += part[i][row][h];
+    if (m0 + row < a.M) a.out[(size_t)(m0 + row) * LTX_H + h] = o + a.gb[h];
+}

@@ -19,6 +19,7 @@ extern "C" {
 #define LTX_HD 128
 #define LTX_FF 16384
 #define LTX_GROUP 128
+#define LTX_IN_CH 128
 
 // AdaLN gather (ltx/block.zig:47-67): ada_i[t][c] = tstab[row(t)][i][c] + sst[i][c],
 // row(t) = tidx[t] when it lies in 1 .. K-1, else 0 (the reference's select
@@ -192,6 +193,15 @@ typedef struct {
     int M;
 } LtxGateArgs;
 
+// The same in mode F32: a f32, gw bf16.
+typedef struct {
+    const float* a;      // [M][D]
+    const uint16_t* gw;  // [H][D]
+    const float* gb;     // [H]
+    float* out;          // [M][H]
+    int M;
+} LtxGate32Args;
+
 // Dequantisation probe: out[n][k] = f32(q[n][k]) * scale[n][k/128], exactly
 // as the GEMM's in-register dequant computes it before the 16-bit rounding.
 typedef struct {
@@ -299,8 +309,19 @@ typedef struct {
     const float* fsst;    // [2][D] (shift row, scale row)
     const float* emb;     // [K][D] embedded timestep per distinct t
     const int32_t* tidx;  // [T]
-    float* y;             // [T][D]
-} LtxTailNormArgs;
+    const uint16_t* w;    // [128][D] bf16
+    const float* bias;    // [128]
+    float* vel;           // [T][128]
+    int T;
+} LtxTailArgs;
+
+typedef struct {
+    const float* lat;     // [T][128]
+    const uint16_t* w;    // [D][128] bf16
+    const float* bias;    // [D]
+    float* x;             // [T][D]
+    int T;
+} LtxPatchifyArgs;
 
 typedef struct {
     const float* x;       // latent [T][stride]

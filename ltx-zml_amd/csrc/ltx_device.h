@@ -165,6 +165,27 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
     return s;
 }
 
+// x = p[0] + p[1] + p[2] exactly, each a bf16: p[0] the bits of x down to the
+// eighth significant one, p[1] the same of the rest, p[2] what is left (at most
+// 8 significant bits). An infinity is its own first plane with nothing left
+// (inf - inf would leave a NaN); a NaN leaves one in the second plane.
+__device__ __forceinline__ void split3(const float (&x)[8], u32x4 (&p)[3]) {
+    uint32_t h[8], m[8], l[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        h[e] = __builtin_bit_cast(uint32_t, x[e]) & 0xffff0000u;
+        const float r = __builtin_isinf(x[e]) ? 0.0f : x[e] - __builtin_bit_cast(float, h[e]);
+        m[e] = __builtin_bit_cast(uint32_t, r) & 0xffff0000u;
+        l[e] = __builtin_bit_cast(uint32_t, r - __builtin_bit_cast(float, m[e]));
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {  // the upper halves of a pair
+        p[0][e] = __builtin_amdgcn_perm(h[2 * e + 1], h[2 * e], 0x07060302u);
+        p[1][e] = __builtin_amdgcn_perm(m[2 * e + 1], m[2 * e], 0x07060302u);
+        p[2][e] = __builtin_amdgcn_perm(l[2 * e + 1], l[2 * e], 0x07060302u);
+    }
+}
+
 // GELU, tanh form: 0.5 x (1 + tanh(u)), u = sqrt(2/pi) (x + 0.044715 x^3),
 // evaluated through the exact identity 0.5 (1 + tanh u) = 1 / (1 + exp(-2u)):
 // x / (1 + 2^(-2u log2 e)). No subtraction, so no cancellation for negative

@@ -149,6 +149,13 @@ def test_patchify_and_tail(ctx, core_np, core_dev, T):
     assert r_wrong > 1e-3
 
 
+@pytest.mark.parametrize("T", [1, 17, 4100])
+def test_patchify_and_tail_edges(ctx, core_np, core_dev, T):
+    """One token, one past a 16-token tile, and enough ragged 32-token tiles to
+    share out the columns over fewer workgroups."""
+    test_patchify_and_tail(ctx, core_np, core_dev, T)
+
+
 @pytest.fixture(scope="module")
 def denoise_case(core_np):
     """Two blocks, the last three stage-2 steps (0.909375 -> 0.725 -> 0.421875
