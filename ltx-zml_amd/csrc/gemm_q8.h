@@ -217,7 +217,9 @@ struct Q8Op<__bf16, false> : Q8Mfma<__bf16> {
 // Raw buffer descriptor word 3 for gfx9-family parts (untyped dword access).
 #define Q8_RSRC_W3 0x00020000
 
-template <typename T, bool SF32, int EPI>
+// RAW: the weights as packed (two's complement); their sign bits are flipped
+// after the LDS read, one XOR for four weights.
+template <typename T, bool SF32, int EPI, bool RAW>
 struct Q8Gemm {
     typedef Q8Op<T, SF32> QO;
     static constexpr int NI = 4, NJ = 2;
@@ -263,6 +265,7 @@ struct Q8Gemm {
         for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int c = 0; c < 2; c++) wb[j][c] = *(const u32x4*)(sb + offb[c] + 2048 * j);
+        constexpr uint32_t kX = RAW ? 0x80808080u : 0u;
 #pragma unroll
         for (int i = 0; i < NI; i++)
 #pragma unroll
@@ -287,7 +290,7 @@ struct Q8Gemm {
 #pragma unroll
                 for (int j = 0; j < NJ; j++) {
                     const u32x4 w = wb[j][t >> 1];
-                    fb0[t][j] = (t & 1) ? QO::deq8(w[2], w[3], s2[j]) : QO::deq8(w[0], w[1], s2[j]);
+                    fb0[t][j] = (t & 1) ? QO::deq8(w[2] ^ kX, w[3] ^ kX, s2[j]) : QO::deq8(w[0] ^ kX, w[1] ^ kX, s2[j]);
                 }
             if (g == 1) wait_dma(more2);
             __builtin_amdgcn_sched_barrier(0);
@@ -306,7 +309,7 @@ struct Q8Gemm {
                 if (t < DQ)
                     fb[j] = fb0[t < DQ ? t : 0][j];
                 else
-                    fb[j] = (t & 1) ? QO::deq8(w[2], w[3], s2[j]) : QO::deq8(w[0], w[1], s2[j]);
+                    fb[j] = (t & 1) ? QO::deq8(w[2] ^ kX, w[3] ^ kX, s2[j]) : QO::deq8(w[0] ^ kX, w[1] ^ kX, s2[j]);
             }
 #pragma unroll
             for (int i = 0; i < NI; i++)
@@ -427,8 +430,8 @@ struct Q8Gemm {
     }
 };
 
-#define Q8_GEMM_KERNEL(NAME, T_, SF32_, EPI_)                                                \
+#define Q8_GEMM_KERNEL(NAME, T_, SF32_, EPI_, RAW_)                                          \
     extern "C" __global__ void __launch_bounds__(512, 1) NAME(const LtxGemmArgs a) {         \
-        Q8Gemm<T_, SF32_, EPI_> k(a);                                                  \
+        Q8Gemm<T_, SF32_, EPI_, RAW_> k(a);                                                  \
         k.run();                                                                             \
     }

@@ -91,10 +91,14 @@ __device__ __forceinline__ void gemm_store_partial_patch(Fill fill, float* patch
     }
 }
 
-template <typename T, int BK, int EPI>
+// RAW: the int8 weights as packed (two's complement); their sign bits are
+// flipped after the LDS read, one XOR for four weights, where a pass over the
+// weights that flips them first would read and write each once more.
+template <typename T, int BK, int EPI, bool RAW>
 struct S4Gemm {
     static constexpr bool Q = BK != LTX_B_W16;
     static constexpr bool SF32 = BK == LTX_B_I8_F32S;
+    static constexpr uint32_t kX = RAW ? 0x80808080u : 0u;
     static constexpr int NDB = Q ? 2 : 4;             // W DMA instructions per wave and tile (A: 4)
     static constexpr int NV = 4 + NDB + (Q ? 1 : 0);  // DMA instructions per wave and tile (+1: scale words)
     typedef Q8Op<T, SF32> QO;
@@ -163,7 +167,7 @@ struct S4Gemm {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if constexpr (Q)
-                xb[j] = QO::deq8(w[j][0], w[j][1], QO::scale(sc[j]));
+                xb[j] = QO::deq8(w[j][0] ^ kX, w[j][1] ^ kX, QO::scale(sc[j]));
             else
                 xb[j] = __builtin_bit_cast(V8, w[j]);
         }
@@ -361,8 +365,8 @@ struct S4Gemm {
     }
 };
 
-#define S4_GEMM_KERNEL(NAME, T_, BK_, EPI_)                                          \
+#define S4_GEMM_KERNEL(NAME, T_, BK_, EPI_, RAW_)                                    \
     extern "C" __global__ void __launch_bounds__(256, 2) NAME(const LtxGemmArgs a) { \
-        S4Gemm<T_, BK_, EPI_> k(a);                                                  \
+        S4Gemm<T_, BK_, EPI_, RAW_> k(a);                                            \
         k.run();                                                                     \
     }

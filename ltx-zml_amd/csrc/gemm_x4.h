@@ -278,8 +278,16 @@ __device__ __forceinline__ void dq16_body(const LtxDq16Args& a) {
     const int n = 32 * nb + (threadIdx.x >> 3);
     const int k = LTX_GROUP * g + 16 * (threadIdx.x & 7);
     if (n >= a.N[j]) return;
-    const u32x4 w = *(const u32x4*)(a.q[j] + (size_t)n * a.K[j] + k);
-    const typename QO::Scale s = QO::scale(a.s2[j][(size_t)g * a.N[j] + n]);
+    u32x4 w = *(const u32x4*)(a.q[j] + (size_t)n * a.K[j] + k);
+    uint32_t word;
+    if (a.raw) {  // weights and scales as packed: no pass that lays them out first
+        w ^= 0x80808080u;
+        const size_t i = (size_t)n * G + g;
+        word = SF32 ? a.s2[j][i] : ((const uint16_t*)a.s2[j])[i] * 0x10001u;
+    } else {
+        word = a.s2[j][(size_t)g * a.N[j] + n];
+    }
+    const typename QO::Scale s = QO::scale(word);
     const typename QO::V8 lo = QO::deq8(w[0], w[1], s), hi = QO::deq8(w[2], w[3], s);
     u32x4* out = (u32x4*)((uint16_t*)a.out[j] + (size_t)n * a.K[j] + k);
     out[0] = __builtin_bit_cast(u32x4, lo);

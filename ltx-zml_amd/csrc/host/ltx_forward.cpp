@@ -82,7 +82,7 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
 // and below that its split-K fills the chip where the other has N / 128
 // workgroups a row tile.
 bool f3_shape(const ltx_ctx* c, int M, int N, int K) {
-    return c->gemm_f3 && M > 0 && N % 128 == 0 && K % 128 == 0 && (uint64_t)M * K * 2 < (1ull << 31) &&
+    return c->gemm_f3 && M > 0 && N % 128 == 0 && K % 128 == 0 && K <= (1 << 15) && (uint64_t)M * K * 2 < (1ull << 31) &&
            (uint64_t)N * K * 2 < (1ull << 31);
 }
 // Its scratch: the three planes of A, and the split-K partial sums (0: no split).
@@ -274,7 +274,7 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
     // out for the LDS-DMA kernels (bytes q + 128, scale words) or 16-bit
     // weights; split K only while even those tiles fill at most half the CUs
     {
-        const void* wb = p.q8 ? (p.qflip && p.s2.p ? p.q.p : nullptr) : (mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p);
+        const void* wb = p.q8 ? ((p.qflip || p.qraw) && p.s2.p ? p.q.p : nullptr) : (mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p);
         if (wb && s4_shape(c, mode, M, p.N, p.K, lda, p.q8) && g.ldo % 8 == 0 && al16(A) && al16(wb) && al16(g.out) &&
             al16(g.out2) && al16(g.resid) && al16(g.bias) && al16(g.ada.tstab) && al16(g.ada.sst)) {
             g.b = wb;
@@ -282,8 +282,8 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
             g.tiles_m = (M + 127) / 128;
             g.tiles_n = p.N / 128;
             g.ksplit = g.part ? gemm_ksplit(c->num_cu, M, p.N, p.K, 128, 128) : 1;
-            std::snprintf(name, sizeof(name), "ltx_gemm_s4_%s_%s_%s", msuffix(mode),
-                          p.q8 ? (p.scale_f16 ? "i8f16" : "i8f32") : "w16", es);
+            std::snprintf(name, sizeof(name), "ltx_gemm_s4_%s_%s_%s%s", msuffix(mode),
+                          p.q8 ? (p.scale_f16 ? "i8f16" : "i8f32") : "w16", es, p.qraw ? "_raw" : "");
             const int nitems = g.tiles_m * g.tiles_n * g.ksplit;
             c->launch(name, c->gemm_persistent ? std::min(nitems, 2 * c->num_cu) : nitems, 1, 1, 256, &g, st, label);
             if (g.ksplit > 1) {
@@ -295,13 +295,13 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
     }
     // LDS-DMA int8 kernel: f16 or bf16 operands, f16 scales, K a multiple of
     // 128, and byte offsets of A and W within 31 bits (32-bit buffer offsets)
-    if ((mode == LTX_MODE_F16 || mode == LTX_MODE_BF16) && p.q8 && p.qflip && p.s2.p &&
+    if ((mode == LTX_MODE_F16 || mode == LTX_MODE_BF16) && p.q8 && (p.qflip || p.qraw) && p.s2.p &&
         c->gemm_dma && p.K % 128 == 0 && (uint64_t)M * lda * 2 < (1ull << 31) && (uint64_t)p.N * p.K < (1ull << 31) && g.ldo % 8 == 0 &&
         al16(g.out) && al16(g.out2) && al16(g.resid) && al16(g.bias) && al16(g.ada.tstab) && al16(g.ada.sst)) {
         // (its epilogue moves 16-byte vectors: outputs, residual and bias 16-byte aligned)
         g.scales = p.s2.p;
-        std::snprintf(name, sizeof(name), "ltx_gemm_q8_%s%s%s", mode == LTX_MODE_BF16 ? "bf16_" : "",
-                      p.scale_f16 ? "" : "s32_", es);
+        std::snprintf(name, sizeof(name), "ltx_gemm_q8_%s%s%s%s", mode == LTX_MODE_BF16 ? "bf16_" : "",
+                      p.scale_f16 ? "" : "s32_", es, p.qraw ? "_raw" : "");
         // few output tiles: split K over more workgroups (when the caller
         // gave a buffer for the partial sums), then reduce + epilogue
         g.ksplit = g.part ? gemm_ksplit(c->num_cu, M, p.N, p.K) : 1;
@@ -354,10 +354,12 @@ static void dequant16(ltx_ctx* c, int mode, const LtxProj* const* p, void* const
         for (int i = 0; i < n; i++) {
             if (sf == 0) done[i] = nullptr;
             const LtxProj& q = *p[i];
-            if (!out[i] || !q.q8 || !q.qflip || !q.s2.p || (q.scale_f16 ? 0 : 1) != sf) continue;
+            if (!out[i] || !q.q8 || (q.scale_f16 ? 0 : 1) != sf) continue;
+            if (!q.qraw && (!q.qflip || !q.s2.p)) continue;
             const int j = a.njobs++;
+            a.raw = q.qraw;  // (of one job: the isolated GEMM)
             a.q[j] = (const uint8_t*)q.q.p;
-            a.s2[j] = (const uint32_t*)q.s2.p;
+            a.s2[j] = (const uint32_t*)(q.qraw ? q.s.p : q.s2.p);
             a.out[j] = out[i];
             a.N[j] = q.N;
             a.K[j] = q.K;
@@ -470,7 +472,7 @@ static void split3(ltx_ctx* c, const float* A, int M, int K, void* planes, hipSt
 // partial sums (f3_part_bytes) or NULL.
 static void gemm32(ltx_ctx* c, const LtxProj& p, int r0, int N, const float* A, int M, float* out, int epi,
                    const float* resid, LtxAda ada, int igate, int gelu, hipStream_t st, const char* label = nullptr,
-                   const void* planes = nullptr, void* part = nullptr) {
+                   const void* planes = nullptr, void* part = nullptr, int ksplit = 0) {
     const size_t G = p.K / LTX_GROUP;
     const void *wb, *ws = nullptr;
     if (p.q8) {
@@ -507,7 +509,7 @@ static void gemm32(ltx_ctx* c, const LtxProj& p, int r0, int N, const float* A, 
         g.qxor = qxor;
         g.tiles_m = (M + 127) / 128;
         g.tiles_n = N / 128;
-        g.ksplit = part ? gemm_ksplit(c->num_cu, M, N, p.K, 128, 128) : 1;
+        g.ksplit = !part ? 1 : ksplit ? ksplit : gemm_ksplit(c->num_cu, M, N, p.K, 128, 128);
         g.part = (float*)part;
         const char* es = epi == LTX_EPI_RESID_GATE ? "resid" : "store";
         char name[48];
@@ -819,9 +821,21 @@ bool linear_q8_needs_scratch(const ltx_ctx* c, int N, int K, int mode) {
     return mode != LTX_MODE_F32 && c->gemm_dma && N % 256 == 0;
 }
 
-// ltx_op_linear_q8 / _noalloc: in the 16-bit modes with the LDS-DMA kernel the
-// weights are first laid out as bytes q + 128 in sc.q and the scales as words
-// [K/128][N] in sc.pairs (both written whole before the GEMM reads them).
+bool linear_aligned(const void* a, const void* q, const void* bias, const void* y) {
+    return (((uintptr_t)a | (uintptr_t)q | (uintptr_t)bias | (uintptr_t)y) & 15) == 0;
+}
+
+size_t linear_part_bytes(const ltx_ctx* c, int M, int N, int K, int mode) {
+    if (!linear_q8_needs_scratch(c, N, K, mode) || x4_shape(c, mode, M, N, K, K)) return 0;
+    const int t = s4_shape(c, mode, M, N, K, K, true) ? 128 : 256, s = gemm_ksplit(c->num_cu, M, N, K, t, t);
+    return s > 1 ? (size_t)s * M * N * 4 : 0;
+}
+
+// ltx_op_linear_q8 / _noalloc: in the 16-bit modes with the LDS-DMA kernels the
+// scales are first laid out as words [K/128][N] in sc.pairs, and weights (or
+// other operands) that are not 16-byte aligned as bytes q + 128 in sc.q, which
+// at 16,384 x 4,096 weights took 28 us of a call (all written whole before the
+// GEMM reads them). The four-wave kernel's dequantisation reads both as packed.
 void check_linear_q8(int M, int N, int K, int mode) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) throw Error("bad GEMM shape (K must be a multiple of 128)");
     if (mode != LTX_MODE_F16 && mode != LTX_MODE_BF16 && mode != LTX_MODE_F32) throw Error("unknown mode");
@@ -845,28 +859,43 @@ void linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, i
         if (mode == LTX_MODE_F32) {
             if (!out_f32) throw Error("mode F32 writes f32 output");
             LtxAda ada{};
-            const bool f3 = sc.planes && ((uintptr_t)a & 15) == 0;
-            if (f3) split3(c, (const float*)a, M, K, sc.planes, st);
-            gemm32(c, p, 0, N, (const float*)a, M, (float*)y, LTX_EPI_STORE, nullptr, ada, 0, gelu, st, nullptr,
-                   f3 ? sc.planes : nullptr, sc.part);
+            const bool f3 = sc.planes && linear_aligned(a, q, bias, y);
+            // as many rows at a time as the scratch takes, split K as for all
+            // of them (the same bits)
+            const int ks = gemm_ksplit(c->num_cu, M, N, K, 128, 128), step = f3 ? sc.plane_rows : M;
+            for (int r = 0; r < M; r += step) {
+                const int m = std::min(step, M - r);
+                const float* ar = (const float*)a + (size_t)r * K;
+                if (f3) split3(c, ar, m, K, sc.planes, st);
+                gemm32(c, p, 0, N, ar, m, (float*)y + (size_t)r * N, LTX_EPI_STORE, nullptr, ada, 0, gelu, st, nullptr,
+                       f3 ? sc.planes : nullptr, sc.part, ks);
+            }
         } else {
-            if (linear_q8_needs_scratch(c, N, K, mode)) {
-                if (!sc.q || !sc.pairs) throw Error("linear_q8: no scratch");
-                // the LDS-DMA kernel reads scale words [K/128][N]
-                const size_t n2 = (size_t)N * (K / LTX_GROUP);
-                LtxPairArgs pa{scales, sc.pairs, N, K / LTX_GROUP, scale_f16 ? 0 : 1};
-                c->launch("ltx_scale_pairs", (unsigned)((n2 + 255) / 256), 1, 1, 256, &pa, st);
-                p.s2.p = sc.pairs;
-                // and its weights as the bytes q + 128
-                const size_t nq = (size_t)N * K / 4;
-                LtxFlipArgs fa{(const uint32_t*)q, sc.q, nq};
-                c->launch("ltx_q8_flip", (unsigned)((nq + 255) / 256), 1, 1, 256, &fa, st);
-                p.q.p = sc.q;
-                p.qflip = true;
+            const bool scratch = linear_q8_needs_scratch(c, N, K, mode);
+            const bool x4 = scratch && sc.w16 && x4_shape(c, mode, M, N, K, K);
+            if (scratch) {
+                // aligned operands: the kernels take the weights as packed
+                p.qraw = linear_aligned(a, q, bias, y);
+                if (!sc.pairs || (!p.qraw && !sc.q)) throw Error("linear_q8: no scratch");
+                if (!p.qraw || !x4) {
+                    // the LDS-DMA kernel reads scale words [K/128][N]
+                    const size_t n2 = (size_t)N * (K / LTX_GROUP);
+                    LtxPairArgs pa{scales, sc.pairs, N, K / LTX_GROUP, scale_f16 ? 0 : 1};
+                    c->launch("ltx_scale_pairs", (unsigned)((n2 + 255) / 256), 1, 1, 256, &pa, st);
+                    p.s2.p = sc.pairs;
+                }
+                if (!p.qraw) {
+                    // and its weights as the bytes q + 128
+                    const size_t nq = (size_t)N * K / 4;
+                    LtxFlipArgs fa{(const uint32_t*)q, sc.q, nq};
+                    c->launch("ltx_q8_flip", (unsigned)((nq + 255) / 256), 1, 1, 256, &fa, st);
+                    p.q.p = sc.q;
+                    p.qflip = true;
+                }
             }
             // the four-wave kernel on the weights dequantised into sc.w16
             const void* w16 = nullptr;
-            if (sc.w16 && p.qflip && x4_shape(c, mode, M, N, K, K)) {
+            if (x4) {
                 const LtxProj* ps[1] = {&p};
                 void* outs[1] = {sc.w16};
                 dequant16(c, mode, ps, outs, 1, &w16, st);
@@ -876,6 +905,7 @@ void linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, i
             g.ldo = N;
             g.gelu = gelu;
             g.out_f32 = out_f32;
+            g.part = p.qraw ? (float*)sc.part : nullptr;
             gemm16(c, mode, p, a, M, K, LTX_EPI_STORE, g, st, nullptr, w16);
         }
     } catch (...) {
@@ -1007,18 +1037,22 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         ltx::LinearScratch sc{};
         hipStream_t st = (hipStream_t)stream;
         // mode F32 splits A into planes (not captured: then the f32 MFMA kernel)
-        bool f3 = false;
+        bool used = false;  // c->op_scratch
         if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
             const size_t np = ltx::f3_planes_bytes(M, K), need = np + ltx::f3_part_bytes(c, M, N, K);
             if ((sc.planes = c->op_scratch.take(need, st))) {
-                f3 = true;
+                used = true;
+                sc.plane_rows = M;
                 sc.part = need > np ? (char*)sc.planes + np : nullptr;
             }
         }
+        // 16-bit modes: split-K partial sums (not captured: then no split)
+        if (const size_t np = ltx::linear_aligned(a, q, bias, y) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0)
+            used = (sc.part = c->op_scratch.take(np, st)) != nullptr;
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
             // scratch owned by the context, grown as needed
             const size_t nq = (size_t)N * K, np = (size_t)N * (K / LTX_GROUP) * 4;
-            if (c->op_q.bytes < nq) c->op_q.alloc(nq);
+            if (!ltx::linear_aligned(a, q, bias, y) && c->op_q.bytes < nq) c->op_q.alloc(nq);
             if (c->op_pairs.bytes < np) c->op_pairs.alloc(np);
             sc.q = (uint32_t*)c->op_q.p;
             sc.pairs = (uint32_t*)c->op_pairs.p;
@@ -1028,7 +1062,7 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
             }
         }
         ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, st);
-        if (f3) c->op_scratch.done(st);
+        if (used) c->op_scratch.done(st);
     })
 }
 

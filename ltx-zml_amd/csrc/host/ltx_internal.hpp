@@ -70,6 +70,7 @@ struct LtxProj {
     int N = 0, K = 0;
     bool q8 = false;          // int8 + scales available
     bool qflip = false;       // q holds the bytes q + 128 (q XOR 0x80)
+    bool qraw = false;        // q as packed, 16-byte aligned: the _raw kernels (plain store) take it
     int scale_f16 = 0;
     ltx::DevBuf q;            // int8 [N][K]
     ltx::DevBuf s;            // [N][K/128] f32 or f16
@@ -195,8 +196,9 @@ float f16_bits_to_f32(uint16_t h);
 struct LinearScratch {
     uint32_t* q;
     uint32_t* pairs;
-    void* planes = nullptr;  // mode F32: f3_planes_bytes and f3_part_bytes, or NULL (the f32 MFMA kernel)
-    void* part = nullptr;
+    void* planes = nullptr;  // mode F32: f3_planes_bytes, or NULL (the f32 MFMA kernel)
+    int plane_rows = 0;      // rows of A that fit in planes (and their partial sums in part)
+    void* part = nullptr;    // split-K partial sums (linear_part_bytes) or NULL (no split)
     void* w16 = nullptr;  // N * K 16-bit weights for the four-wave GEMM, or NULL (the W8A16 kernel)
 };
 // Whether the four-wave 16-bit GEMM takes an M x N x K product with A rows of
@@ -209,6 +211,10 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
 bool f3_shape(const ltx_ctx* c, int M, int N, int K);
 size_t f3_planes_bytes(int M, int K);
 size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K);
+// Bytes of split-K partial sums of the isolated int8 GEMM in the 16-bit modes
+// (0: no split, or operands that are not 16-byte aligned).
+bool linear_aligned(const void* a, const void* q, const void* bias, const void* y);
+size_t linear_part_bytes(const ltx_ctx* c, int M, int N, int K, int mode);
 // Shape and mode checks of the isolated int8 GEMM (throws Error), made before
 // any scratch is sized from N and K.
 void check_linear_q8(int M, int N, int K, int mode);

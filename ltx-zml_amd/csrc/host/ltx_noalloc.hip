@@ -72,6 +72,32 @@ extern "C" int ltx_op_linear_q8_noalloc(ltx_ctx* c, const void* a, const int8_t*
             sc.pairs = (uint32_t*)(base + nq);
             sc.w16 = nw ? base + nq + np : nullptr;
         }
+        char* base = (char*)ltx::noalloc_scratch(c->device);
+        if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
+            // the planes of as many rows of A as fit, with their partial sums;
+            // at least 128: a split has at most 256 tiles x slices of 64 KB,
+            // and K is at most 32,768
+            const size_t part = ltx::f3_part_bytes(c, M, N, K);
+            int rows = M;
+            while (rows > 128 && ltx::f3_planes_bytes(rows, K) + (part ? part / M * rows : 0) > LTX_NOALLOC_SCRATCH_BYTES)
+                rows = (rows / 2 + 127) / 128 * 128;
+            const size_t np = ltx::f3_planes_bytes(rows, K);
+            if (!base) throw ltx::Error("ltx_op_linear_q8_noalloc: scratch not set up on this device");
+            if (np + (part ? part / M * rows : 0) > LTX_NOALLOC_SCRATCH_BYTES)
+                throw ltx::Error("ltx_op_linear_q8_noalloc: scratch too small for 128 rows");  // (cannot happen)
+            sc.planes = base;
+            sc.plane_rows = rows;
+            sc.part = part ? base + np : nullptr;
+        }
+        if (const size_t part = ltx::linear_aligned(a, q, bias, y) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0) {
+            // beside the scale words; the room of the bytes q + 128 is free
+            // (aligned operands). At most 64 MiB: 256 tiles x slices of 256 KB
+            const size_t np = ((size_t)N * (K / LTX_GROUP) * 4 + 255) & ~(size_t)255;
+            if (np + part > LTX_NOALLOC_SCRATCH_BYTES)
+                throw ltx::Error("ltx_op_linear_q8_noalloc: scratch too small for the partial sums");  // (cannot happen)
+            sc.pairs = (uint32_t*)base;
+            sc.part = base + np;
+        }
         HIPC(hipSetDevice(c->device));
         ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, (hipStream_t)stream);
     })

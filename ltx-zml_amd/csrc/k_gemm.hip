@@ -194,19 +194,24 @@ GEMM_KERNEL(ltx_gemm_bf16_w16_resid, __bf16, LTX_B_W16, LTX_EPI_RESID_GATE)
 GEMM_KERNEL(ltx_gemm_bf16_w16_qkv, __bf16, LTX_B_W16, LTX_EPI_QKV)
 
 // LDS-DMA W8A16 kernels (ping-pong schedule): ltx_gemm_q8_[bf16_][s32_]{store,
-// resid,qkv} for f16 (bf16_: bf16) operands with f16 (s32_: f32) scales.
-Q8_GEMM_KERNEL(ltx_gemm_q8_store, _Float16, false, LTX_EPI_STORE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_resid, _Float16, false, LTX_EPI_RESID_GATE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_qkv, _Float16, false, LTX_EPI_QKV)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store, __bf16, false, LTX_EPI_STORE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_resid, __bf16, false, LTX_EPI_RESID_GATE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_qkv, __bf16, false, LTX_EPI_QKV)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store, _Float16, true, LTX_EPI_STORE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_resid, _Float16, true, LTX_EPI_RESID_GATE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_qkv, _Float16, true, LTX_EPI_QKV)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store, __bf16, true, LTX_EPI_STORE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_resid, __bf16, true, LTX_EPI_RESID_GATE)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_qkv, __bf16, true, LTX_EPI_QKV)
+// resid,qkv} for f16 (bf16_: bf16) operands with f16 (s32_: f32) scales;
+// _store_raw for weights as packed.
+Q8_GEMM_KERNEL(ltx_gemm_q8_store, _Float16, false, LTX_EPI_STORE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_resid, _Float16, false, LTX_EPI_RESID_GATE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_qkv, _Float16, false, LTX_EPI_QKV, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store, __bf16, false, LTX_EPI_STORE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_resid, __bf16, false, LTX_EPI_RESID_GATE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_qkv, __bf16, false, LTX_EPI_QKV, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store, _Float16, true, LTX_EPI_STORE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_resid, _Float16, true, LTX_EPI_RESID_GATE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_qkv, _Float16, true, LTX_EPI_QKV, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store, __bf16, true, LTX_EPI_STORE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_resid, __bf16, true, LTX_EPI_RESID_GATE, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_qkv, __bf16, true, LTX_EPI_QKV, false)
+Q8_GEMM_KERNEL(ltx_gemm_q8_store_raw, _Float16, false, LTX_EPI_STORE, true)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store_raw, __bf16, false, LTX_EPI_STORE, true)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store_raw, _Float16, true, LTX_EPI_STORE, true)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store_raw, __bf16, true, LTX_EPI_STORE, true)
 
 // LDS-DMA W16A16 kernels (unquantised weights): ltx_gemm_w16dma_{f16,bf16}_
 // {store,resid,qkv}, 256 x 128 output tiles.

@@ -122,6 +122,7 @@ typedef struct {
     int N[LTX_DQ_JOBS], K[LTX_DQ_JOBS];
     int start[LTX_DQ_JOBS + 1];
     int njobs;
+    int raw;  // q: int8 as packed, s2: the scales as packed ([N][K / 128] f16 or f32)
 } LtxDq16Args;
 
 // Full-row qk RMSNorm (weighted, over all 4096 channels) + optional split-half

@@ -245,6 +245,29 @@ def test_linear_q8_f32_mode(ctx, M, N, K, scale_f16, gelu):
     assert oracle.rel_rms(f64(y), want) <= (1e-5 if gelu else 1e-6)
 
 
+# int8 weights as packed (aligned operands) against the pass that lays them out
+# first (weights 4 bytes past alignment), and both against the oracle: split K on
+# the small-grid and the 256 x 256 kernels, no split, and the dequantising path
+@pytest.mark.parametrize("mode,scale_f16", [("f16", True), ("bf16", False)])
+@pytest.mark.parametrize("M,N,K", [(16, 512, 1024), (129, 4096, 2048), (40, 1024, 16384), (3000, 4096, 256),
+                                   (4100, 4096, 384)])
+def test_linear_q8_packed_weights(ctx, mode, scale_f16, M, N, K):
+    say(f"linear_q8 packed weights mode={mode} scale_f16={scale_f16} M={M} N={N} K={K}")
+    m, dt = MODES[mode]
+    a, q, s, b = _gemm_case(M, N, K, seed=M + K, scale_f16=scale_f16)
+    da, ds, db = to16(a, dt).cuda(), torch.from_numpy(s).cuda(), torch.from_numpy(b).cuda()
+    buf = torch.empty(N * K + 4, dtype=torch.int8, device="cuda")
+    want = f64(da) @ oracle.dequant(q, s).astype(np.float64).T + b
+    for off in (0, 4):
+        dq = buf[off:off + N * K].view(N, K)
+        dq.copy_(torch.from_numpy(q))
+        y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+        ctx.linear_q8(da, dq, ds, db, y, mode=m)
+        torch.cuda.synchronize()
+        # as test_linear_q8: the weights' rounding to 16 bits
+        assert oracle.rel_rms(f64(y), want) <= (1e-3 if mode == "f16" else 6e-3), off
+
+
 # mode F32 where N is a multiple of 128: bf16 MFMAs on three exact planes of A
 # (one K group, an odd number of groups, ragged rows on both sides of a 128-row
 # tile, split K), or the f32 MFMA kernel

@@ -101,3 +101,15 @@ def test_noalloc_refuses_oversized_scratch(ctx):
     y = torch.empty((M, N), dtype=torch.float16, device="cuda")
     with pytest.raises(rt.LtxError, match="2 N K bytes"):
         ctx.linear_q8(a, q, s, None, y, mode=rt.MODE_F16, noalloc=True)
+
+
+@pytest.mark.parametrize("mode,M,N,K,scale_f16", [
+    (rt.MODE_F16, 16, 4096, 4096, 1), (rt.MODE_BF16, 130, 4096, 16384, 0),  # split K, on both small-row kernels
+    (rt.MODE_F32, 300, 256, 4096, 1),    # planes, split K
+    (rt.MODE_F32, 3000, 128, 4096, 0),   # planes of 3,000 rows (74 MB) exceed the array: rows in passes
+])
+def test_noalloc_split_and_planes(ctx, mode, M, N, K, scale_f16):
+    say(f"linear_q8_noalloc split / planes mode={mode} M={M} N={N} K={K}")
+    y0, y1 = _both(ctx, mode, M, N, K, 3, scale_f16, False, mode == rt.MODE_F32)
+    assert torch.isfinite(y0).all().item()
+    assert torch.equal(y0, y1)
