@@ -296,10 +296,11 @@ template <typename T, int EPI, int NI, int NJ, int OUT, bool GELU, int HOLD, typ
 __device__ __forceinline__ void gemm_epilogue_rows(const LtxGemmArgs& a, Fill fill, float* patch, int mw, int nw) {
     // The form of the test decides the four-wave kernel's register allocation:
     // with the row test alone its 16-bit store spills 57 registers instead of 16
-    // (2 % of its time at 28,672 x 4,096 x 4,096), with the hint on the QKV form
-    // that one spills 52 instead of 76. (ldo is a multiple of 8 in every launch.)
+    // (2 % of its time at 28,672 x 4,096 x 4,096) and its gated residual, though
+    // it spills fewer, takes 833 instead of 792 us there; with the hint the QKV
+    // form spills 52 instead of 76. (ldo is a multiple of 8 in every launch.)
     const bool rows = mw + 32 * NI <= a.M;
-    if ((EPI == LTX_EPI_QKV ? __builtin_expect(rows, 1) : rows) && (EPI != LTX_EPI_STORE || (a.ldo & 7) == 0))
+    if (EPI == LTX_EPI_QKV ? __builtin_expect(rows, 1) : rows && (a.ldo & 7) == 0)
         gemm_epilogue_body<T, EPI, NI, NJ, OUT, GELU, true, HOLD>(a, fill, patch, mw, nw);
     else
         gemm_epilogue_body<T, EPI, NI, NJ, OUT, GELU, false, 1>(a, fill, patch, mw, nw);
