@@ -4,8 +4,8 @@
 // The scales arrive as words: a.scales is u32 [K / 128][N], each word an f16
 // scale in both halves or an f32 scale's bits (laid out once at upload).
 //
-// Workgroup: 8 waves (two per SIMD), output tile 256 x 256; wave w owns rows
-// 128 (w / 4) .. +127 and columns 64 (w % 4) .. +63 (4 x 2 blocks of 32 x 32,
+// Workgroup: 8 waves (two per SIMD), output tile 256 x 256 (or 192 x 256, NI =
+// 3; the figures here are for 256); wave w owns rows 128 (w / 4) .. +127 and columns 64 (w % 4) .. +63 (4 x 2 blocks of 32 x 32,
 // v_mfma_f32_32x32x16_f16 or _bf16, f32 accumulate).
 //
 // K is walked in tiles of 64. Each tile's A (256 x 64 f16, 32 KB) and W
@@ -219,15 +219,16 @@ struct Q8Op<__bf16, false> : Q8Mfma<__bf16> {
 
 // RAW: the weights as packed (two's complement); their sign bits are flipped
 // after the LDS read, one XOR for four weights.
-template <typename T, bool SF32, int EPI, bool RAW>
+// NI: 32-row blocks of a wave: tiles of 256 rows (4) or 192 (3; tile_rows).
+template <typename T, bool SF32, int EPI, bool RAW, int NI>
 struct Q8Gemm {
     typedef Q8Op<T, SF32> QO;
-    static constexpr int NI = 4, NJ = 2;
+    static constexpr int NJ = 2;
     const LtxGemmArgs& a;
     f32x16 acc[NI][NJ];
     __amdgpu_buffer_rsrc_t ra_, rb_, rs_;  // A, W and scale-pair buffers
     int g, nk, ng;
-    uint32_t ga[4], gb[2];  // per-lane byte offsets of this wave's DMA sources (k-tile 0)
+    uint32_t ga[NI], gb[2];  // per-lane byte offsets of this wave's DMA sources (k-tile 0)
     int la, lb;             // this wave's DMA destinations within a stage (uniform)
     uint32_t offa[4], offb[2];
     uint32_t so;            // byte offset of the lane's first scale pair in group 0
@@ -240,7 +241,7 @@ struct Q8Gemm {
         uint8_t* da = q8_stage_a<S>() + la;
         uint8_t* db = q8_stage_b<S>() + lb;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < NI; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_, (lds_vptr)(da + 1024 * i), 16, ga[i], k * 128, 0, 0);
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -249,7 +250,7 @@ struct Q8Gemm {
 
     __device__ __forceinline__ void wait_dma(bool more2) {
         if (more2)
-            __builtin_amdgcn_s_waitcnt(Q8_WAIT_VM(6));
+            __builtin_amdgcn_s_waitcnt(Q8_WAIT_VM(NI + 2));
         else
             __builtin_amdgcn_s_waitcnt(Q8_WAIT_VM(0));
     }
@@ -347,14 +348,14 @@ struct Q8Gemm {
         rb_ = __builtin_amdgcn_make_buffer_rsrc((void*)a.b, 0, (int)((uint32_t)a.N * (uint32_t)a.K), Q8_RSRC_W3);
         rs_ = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, 0,
                                                 (int)((uint32_t)(a.K / LTX_GROUP) * (uint32_t)a.N * 4u), Q8_RSRC_W3);
-        la = 4096 * w;
+        la = 1024 * NI * w;
         lb = 2048 * w;
-        // fragment reads: A row 128 g + 32 i + lane % 32, chunks 4 h + t;
+        // fragment reads: A row 32 NI g + 32 i + lane % 32, chunks 4 h + t;
         // W row 64 q + 32 j + lane % 32, chunks 2 h + c (h = lane / 32)
         {
             const int h = lane >> 5, r = lane & 31;
 #pragma unroll
-            for (int t = 0; t < 4; t++) offa[t] = (128 * g + r) * 128 + 16 * ((4 * h + t) ^ ((r >> 1) & 7));
+            for (int t = 0; t < 4; t++) offa[t] = (32 * NI * g + r) * 128 + 16 * ((4 * h + t) ^ ((r >> 1) & 7));
 #pragma unroll
             for (int c = 0; c < 2; c++) offb[c] = (64 * q + r) * 64 + 16 * ((2 * h + c) ^ ((r >> 2) & 3));
         }
@@ -362,13 +363,13 @@ struct Q8Gemm {
         for (int item = blockIdx.x; item < ntiles; item += gridDim.x) {
             const int ks = item % ks_n;
             const TileIdx ti = tile_of(item / ks_n, a.tiles_m, a.tiles_n);
-            const int m0 = ti.tm * 256, n0 = ti.tn * 256;
+            const int m0 = ti.tm * (64 * NI), n0 = ti.tn * 256;
             const uint32_t k0 = (uint32_t)(ks * kc);  // first k of this slice
-            // DMA sources. A: instruction i of wave w fills rows 8 (4 w + i) ..
+            // DMA sources. A: instruction i of wave w fills rows 8 (NI w + i) ..
             // +7, 8 lanes a row; W: rows 16 (2 w + i) .. +15, 4 lanes a row.
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int tr = 8 * (4 * w + i) + (lane >> 3);  // row within the tile
+            for (int i = 0; i < NI; i++) {
+                const int tr = 8 * (NI * w + i) + (lane >> 3);  // row within the tile
                 const int c = (lane & 7) ^ ((tr >> 1) & 7);
                 const int row = min(m0 + tr, a.M - 1);
                 ga[i] = (uint32_t)row * (uint32_t)a.lda * 2u + 2u * k0 + 16u * c;
@@ -417,9 +418,9 @@ struct Q8Gemm {
             uint8_t* patch = w < 3 ? q8_sa0 + 9216 * w : w < 6 ? q8_sa1 + 9216 * (w - 3) : q8_sa2 + 9216 * (w - 6);
             if (ks_n > 1)  // a slice's partial sums; ltx_gemm_reduce_* applies the epilogue
                 gemm_store_partial<NI, NJ>(acc, (float*)patch, a.part + (size_t)ks * a.M * a.N, a.M, a.N,
-                                           m0 + 128 * g, n0 + 64 * q);
+                                           m0 + 32 * NI * g, n0 + 64 * q);
             else
-                gemm_epilogue_lds<T, EPI, NI, NJ>(a, acc, (float*)patch, m0 + 128 * g, n0 + 64 * q, n0);
+                gemm_epilogue_lds<T, EPI, NI, NJ>(a, acc, (float*)patch, m0 + 32 * NI * g, n0 + 64 * q, n0);
             // every patch has been read back before the next tile's DMA fills
             // the stages it lives in
             __builtin_amdgcn_sched_barrier(0);
@@ -430,8 +431,8 @@ struct Q8Gemm {
     }
 };
 
-#define Q8_GEMM_KERNEL(NAME, T_, SF32_, EPI_, RAW_)                                          \
+#define Q8_GEMM_KERNEL(NAME, T_, SF32_, EPI_, RAW_, NI_)                                     \
     extern "C" __global__ void __launch_bounds__(512, 1) NAME(const LtxGemmArgs a) {         \
-        Q8Gemm<T_, SF32_, EPI_, RAW_> k(a);                                                  \
+        Q8Gemm<T_, SF32_, EPI_, RAW_, NI_> k(a);                                             \
         k.run();                                                                             \
     }

@@ -5,9 +5,10 @@
 // ltx_gemm_dq16_* has dequantised their weights for the forward (the same
 // operand bits as the W8A16 kernel's in-register dequantisation).
 //
-// Workgroup: 4 waves, one per SIMD, output tile 256 x 256; wave w owns rows
-// 128 (w / 2) .. +127 and columns 128 (w % 2) .. +127 as 8 x 8 blocks of
-// 16 x 16 on v_mfma_f32_16x16x32_{f16,bf16}: 256 accumulator registers
+// Workgroup: 4 waves, one per SIMD, output tile 256 x 256 (NI = 8; the host may
+// take NI = 6, 192 rows, where whole rounds of 256 rows would leave CUs idle:
+// tile_rows); wave w owns rows 16 NI (w / 2) .. and columns 128
+// (w % 2) .. +127 as NI x 8 blocks of 16 x 16 on v_mfma_f32_16x16x32_{f16,bf16}: 256 accumulator registers
 // (AGPRs), every fragment read from LDS feeds 8 MFMAs (0.25 KB of LDS per
 // MFMA of 16 K flops, half the W8A16 kernel's bytes per flop), and the
 // 16 x 16 x 32 shape runs at a higher rate than 32 x 32 x 16 at the board's
@@ -71,18 +72,20 @@ __device__ __forceinline__ int x4_sofs(int x) {
 
 // SF: the STORE epilogue's form (bit 0 GELU, bit 1 f32 output), one kernel
 // each, so that a kernel holds only the epilogue it runs.
-template <typename T, int EPI, int SF = 0>
+template <typename T, int EPI, int SF = 0, int NI = 8>
 struct X4Gemm {
+    static constexpr int TM = 32 * NI;          // rows of the output tile
+    static constexpr int NR = NI + 8;           // fragment reads of a step, and DMA instructions of a K-tile
     typedef typename Op<T>::v8 V8;
     const LtxGemmArgs& a;
-    f32x4 acc[8][8];
+    f32x4 acc[NI][8];
     __amdgpu_buffer_rsrc_t ra_, rb_;
-    uint32_t ga[8];     // A: per-lane source offset of DMA instruction i (rows clamped to M - 1), k-tile 0
+    uint32_t ga[NI];    // A: per-lane source offset of DMA instruction i (rows clamped to M - 1), k-tile 0
     uint32_t gb[2];     // W: of even and odd instructions; instruction i adds (i & ~1) 8-row steps
     uint32_t wstep;     // bytes of 8 W rows
-    int lw;             // this wave's DMA destination within a stage
+    int lwa, lw;        // this wave's DMA destinations within a stage (A, W)
     uint32_t offa[2], offb[2];  // fragment reads of step s (row block i adds 2048 i)
-    u32x4 fa0[8], fb0[8], fa1[8], fb1[8];
+    u32x4 fa0[NI], fb0[8], fa1[NI], fb1[8];
 
     __device__ __forceinline__ X4Gemm(const LtxGemmArgs& args) : a(args) {}
 
@@ -91,11 +94,11 @@ struct X4Gemm {
     }
 
     template <int RS, int RSTEP>
-    __device__ __forceinline__ void read_all(u32x4 (&ya)[8], u32x4 (&yb)[8]) {
+    __device__ __forceinline__ void read_all(u32x4 (&ya)[NI], u32x4 (&yb)[8]) {
         const uint8_t* sa = x4_stage_a<RS>() + x4_vofs(offa[RSTEP]);
         const uint8_t* sb = x4_stage_b<RS>() + x4_vofs(offb[RSTEP]);
 #pragma unroll
-        for (int i = 0; i < 8; i++) ya[i] = *(const u32x4*)(sa + 2048 * i);
+        for (int i = 0; i < NI; i++) ya[i] = *(const u32x4*)(sa + 2048 * i);
 #pragma unroll
         for (int j = 0; j < 8; j++) yb[j] = *(const u32x4*)(sb + 2048 * j);
     }
@@ -103,10 +106,10 @@ struct X4Gemm {
     template <int DS>
     __device__ __forceinline__ void dma(int k) {
         const int l = x4_sofs(lw);
-        uint8_t* da = x4_stage_a<DS>() + l;
+        uint8_t* da = x4_stage_a<DS>() + (NI == 8 ? l : x4_sofs(lwa));
         uint8_t* db = x4_stage_b<DS>() + l;
 #pragma unroll
-        for (int i = 0; i < 8; i++)
+        for (int i = 0; i < NI; i++)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_, (lds_vptr)(da + 1024 * i), 16, ga[i], k * 128, 0, 0);
 #pragma unroll
         for (int i = 0; i < 8; i++)
@@ -114,33 +117,34 @@ struct X4Gemm {
                                                      k * 128 + (i & ~1) * wstep, 0, 0);
     }
 
-    __device__ __forceinline__ void mfma_all(const u32x4 (&xa)[8], const u32x4 (&xb)[8]) {
+    __device__ __forceinline__ void mfma_all(const u32x4 (&xa)[NI], const u32x4 (&xb)[8]) {
 #pragma unroll
-        for (int i = 0; i < 8; i++)
+        for (int i = 0; i < NI; i++)
 #pragma unroll
             for (int j = 0; j < 8; j++) mfma(xa[i], xb[j], acc[i][j]);
     }
 
-    // The 64 MFMAs of one step (xa, xb) with the 16 fragment reads of another
-    // (stage RS, step RSTEP, into ya, yb) and, when DMA, the 16 DMA
-    // instructions of tile kd into stage DS, one of each after every fourth
-    // MFMA; reads in the order the next step needs them (A0, W0..W7, A1..A7).
+    // The 8 NI MFMAs of one step (xa, xb) with the NR fragment reads of another
+    // (stage RS, step RSTEP, into ya, yb) and, when DMA, the NR DMA
+    // instructions of tile kd into stage DS, spread evenly, one of each after
+    // every fourth MFMA for NI = 8; reads in the order the next step needs them
+    // (A0, W0..W7, A1..).
     // Measured against one after every third MFMA: 1-3 % faster at 28,672
     // rows; every second: 10 % slower; all DMA at the region's start: 10-14 %
     // slower.
     template <int RS, int RSTEP, int DS, bool DMA>
-    __device__ __forceinline__ void region(const u32x4 (&xa)[8], const u32x4 (&xb)[8], u32x4 (&ya)[8],
+    __device__ __forceinline__ void region(const u32x4 (&xa)[NI], const u32x4 (&xb)[8], u32x4 (&ya)[NI],
                                            u32x4 (&yb)[8], int kd) {
         const uint8_t* sa = x4_stage_a<RS>() + x4_vofs(offa[RSTEP]);
         const uint8_t* sb = x4_stage_b<RS>() + x4_vofs(offb[RSTEP]);
         const int l = DMA ? x4_sofs(lw) : 0;
-        uint8_t* da = x4_stage_a<DS>() + l;
+        uint8_t* da = x4_stage_a<DS>() + (NI == 8 || !DMA ? l : x4_sofs(lwa));
         uint8_t* db = x4_stage_b<DS>() + l;
 #pragma unroll
-        for (int m = 0; m < 64; m++) {
+        for (int m = 0; m < 8 * NI; m++) {
             mfma(xa[m >> 3], xb[m & 7], acc[m >> 3][m & 7]);
-            if (m % 4 == 3) {
-                const int g = m / 4;
+            const int g = ((m + 1) * NR - 1) / (8 * NI);  // slot g follows MFMA (g + 1) 8 NI / NR, rounded up
+            if (((m + 2) * NR - 1) / (8 * NI) > g) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (g == 0)
                     ya[0] = *(const u32x4*)sa;
@@ -149,12 +153,13 @@ struct X4Gemm {
                 else
                     ya[g - 8] = *(const u32x4*)(sa + 2048 * (g - 8));
                 if (DMA) {
-                    if (g < 8)
+                    if (g < NI)
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_, (lds_vptr)(da + 1024 * g), 16, ga[g], kd * 128,
                                                                  0, 0);
                     else
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb_, (lds_vptr)(db + 1024 * (g - 8)), 16, gb[g & 1],
-                                                                 kd * 128 + ((g - 8) & ~1) * wstep, 0, 0);
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rb_, (lds_vptr)(db + 1024 * (g - NI)), 16,
+                                                                 gb[(g - NI) & 1], kd * 128 + ((g - NI) & ~1) * wstep,
+                                                                 0, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -183,11 +188,12 @@ struct X4Gemm {
     __device__ __forceinline__ void run() {
         const int tid = threadIdx.x, lane = tid & 63;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const int wm = 128 * (w >> 1), wn = 128 * (w & 1);
+        const int wm = 16 * NI * (w >> 1), wn = 128 * (w & 1);
         const int nk = a.K / 64;  // even: K is a multiple of 128
         ra_ = __builtin_amdgcn_make_buffer_rsrc((void*)a.a, 0, (int)((uint32_t)a.M * (uint32_t)a.lda * 2u), Q8_RSRC_W3);
         rb_ = __builtin_amdgcn_make_buffer_rsrc((void*)a.b, 0, (int)((uint32_t)a.N * (uint32_t)a.K * 2u), Q8_RSRC_W3);
         lw = 8192 * w;
+        lwa = 1024 * NI * w;
         wstep = 16u * (uint32_t)a.K;
         {
             const int h = lane >> 4, r = lane & 15;
@@ -201,12 +207,12 @@ struct X4Gemm {
         const int ntiles = a.tiles_m * a.tiles_n;
         for (int item = blockIdx.x; item < ntiles; item += gridDim.x) {
             const TileIdx ti = tile_of(item, a.tiles_m, a.tiles_n);
-            const int m0 = ti.tm * 256, n0 = ti.tn * 256;
-            // DMA instruction i of wave w fills tile rows 8 (8 w + i) .. +7,
-            // 8 lanes a row; the row's swizzle (row / 2) & 7 is (4 i + lane / 16) & 7
+            const int m0 = ti.tm * TM, n0 = ti.tn * 256;
+            // DMA instruction i of wave w fills A rows 8 (NI w + i) .. +7 and W
+            // rows 8 (8 w + i) .. +7, 8 lanes a row
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int tr = 8 * (8 * w + i) + (lane >> 3);
+            for (int i = 0; i < NI; i++) {
+                const int tr = 8 * (NI * w + i) + (lane >> 3);
                 const int c = (lane & 7) ^ ((tr >> 1) & 7);
                 ga[i] = (uint32_t)min(m0 + tr, a.M - 1) * (uint32_t)a.lda * 2u + 16u * c;
             }
@@ -217,7 +223,7 @@ struct X4Gemm {
                 gb[i] = (uint32_t)(n0 + tr) * (uint32_t)a.K * 2u + 16u * c;
             }
 #pragma unroll
-            for (int i = 0; i < 8; i++)
+            for (int i = 0; i < NI; i++)
 #pragma unroll
                 for (int j = 0; j < 8; j++) acc[i][j] = f32x4{0, 0, 0, 0};
             dma<0>(0);
@@ -246,7 +252,7 @@ struct X4Gemm {
                         for (int r = 0; r < 4; r++)
                             p[(16 * e + 4 * (el >> 4) + r) * LD + 16 * j + (el & 15)] = acc[2 * b + e][j][r];
             };
-            gemm_epilogue_patch<T, EPI, 4, 4, decltype(fill), EPI == LTX_EPI_STORE ? SF : -1, 4>(
+            gemm_epilogue_patch<T, EPI, NI / 2, 4, decltype(fill), EPI == LTX_EPI_STORE ? SF : -1, NI / 2>(
                 a, fill, (float*)patch, m0 + wm, n0 + wn, n0);
             // every patch has been read back before the next tile's DMA
             meet();
@@ -254,9 +260,9 @@ struct X4Gemm {
     }
 };
 
-#define X4_GEMM_KERNEL(NAME, T_, EPI_, SF_)                                          \
+#define X4_GEMM_KERNEL(NAME, T_, EPI_, SF_, NI_)                                     \
     extern "C" __global__ void __launch_bounds__(256, 1) NAME(const LtxGemmArgs a) { \
-        X4Gemm<T_, EPI_, SF_> k(a);                                                  \
+        X4Gemm<T_, EPI_, SF_, NI_> k(a);                                             \
         k.run();                                                                     \
     }
 

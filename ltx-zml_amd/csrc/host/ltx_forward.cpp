@@ -51,14 +51,31 @@ static int gemm_ksplit(int num_cu, int M, int N, int K, int tn = 256, int tm = 2
     return s;
 }
 
-bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda) {
+// Rows of a persistent GEMM's 256-column tiles, 256 or 192: the height whose
+// whole rounds of one tile a CU are the fewest rows, a row of the lower tiles
+// counted 1.05 times (they read more LDS and move more operand bytes per MFMA).
+// Measured, 192 against 256 rows, us (rows x N x K, the dequantisation
+// included): 4,100 x 4,096 x 4,096 147 : 182, 2,970 x 12,288 x 4,096 271 : 303,
+// 1,600 x 12,288 x 4,096 164 : 192, 4,100 x 4,096 x 16,384 588 : 685; where the
+// rule stays at 256: 4,095 x 4,096 x 4,096 150 : 120, 8,000 x 4,096 x 4,096 229
+// : 211, 2,048 x 16,384 x 4,096 254 : 231. Tiles of 128 rows lost everywhere.
+static int tile_rows(const ltx_ctx* c, int M, int N) {
+    if (c->gemm_rows == 192 || c->gemm_rows == 256) return c->gemm_rows;
+    auto rounds = [&](int rows) { return (((M + rows - 1) / rows) * (N / 256) + c->num_cu - 1) / c->num_cu; };
+    return rounds(192) * 192 * 1.05f < rounds(256) * 256 ? 192 : 256;
+}
+
+bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool w16) {
     if (mode != LTX_MODE_F16 && mode != LTX_MODE_BF16) return false;
     if (!c->gemm_x4 || !c->gemm_dma) return false;
     if (M <= 0 || N % 256 || K % 128 || lda < K || lda % 8) return false;
     if ((uint64_t)M * lda * 2 >= (1ull << 31) || (uint64_t)N * K * 2 >= (1ull << 31)) return false;
     if (c->gemm_x4 == 2) return true;
-    // where its 256 x 256 tiles fill the CUs: the sizes that need no split-K
-    return M >= 4096 && gemm_ksplit(c->num_cu, M, N, K) == 1;
+    // where its 256 x 256 tiles fill the CUs: the sizes that need no split-K.
+    // 16-bit weights (no dequantisation): as soon as the 256 x 128 tiles of the
+    // other kernel need a second round for 4,096 columns (o1 and o2 at 2,970
+    // rows 84 against 120 us)
+    return M >= (w16 ? 2049 : 4096) && gemm_ksplit(c->num_cu, M, N, K) == 1;
 }
 
 bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8) {
@@ -258,13 +275,16 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
     // epilogue move 16-byte vectors)
     {
         const void* wb = p.q8 ? w16 : (mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p);
-        if (wb && x4_shape(c, mode, M, p.N, p.K, lda) && g.ldo % 8 == 0 && al16(A) && al16(wb) && al16(g.out) &&
+        if (wb && x4_shape(c, mode, M, p.N, p.K, lda, !p.q8) && g.ldo % 8 == 0 && al16(A) && al16(wb) && al16(g.out) &&
             al16(g.out2) && al16(g.resid) && al16(g.bias) && al16(g.ada.tstab) && al16(g.ada.sst)) {
             g.b = wb;
             g.scales = nullptr;
             g.ksplit = 1;
             std::snprintf(name, sizeof(name), "ltx_gemm_x4_%s_%s%s%s", msuffix(mode), es,
                           epi == LTX_EPI_STORE && g.out_f32 ? "32" : "", epi == LTX_EPI_STORE && g.gelu ? "_gelu" : "");
+            const int tr = tile_rows(c, M, p.N);
+            if (tr != 256) std::snprintf(name + std::strlen(name), sizeof(name) - std::strlen(name), "_h%d", tr);
+            g.tiles_m = (M + tr - 1) / tr;
             const int nitems = g.tiles_m * g.tiles_n;
             c->launch(name, c->gemm_persistent ? std::min(nitems, c->num_cu) : nitems, 1, 1, 256, &g, st, label);
             return;
@@ -305,6 +325,9 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
         // few output tiles: split K over more workgroups (when the caller
         // gave a buffer for the partial sums), then reduce + epilogue
         g.ksplit = g.part ? gemm_ksplit(c->num_cu, M, p.N, p.K) : 1;
+        const int tr = g.ksplit > 1 ? 256 : tile_rows(c, M, p.N);
+        if (tr != 256) std::snprintf(name + std::strlen(name), sizeof(name) - std::strlen(name), "_h%d", tr);
+        g.tiles_m = (M + tr - 1) / tr;
         const int nitems = g.tiles_m * g.tiles_n * g.ksplit;
         c->launch(name, c->gemm_persistent ? std::min(nitems, c->num_cu) : nitems, 1, 1, 512, &g, st, label);
         if (g.ksplit > 1) {

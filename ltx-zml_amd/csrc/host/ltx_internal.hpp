@@ -118,6 +118,9 @@ struct ltx_ctx {
     // mode F32's GEMM on bf16 MFMAs (three exact planes of A) where the shape
     // allows, or the f32 MFMA kernel everywhere (false: tests)
     bool gemm_f3 = true;
+    // rows of the 256-column GEMM tiles: 0 by the rule of tile_rows, or 192 or
+    // 256 everywhere (tests)
+    int gemm_rows = 0;
     int num_cu = 256;             // compute units: the persistent GEMM's grid bound
     bool gemm_persistent = true;  // LDS-DMA GEMM: at most one workgroup per CU, looping over tiles
     bool attn_pp = true;
@@ -202,8 +205,9 @@ struct LinearScratch {
     void* w16 = nullptr;  // N * K 16-bit weights for the four-wave GEMM, or NULL (the W8A16 kernel)
 };
 // Whether the four-wave 16-bit GEMM takes an M x N x K product with A rows of
-// lda elements (shape, 32-bit buffer offsets and the context's setting).
-bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda);
+// lda elements (shape, 32-bit buffer offsets and the context's setting; w16:
+// weights that are 16-bit already).
+bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool w16 = false);
 // Whether the small-grid GEMM takes it (q8: int8 weights, else 16-bit).
 bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8);
 // The f32 GEMM on bf16 MFMAs: whether it takes an M x N x K product, and the

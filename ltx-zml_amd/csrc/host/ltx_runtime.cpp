@@ -10,7 +10,7 @@
 // gfx950 code objects, embedded at build time (ltx_codeobjects.S).
 extern "C" {
 extern const unsigned char ltx_co_k_gemm[], ltx_co_k_gemm_s4[], ltx_co_k_gemm_f3[],
-    ltx_co_k_attn[], ltx_co_k_norm[], ltx_co_k_f32[],
+    ltx_co_k_gemm_x4h[], ltx_co_k_gemm_q8h[], ltx_co_k_attn[], ltx_co_k_norm[], ltx_co_k_f32[],
     ltx_co_k_core[];
 }
 
@@ -208,6 +208,7 @@ int ltx_init(int device, ltx_ctx** out) {
             c->gemm_x4 = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
         if (const char* e = std::getenv("LTX_GEMM_S4"))
             c->gemm_s4 = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
+        if (const char* e = std::getenv("LTX_GEMM_ROWS")) c->gemm_rows = std::atoi(e);
         if (const char* e = std::getenv("LTX_GEMM_F3")) c->gemm_f3 = std::strcmp(e, "off") != 0;
         if (const char* e = std::getenv("LTX_SIDE_EARLY"))
             c->side_early = std::strcmp(e, "off") == 0 ? 0 : std::strcmp(e, "all") == 0 ? 2 : 1;
@@ -219,8 +220,8 @@ int ltx_init(int device, ltx_ctx** out) {
         for (auto& e : c->side_ev) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         for (auto& e : c->marks) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence));
         for (const unsigned char* co :
-             {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_gemm_f3, ltx_co_k_attn, ltx_co_k_norm, ltx_co_k_f32,
-              ltx_co_k_core}) {
+             {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_gemm_f3, ltx_co_k_gemm_x4h, ltx_co_k_gemm_q8h, ltx_co_k_attn,
+              ltx_co_k_norm, ltx_co_k_f32, ltx_co_k_core}) {
             hipModule_t m;
             HIPC(hipModuleLoadData(&m, co));
             c->modules.push_back(m);

@@ -196,22 +196,22 @@ GEMM_KERNEL(ltx_gemm_bf16_w16_qkv, __bf16, LTX_B_W16, LTX_EPI_QKV)
 // LDS-DMA W8A16 kernels (ping-pong schedule): ltx_gemm_q8_[bf16_][s32_]{store,
 // resid,qkv} for f16 (bf16_: bf16) operands with f16 (s32_: f32) scales;
 // _store_raw for weights as packed.
-Q8_GEMM_KERNEL(ltx_gemm_q8_store, _Float16, false, LTX_EPI_STORE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_resid, _Float16, false, LTX_EPI_RESID_GATE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_qkv, _Float16, false, LTX_EPI_QKV, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store, __bf16, false, LTX_EPI_STORE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_resid, __bf16, false, LTX_EPI_RESID_GATE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_qkv, __bf16, false, LTX_EPI_QKV, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store, _Float16, true, LTX_EPI_STORE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_resid, _Float16, true, LTX_EPI_RESID_GATE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_qkv, _Float16, true, LTX_EPI_QKV, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store, __bf16, true, LTX_EPI_STORE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_resid, __bf16, true, LTX_EPI_RESID_GATE, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_qkv, __bf16, true, LTX_EPI_QKV, false)
-Q8_GEMM_KERNEL(ltx_gemm_q8_store_raw, _Float16, false, LTX_EPI_STORE, true)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store_raw, __bf16, false, LTX_EPI_STORE, true)
-Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store_raw, _Float16, true, LTX_EPI_STORE, true)
-Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store_raw, __bf16, true, LTX_EPI_STORE, true)
+Q8_GEMM_KERNEL(ltx_gemm_q8_store, _Float16, false, LTX_EPI_STORE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_resid, _Float16, false, LTX_EPI_RESID_GATE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_qkv, _Float16, false, LTX_EPI_QKV, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store, __bf16, false, LTX_EPI_STORE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_resid, __bf16, false, LTX_EPI_RESID_GATE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_qkv, __bf16, false, LTX_EPI_QKV, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store, _Float16, true, LTX_EPI_STORE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_resid, _Float16, true, LTX_EPI_RESID_GATE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_qkv, _Float16, true, LTX_EPI_QKV, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store, __bf16, true, LTX_EPI_STORE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_resid, __bf16, true, LTX_EPI_RESID_GATE, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_qkv, __bf16, true, LTX_EPI_QKV, false, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_store_raw, _Float16, false, LTX_EPI_STORE, true, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_store_raw, __bf16, false, LTX_EPI_STORE, true, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_s32_store_raw, _Float16, true, LTX_EPI_STORE, true, 4)
+Q8_GEMM_KERNEL(ltx_gemm_q8_bf16_s32_store_raw, __bf16, true, LTX_EPI_STORE, true, 4)
 
 // LDS-DMA W16A16 kernels (unquantised weights): ltx_gemm_w16dma_{f16,bf16}_
 // {store,resid,qkv}, 256 x 128 output tiles.
@@ -227,18 +227,18 @@ W16_GEMM_KERNEL(ltx_gemm_w16dma_bf16_qkv, __bf16, LTX_EPI_QKV)
 // (store32: f32 output), and the per-forward dequantisation of the int8
 // weights they take: ltx_gemm_dq16_{f16,bf16} (fp16 scale pairs), _s32 (f32
 // scales).
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_store, _Float16, LTX_EPI_STORE, 0)
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_store_gelu, _Float16, LTX_EPI_STORE, 1)
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_store32, _Float16, LTX_EPI_STORE, 2)
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_store32_gelu, _Float16, LTX_EPI_STORE, 3)
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_resid, _Float16, LTX_EPI_RESID_GATE, 0)
-X4_GEMM_KERNEL(ltx_gemm_x4_f16_qkv, _Float16, LTX_EPI_QKV, 0)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store, __bf16, LTX_EPI_STORE, 0)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store_gelu, __bf16, LTX_EPI_STORE, 1)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store32, __bf16, LTX_EPI_STORE, 2)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store32_gelu, __bf16, LTX_EPI_STORE, 3)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_resid, __bf16, LTX_EPI_RESID_GATE, 0)
-X4_GEMM_KERNEL(ltx_gemm_x4_bf16_qkv, __bf16, LTX_EPI_QKV, 0)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_store, _Float16, LTX_EPI_STORE, 0, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_store_gelu, _Float16, LTX_EPI_STORE, 1, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_store32, _Float16, LTX_EPI_STORE, 2, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_store32_gelu, _Float16, LTX_EPI_STORE, 3, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_resid, _Float16, LTX_EPI_RESID_GATE, 0, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_f16_qkv, _Float16, LTX_EPI_QKV, 0, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store, __bf16, LTX_EPI_STORE, 0, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store_gelu, __bf16, LTX_EPI_STORE, 1, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store32, __bf16, LTX_EPI_STORE, 2, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_store32_gelu, __bf16, LTX_EPI_STORE, 3, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_resid, __bf16, LTX_EPI_RESID_GATE, 0, 8)
+X4_GEMM_KERNEL(ltx_gemm_x4_bf16_qkv, __bf16, LTX_EPI_QKV, 0, 8)
 extern "C" __global__ void __launch_bounds__(256) ltx_gemm_dq16_f16(const LtxDq16Args a) { dq16_body<_Float16, false>(a); }
 extern "C" __global__ void __launch_bounds__(256) ltx_gemm_dq16_f16_s32(const LtxDq16Args a) {
     dq16_body<_Float16, true>(a);

@@ -268,6 +268,44 @@ def test_linear_q8_packed_weights(ctx, mode, scale_f16, M, N, K):
         assert oracle.rel_rms(f64(y), want) <= (1e-3 if mode == "f16" else 6e-3), off
 
 
+# tiles of 192 rows against 256: the same products in the same order for every
+# output, so the same bits, except that GELU's last product may be rounded to 16
+# bits at once in whole wave tiles and through f32 in ragged ones (or the other
+# way round), one unit apart where those differ; rows on both sides of one and of
+# several tiles
+@pytest.mark.parametrize("kernel", [("LTX_GEMM_X4", "all"), ("LTX_GEMM_S4", "off")])
+@pytest.mark.parametrize("mode,scale_f16,gelu,out_f32", [("f16", True, True, False), ("bf16", False, False, True),
+                                                         ("f16", False, True, True), ("bf16", True, False, False)])
+def test_linear_q8_tile_rows(monkeypatch, kernel, mode, scale_f16, gelu, out_f32):
+    say(f"linear_q8 tile rows {kernel} {mode} scale_f16={scale_f16} gelu={gelu} out_f32={out_f32}")
+    m, dt = MODES[mode]
+    monkeypatch.setenv(*kernel)
+    ctxs = []
+    try:
+        for rows in ("192", "256"):
+            monkeypatch.setenv("LTX_GEMM_ROWS", rows)
+            ctxs.append(rt.Context(0))
+        for M, N, K in ((1, 256, 256), (191, 512, 384), (193, 256, 4096), (577, 768, 256), (5000, 4096, 128)):
+            a, q, s, b = _gemm_case(M, N, K, seed=M, scale_f16=scale_f16)
+            da, dq, ds, db = (to16(a, dt).cuda(), torch.from_numpy(q).cuda(), torch.from_numpy(s).cuda(),
+                              torch.from_numpy(b).cuda())
+            ys = []
+            for c in ctxs:
+                y = torch.full((M, N), float("nan"), dtype=torch.float32 if out_f32 else dt, device="cuda")
+                c.linear_q8(da, dq, ds, db, y, mode=m, gelu=gelu)
+                ys.append(y)
+            torch.cuda.synchronize()
+            assert torch.isfinite(ys[0]).all()
+            if gelu and not out_f32:
+                d = (ys[0].view(torch.int16).int() - ys[1].view(torch.int16).int()).abs()
+                assert d.max() <= 1 and (d > 0).float().mean() < 0.01, (M, N, K)
+            else:
+                assert torch.equal(*ys), (M, N, K)
+    finally:
+        for c in ctxs:
+            c.close()
+
+
 # mode F32 where N is a multiple of 128: bf16 MFMAs on three exact planes of A
 # (one K group, an odd number of groups, ragged rows on both sides of a 128-row
 # tile, split K), or the f32 MFMA kernel

@@ -303,3 +303,32 @@ def test_int8_recipe_error_budgets(ctx, dist):
     held = [k for k in r if not (dist == "t3" and k == "attention")]
     assert all(r[k] <= budget[k] for k in held), r
     assert r["ffn"] > 1e-3  # the int8 block is not the unquantised one: the probe measures something
+
+
+@pytest.mark.parametrize("x4,T,S,weights", [("all", 250, 40, "int8"), ("all", 200, 64, "bf16"),
+                                            # the W8A16 kernel without split K, the ragged last tile of every projection
+                                            ("off", 2200, 77, "int8")])
+@pytest.mark.parametrize("mode", ["f16", "bf16"])
+def test_block_tile_rows(monkeypatch, block0, block0_w16, mode, x4, T, S, weights):
+    """GEMM tiles of 192 rows against 256 (every epilogue: QKV split with V^T
+    and its padding, gated residual, GELU): the same bits up to the FFN's hidden
+    values, of which a few are one 16-bit unit apart (their last rounding, see
+    test_linear_q8_tile_rows): half a unit of the type bounds y's difference."""
+    say(f"block tile rows mode={mode} x4={x4} T={T} S={S} weights={weights}")
+    monkeypatch.setenv("LTX_GEMM_X4", x4)
+    inp = synth.make_inputs(T, S, sigma=0.7)
+    cos, sin = rt.rope_tables(inp["grid"])
+    ys, xs = [], []
+    for rows in ("192", "256"):
+        monkeypatch.setenv("LTX_GEMM_ROWS", rows)
+        c = rt.Context(0)
+        try:
+            w = c.upload(block0 if weights == "int8" else block0_w16)
+            ys.append(forward(c, w, inp, cos, sin, mode))
+            xs.append([stage(c, n, torch.float32, (T, D)) for n in ("x_sa", "x_ca")])
+            w.free()
+        finally:
+            c.close()
+    assert np.isfinite(ys[0]).all()
+    assert oracle.rel_rms(*ys) <= (2.0 ** -11 if mode == "f16" else 2.0 ** -8)
+    assert all(np.array_equal(*x) for x in zip(*xs))
