@@ -400,13 +400,7 @@ static void dequant16(ltx_ctx* c, int mode, const LtxProj* const* p, void* const
 
 static void gate16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M, float* out, hipStream_t st) {
     LtxGateArgs g{A, mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p, (const float*)p.bias.p, out, M};
-    // one wave per 32 rows while that gives every CU at least one wave
-    // (each wave's 256 MFMAs form one dependent chain); below that, K split
-    // over the four waves of a workgroup per 32 rows
-    if ((M + 31) / 32 >= c->num_cu)
-        c->launch(mode == LTX_MODE_BF16 ? "ltx_gate_bf16" : "ltx_gate_f16", (M + 127) / 128, 1, 1, 256, &g, st);
-    else
-        c->launch(mode == LTX_MODE_BF16 ? "ltx_gate_ks_bf16" : "ltx_gate_ks_f16", (M + 31) / 32, 1, 1, 256, &g, st);
+    c->launch(mode == LTX_MODE_BF16 ? "ltx_gate_bf16" : "ltx_gate_f16", (M + 15) / 16, 1, 1, 512, &g, st);
 }
 
 // Whether ltx_op_attention pads V^T (lkv no multiple of 64) for the LDS-DMA
@@ -689,9 +683,6 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         const LtxProj* ps[6] = {&w->qkv1, &w->o1, &w->q2, &w->o2, &w->f1, &w->f2};
         dequant16(c, mode, ps, b.dq, 6, dq, st);
     }
-    // self-attention: n = modulate(rms(x), ada1, ada0); fused q|k|v GEMM
-    norm_mod(c, mode, x, b.n_msa, ada, T, 0, 1, st,
-             mode == LTX_MODE_F16 ? (const unsigned long long*)w->f16_over.p : nullptr);
     hipStream_t sd = c->side;
     auto fail_check = [&]() {
         if (fail_in_capture()) {
@@ -714,23 +705,45 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         gk.part = (float*)part;
         gemm16(c, mode, w->kv2, b.enc, S, LTX_D, LTX_EPI_QKV, gk, s, "gemm:kv2");
     };
-    // Small T (early): the 256-row GEMM tiles and attention query tiles
-    // leave CUs idle, and the side stream fills them from here on: the
-    // self-attention gate logits beside the q|k|v GEMM, then the whole
-    // context side (K/V modulation, k|v GEMM with its own partial sums, k
-    // norm) beside the self-attention branch; later the cross-attention
-    // gate logits beside the q2 GEMM. Large T: side work starts only after
-    // the persistent GEMMs, whose one-workgroup-per-CU grids it would
-    // otherwise hold back, and ends before the attentions, which it would
-    // slow as much as it gains.
+    // Small T (early): the side stream fills the CUs that the main chain leaves
+    // idle. Where the last round of the q|k|v GEMM's tiles leaves an eighth of
+    // them, it starts after the first norm: the gate logits beside that GEMM,
+    // then the context side (K/V modulation, k|v GEMM with its own partial sums,
+    // k norm), and later the cross-attention's gate logits beside the q2 GEMM
+    // (1,024 tokens: 653 us; with the gate logits on the main stream 667, with
+    // the context side from the start 669). Where that GEMM fills the chip, side
+    // work beside it would wait for its end and then slow the q and k norms: the
+    // context side starts with the forward, beside the first norm, and the gate
+    // logits run on the main stream (2,970 tokens: 1,613 against 1,645 us).
+    // Large T: side work starts only after the persistent GEMMs, whose
+    // one-workgroup-per-CU grids it would otherwise hold back, and ends before
+    // the attentions, which it would slow as much as it gains.
     const bool early = side_early(c, (size_t)T);
+    bool side_gates = !early;
+    auto early_ctx = [&]() {
+        ctx_side(sd, b.part2);
+        qknorm16(c, mode, b.k2_16, LTX_D, w->kn2.p, nullptr, nullptr, b.kh2, S, 1.0f, sd);
+    };
     if (early) {
+        const int tr = tile_rows(c, T, 3 * LTX_D), last = (T + tr - 1) / tr * (3 * LTX_D / 256) % c->num_cu;
+        side_gates = last > 0 && last <= c->num_cu - c->num_cu / 8;
+        if (!side_gates) {
+            stream_after(sd, st, c->side_ev[0]);
+            fail_check();
+            early_ctx();
+        }
+    }
+    // self-attention: n = modulate(rms(x), ada1, ada0); fused q|k|v GEMM
+    norm_mod(c, mode, x, b.n_msa, ada, T, 0, 1, st,
+             mode == LTX_MODE_F16 ? (const unsigned long long*)w->f16_over.p : nullptr);
+    if (early && side_gates) {
         stream_after(sd, st, c->side_ev[0]);
         fail_check();
         gate16(c, mode, w->g1, b.n_msa, T, (float*)b.glog1, sd);
         HIPC(hipEventRecord(c->side_ev[1], sd));  // glog1 ready
-        ctx_side(sd, b.part2);
-        qknorm16(c, mode, b.k2_16, LTX_D, w->kn2.p, nullptr, nullptr, b.kh2, S, 1.0f, sd);
+        early_ctx();
+    } else if (early) {
+        gate16(c, mode, w->g1, b.n_msa, T, (float*)b.glog1, st);
     }
     LtxGemmArgs g{};
     g.out = b.qk16;
@@ -753,7 +766,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
                           T, 2 * LTX_D, kAttnC, 1.0f, sat};
         c->launch(mode == LTX_MODE_BF16 ? "ltx_qknorm2_bf16" : "ltx_qknorm2_f16", T, 1, 1, 256, &qa, st);
     }
-    HIPC(hipStreamWaitEvent(st, c->side_ev[1], 0));
+    if (side_gates) HIPC(hipStreamWaitEvent(st, c->side_ev[1], 0));
     attn16(c, mode, b.qh1, b.kh1, b.vt1, vt_ld(T), (const float*)b.glog1, b.o1, T, T, true, st, "attn:self", sat, true);
     g = LtxGemmArgs{};
     g.out = b.x_sa;
@@ -766,8 +779,8 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     // cross-attention
     norm_mod(c, mode, (const float*)b.x_sa, b.attn_in, ada, T, 6, 7, st);
     if (early) {
-        stream_after(sd, st, c->side_ev[2]);
-        gate16(c, mode, w->g2, b.attn_in, T, (float*)b.glog2, sd);
+        if (side_gates) stream_after(sd, st, c->side_ev[2]);
+        gate16(c, mode, w->g2, b.attn_in, T, (float*)b.glog2, side_gates ? sd : st);
     }
     g = LtxGemmArgs{};
     g.out = b.q2_16;
@@ -792,7 +805,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
             qknorm16(c, mode, b.q2_16, LTX_D, w->qn2.p, nullptr, nullptr, b.qh2, T, kAttnC, st);
             qknorm16(c, mode, b.k2_16, LTX_D, w->kn2.p, nullptr, nullptr, b.kh2, S, 1.0f, st);
         }
-        stream_after(st, sd, c->side_ev[3]);  // glog2 (and, early, the context side) ready
+        stream_after(st, sd, c->side_ev[3]);  // glog2, or (early) the context side, ready
         attn16(c, mode, b.qh2, b.kh2, b.vt2, vt_ld(S), (const float*)b.glog2, b.o2, T, S, true, st, "attn:cross", sat, true);
     }
     g = LtxGemmArgs{};

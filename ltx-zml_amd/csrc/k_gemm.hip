@@ -249,71 +249,41 @@ extern "C" __global__ void __launch_bounds__(256) ltx_gemm_dq16_bf16_s32(const L
 }
 
 // Gate logits (ltx/block.zig:238, 526, 564): glog[t][h] = a[t] . gw[h] + gb[h].
-// One wave per 32 token rows: 256 MFMAs over K = 4096, operands straight
-// from global memory (the 32 x 4096 weight stays L2-resident).
+// Bound by reading a. A workgroup of 8 waves takes 16 rows, each wave 512 of
+// the 4,096 channels (its 48 operand loads straight from global memory, all in
+// flight before its 32 MFMAs: the 32 x 4,096 weight stays in L2), and the
+// waves' sums meet in LDS.
 template <typename T>
 __device__ void gate_body(const LtxGateArgs& a) {
     typedef typename Op<T>::v8 v8;
-    const int lane = threadIdx.x & 63;
-    const int m0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 32;
-    if (m0 >= a.M) return;
-    const int fr = lane & 31, fk = 8 * (lane >> 5);
-    const uint16_t* pa = (const uint16_t*)a.a + (size_t)min(m0 + fr, a.M - 1) * LTX_D + fk;
-    const uint16_t* pb = (const uint16_t*)a.gw + (size_t)fr * LTX_D + fk;
-    f32x16 acc = f32x16{0};
-#pragma unroll 8
-    for (int k = 0; k < LTX_D; k += 16) {
-        v8 fa = __builtin_bit_cast(v8, *(const u32x4*)(pa + k));
-        v8 fb = __builtin_bit_cast(v8, *(const u32x4*)(pb + k));
-        acc = Op<T>::mfma32(fa, fb, acc);
-    }
-    const float bias = a.gb[fr];
+    __shared__ float part[8][16][LTX_H + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lr = lane & 15, lg = lane >> 4;
+    const int m0 = blockIdx.x * 16, c0 = 512 * w + 8 * lg;
+    const uint16_t* pa = (const uint16_t*)a.a + (size_t)min(m0 + lr, a.M - 1) * LTX_D + c0;
+    const uint16_t* pb = (const uint16_t*)a.gw + (size_t)lr * LTX_D + c0;
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        int m = m0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < a.M) a.out[(size_t)m * LTX_H + fr] = acc[r] + bias;
+    for (int ks = 0; ks < 16; ks++) {
+        const v8 fa = __builtin_bit_cast(v8, *(const u32x4*)(pa + 32 * ks));
+#pragma unroll
+        for (int nb = 0; nb < 2; nb++)
+            acc[nb] = Op<T>::mfma16(fa, __builtin_bit_cast(v8, *(const u32x4*)(pb + 16 * nb * LTX_D + 32 * ks)), acc[nb]);
     }
-}
-
-extern "C" __global__ void __launch_bounds__(256) ltx_gate_f16(const LtxGateArgs a) { gate_body<_Float16>(a); }
-extern "C" __global__ void __launch_bounds__(256) ltx_gate_bf16(const LtxGateArgs a) { gate_body<__bf16>(a); }
-
-// The same logits for few rows: one workgroup per 32 rows, wave q sums
-// k in [1024 q, 1024 q + 1024) over two alternating accumulators (two
-// independent MFMA chains), and wave 0 adds the four partial sums in wave
-// order through LDS.
-template <typename T>
-__device__ void gate_ks_body(const LtxGateArgs& a) {
-    typedef typename Op<T>::v8 v8;
-    __shared__ f32x16 red[3][64];
-    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    const int m0 = blockIdx.x * 32;
-    const int fr = lane & 31, fk = 8 * (lane >> 5) + q * (LTX_D / 4);
-    const uint16_t* pa = (const uint16_t*)a.a + (size_t)min(m0 + fr, a.M - 1) * LTX_D + fk;
-    const uint16_t* pb = (const uint16_t*)a.gw + (size_t)fr * LTX_D + fk;
-    f32x16 acc0 = f32x16{0}, acc1 = f32x16{0};
-#pragma unroll 8
-    for (int k = 0; k < LTX_D / 4; k += 32) {
-        acc0 = Op<T>::mfma32(__builtin_bit_cast(v8, *(const u32x4*)(pa + k)),
-                             __builtin_bit_cast(v8, *(const u32x4*)(pb + k)), acc0);
-        acc1 = Op<T>::mfma32(__builtin_bit_cast(v8, *(const u32x4*)(pa + k + 16)),
-                             __builtin_bit_cast(v8, *(const u32x4*)(pb + k + 16)), acc1);
-    }
-    const f32x16 acc = acc0 + acc1;
-    if (q > 0) red[q - 1][lane] = acc;
+#pragma unroll
+    for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) part[w][4 * lg + i][16 * nb + lr] = acc[nb][i];
     __syncthreads();
-    if (q > 0) return;
-    const f32x16 sum = ((acc + red[0][lane]) + red[1][lane]) + red[2][lane];
-    const float bias = a.gb[fr];
+    const int row = tid >> 5, h = tid & 31;
+    float o = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        int m = m0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        if (m < a.M) a.out[(size_t)m * LTX_H + fr] = sum[r] + bias;
-    }
+    for (int i = 0; i < 8; i++) o += part[i][row][h];
+    if (m0 + row < a.M) a.out[(size_t)(m0 + row) * LTX_H + h] = o + a.gb[h];
 }
 
-extern "C" __global__ void __launch_bounds__(256) ltx_gate_ks_f16(const LtxGateArgs a) { gate_ks_body<_Float16>(a); }
-extern "C" __global__ void __launch_bounds__(256) ltx_gate_ks_bf16(const LtxGateArgs a) { gate_ks_body<__bf16>(a); }
+extern "C" __global__ void __launch_bounds__(512) ltx_gate_f16(const LtxGateArgs a) { gate_body<_Float16>(a); }
+extern "C" __global__ void __launch_bounds__(512) ltx_gate_bf16(const LtxGateArgs a) { gate_body<__bf16>(a); }
 
 // Split-K completion: v = sum over s = 0 .. S-1 of part[s][m][n] (in that
 // order) + bias[n], then the GEMM's epilogue. A workgroup of 256 threads owns
