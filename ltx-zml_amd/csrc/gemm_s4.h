@@ -91,10 +91,14 @@ __device__ __forceinline__ void gemm_store_partial_patch(Fill fill, float* patch
     }
 }
 
-// RAW: the int8 weights as packed (two's complement); their sign bits are
-// flipped after the LDS read, one XOR for four weights, where a pass over the
-// weights that flips them first would read and write each once more.
-template <typename T, int BK, int EPI, bool RAW>
+// RAW 1: the int8 weights as packed. Their sign bits are flipped after the LDS
+// read, one XOR for four weights, where a pass over the weights that flips them
+// first would read and write each once more.
+// RAW 2: the scales as packed too. The scale DMA gathers from [N][K / 128]: f32
+// scales word by word; f16 scales (K / 128 even) as the aligned pair of groups
+// that holds the tile's, the half taken where the word is used. This saves a
+// launch that lays them out, and costs a 64-line gather a K-tile and wave.
+template <typename T, int BK, int EPI, int RAW>
 struct S4Gemm {
     static constexpr bool Q = BK != LTX_B_W16;
     static constexpr bool SF32 = BK == LTX_B_I8_F32S;
@@ -111,6 +115,7 @@ struct S4Gemm {
     uint32_t so;            // byte offset of scale word n0 + wn + lane, first group of the slice
     uint32_t lsc;           // LDS offset of the lane's scale word (column block 0) within a W stage
     int la, lb, ls;         // this wave's DMA destinations within a stage (A, W, int8 scale words)
+    int g0 = 0;             // first group of the slice (RAW 2)
     uint32_t offa[2], offb[2];  // fragment reads of step s (block i adds 2048 i; int8 W 1024 i)
     // fragments of one 32-k step (A, W as read, W's scale words): step 0 of
     // the next tile and step 1 of the current one
@@ -128,7 +133,10 @@ struct S4Gemm {
         constexpr int Q1 = Q ? 1 : 0;
         if (Q && d == 0)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_, (lds_vptr)(s4_stage_b<Q, S>() + ls), 4, so,
-                                                     (kt >> 1) * a.N * 4, 0, 0);
+                                                     RAW < 2 ? (kt >> 1) * a.N * 4
+                                                     : SF32 ? (g0 + (kt >> 1)) * 4
+                                                            : (g0 + (kt >> 1)) / 2 * 4,
+                                                     0, 0);
         else if (d < Q1 + 4)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_, (lds_vptr)(s4_stage_a<Q, S>() + la + 1024 * (d - Q1)), 16,
                                                      ga[d - Q1], kt * 128, 0, 0);
@@ -162,12 +170,16 @@ struct S4Gemm {
         for (int r = 0; r < 8; r++) read1<S, STEP>(r, ya, yw, ysc);
     }
 
-    // the W fragments as MFMA operands (int8: dequantised with their scales)
-    __device__ __forceinline__ void operands(const WF (&w)[4], const uint32_t (&sc)[4], V8 (&xb)[4]) {
+    // the W fragments of K-tile kt as MFMA operands (int8: dequantised with
+    // their scales)
+    __device__ __forceinline__ void operands(const WF (&w)[4], const uint32_t (&sc)[4], V8 (&xb)[4], int kt) {
+        // packed f16 scales: the half of the pair, into both halves
+        const uint32_t sel = (g0 + (kt >> 1)) & 1 ? 0x03020302u : 0x01000100u;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             if constexpr (Q)
-                xb[j] = QO::deq8(w[j][0] ^ kX, w[j][1] ^ kX, QO::scale(sc[j]));
+                xb[j] = QO::deq8(w[j][0] ^ kX, w[j][1] ^ kX,
+                                 QO::scale(RAW == 2 && !SF32 ? __builtin_amdgcn_perm(sc[j], sc[j], sel) : sc[j]));
             else
                 xb[j] = __builtin_bit_cast(V8, w[j]);
         }
@@ -222,7 +234,7 @@ struct S4Gemm {
     __device__ __forceinline__ void pair(int k, int nk) {
         constexpr int R = (S + 1) % 3;
         V8 xb[4];
-        operands(fw1, sc1, xb);
+        operands(fw1, sc1, xb, k);
         region<R, 0, S, true>(fa1, xb, fa0, fw0, sc0, min(k + 3, nk - 1));
         __builtin_amdgcn_sched_barrier(0);
         // step 0's scale words and W fragments landed (its A fragments, read
@@ -230,7 +242,7 @@ struct S4Gemm {
         __builtin_amdgcn_s_waitcnt(Q8_WAIT_LGKM(4));
         // nothing that reads the scale words may move above that wait
         __builtin_amdgcn_sched_barrier(0);
-        operands(fw0, sc0, xb);
+        operands(fw0, sc0, xb, k + 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) sc1[j] = sc0[j];
         region<R, 1, S, false>(fa0, xb, fa1, fw1, sc1, 0);
@@ -251,7 +263,8 @@ struct S4Gemm {
                                                 Q8_RSRC_W3);
         if constexpr (Q)
             rs_ = __builtin_amdgcn_make_buffer_rsrc((void*)a.scales, 0,
-                                                    (int)((uint32_t)(a.K / LTX_GROUP) * (uint32_t)a.N * 4u), Q8_RSRC_W3);
+                                                    (int)((uint32_t)(a.K / LTX_GROUP) * (uint32_t)a.N * (RAW == 2 && !SF32 ? 2u : 4u)),
+                                                    Q8_RSRC_W3);
         // wave w's DMA fills A rows 32 w .. 32 w + 31 (4 KB), int8 W rows
         // 32 w .. + 31 (2 KB), 16-bit W rows 32 w .. + 31 (4 KB); int8 scale
         // words of columns wn .. wn + 63 at 8192 + 256 w
@@ -295,7 +308,9 @@ struct S4Gemm {
                 const int nr = lane >> 2, nc = (lane & 3) ^ ((lane >> 4) & 3);
 #pragma unroll
                 for (int i = 0; i < 2; i++) gb[i] = (uint32_t)(n0 + 16 * (2 * w + i) + nr) * (uint32_t)a.K + k0 + 16u * nc;
-                so = 4u * ((k0 / LTX_GROUP) * (uint32_t)a.N + (uint32_t)(n0 + wn + lane));
+                g0 = (int)(k0 / LTX_GROUP);
+                so = RAW == 2 ? (uint32_t)(n0 + wn + lane) * (uint32_t)(a.K / LTX_GROUP) * (SF32 ? 4u : 2u)
+                         : 4u * ((uint32_t)g0 * (uint32_t)a.N + (uint32_t)(n0 + wn + lane));
             }
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -316,7 +331,7 @@ struct S4Gemm {
                 // step 0's scale words and W fragments landed (12 reads after them)
                 __builtin_amdgcn_s_waitcnt(Q8_WAIT_LGKM(12));
                 __builtin_amdgcn_sched_barrier(0);
-                operands(fw0, sc0, xb);
+                operands(fw0, sc0, xb, 0);
 #pragma unroll
                 for (int m = 0; m < 16; m++) mfma1(m, fa0, xb);
             }
@@ -334,7 +349,7 @@ struct S4Gemm {
             if (k + 2 < nk) pair<1>(k + 1, nk);
             {
                 V8 xb[4];
-                operands(fw1, sc1, xb);
+                operands(fw1, sc1, xb, nk - 1);
 #pragma unroll
                 for (int m = 0; m < 16; m++) mfma1(m, fa1, xb);
             }

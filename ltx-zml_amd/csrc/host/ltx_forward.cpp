@@ -109,6 +109,13 @@ size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K) {
     return s > 1 ? (size_t)s * M * N * 4 : 0;
 }
 
+// Whether the small-grid kernel gathers the isolated GEMM's scales as packed
+// instead of from the words that a launch of 5 us lays out: the gathers cost more
+// with more row tiles on the chip. Measured, packed against words, us (rows x N,
+// K = 4,096): 16 x 4,096 17.8 : 21.4, 128 x 4,096 24.2 : 27.4, 256 x 8,192 34.5 :
+// 36.3; 512 x 8,192 50.2 : 44.7, 1,024 x 4,096 49.4 : 45.2.
+static bool s4_packed_scales(int M) { return M <= 256; }
+
 // The small-T schedule of the block forward (side stream from the first
 // RMSNorm + modulate on).
 static bool side_early(const ltx_ctx* c, size_t T) {
@@ -294,16 +301,17 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
     // out for the LDS-DMA kernels (bytes q + 128, scale words) or 16-bit
     // weights; split K only while even those tiles fill at most half the CUs
     {
-        const void* wb = p.q8 ? ((p.qflip || p.qraw) && p.s2.p ? p.q.p : nullptr) : (mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p);
+        const void* wb = p.q8 ? ((p.qraw && s4_packed_scales(M)) || ((p.qflip || p.qraw) && p.s2.p) ? p.q.p : nullptr) : (mode == LTX_MODE_BF16 ? p.w_bf16.p : p.w_f16.p);
         if (wb && s4_shape(c, mode, M, p.N, p.K, lda, p.q8) && g.ldo % 8 == 0 && al16(A) && al16(wb) && al16(g.out) &&
             al16(g.out2) && al16(g.resid) && al16(g.bias) && al16(g.ada.tstab) && al16(g.ada.sst)) {
             g.b = wb;
-            g.scales = p.q8 ? p.s2.p : nullptr;
+            const bool sp = p.qraw && s4_packed_scales(M);
+            g.scales = !p.q8 ? nullptr : sp ? p.s.p : p.s2.p;
             g.tiles_m = (M + 127) / 128;
             g.tiles_n = p.N / 128;
             g.ksplit = g.part ? gemm_ksplit(c->num_cu, M, p.N, p.K, 128, 128) : 1;
             std::snprintf(name, sizeof(name), "ltx_gemm_s4_%s_%s_%s%s", msuffix(mode),
-                          p.q8 ? (p.scale_f16 ? "i8f16" : "i8f32") : "w16", es, p.qraw ? "_raw" : "");
+                          p.q8 ? (p.scale_f16 ? "i8f16" : "i8f32") : "w16", es, sp ? "_packed" : p.qraw ? "_raw" : "");
             const int nitems = g.tiles_m * g.tiles_n * g.ksplit;
             c->launch(name, c->gemm_persistent ? std::min(nitems, 2 * c->num_cu) : nitems, 1, 1, 256, &g, st, label);
             if (g.ksplit > 1) {
@@ -861,17 +869,24 @@ bool linear_aligned(const void* a, const void* q, const void* bias, const void* 
     return (((uintptr_t)a | (uintptr_t)q | (uintptr_t)bias | (uintptr_t)y) & 15) == 0;
 }
 
+bool linear_packed(const void* a, const void* q, const void* scales, int scale_f16, const void* bias, const void* y,
+                   int K) {
+    return linear_aligned(a, q, bias, y) && ((uintptr_t)scales & 3) == 0 && !(scale_f16 && (K / LTX_GROUP) % 2);
+}
+
 size_t linear_part_bytes(const ltx_ctx* c, int M, int N, int K, int mode) {
     if (!linear_q8_needs_scratch(c, N, K, mode) || x4_shape(c, mode, M, N, K, K)) return 0;
     const int t = s4_shape(c, mode, M, N, K, K, true) ? 128 : 256, s = gemm_ksplit(c->num_cu, M, N, K, t, t);
     return s > 1 ? (size_t)s * M * N * 4 : 0;
 }
 
-// ltx_op_linear_q8 / _noalloc: in the 16-bit modes with the LDS-DMA kernels the
-// scales are first laid out as words [K/128][N] in sc.pairs, and weights (or
-// other operands) that are not 16-byte aligned as bytes q + 128 in sc.q, which
-// at 16,384 x 4,096 weights took 28 us of a call (all written whole before the
-// GEMM reads them). The four-wave kernel's dequantisation reads both as packed.
+// ltx_op_linear_q8 / _noalloc: in the 16-bit modes the kernels take the weights as
+// packed (linear_packed), the four-wave kernel's dequantisation and the small-grid
+// kernel up to 256 rows also the scales; else the scales are first laid out as
+// words [K/128][N] in sc.pairs.
+// Operands that are not linear_packed: the scale words, and the weights as bytes
+// q + 128 in sc.q, which at 16,384 x 4,096 weights takes 28 us of a call (all
+// written whole before the GEMM reads them).
 void check_linear_q8(int M, int N, int K, int mode) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 128) throw Error("bad GEMM shape (K must be a multiple of 128)");
     if (mode != LTX_MODE_F16 && mode != LTX_MODE_BF16 && mode != LTX_MODE_F32) throw Error("unknown mode");
@@ -910,11 +925,10 @@ void linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, i
             const bool scratch = linear_q8_needs_scratch(c, N, K, mode);
             const bool x4 = scratch && sc.w16 && x4_shape(c, mode, M, N, K, K);
             if (scratch) {
-                // aligned operands: the kernels take the weights as packed
-                p.qraw = linear_aligned(a, q, bias, y);
+                p.qraw = linear_packed(a, q, scales, scale_f16, bias, y, K);
                 if (!sc.pairs || (!p.qraw && !sc.q)) throw Error("linear_q8: no scratch");
-                if (!p.qraw || !x4) {
-                    // the LDS-DMA kernel reads scale words [K/128][N]
+                if (!p.qraw || !(x4 || (s4_shape(c, mode, M, N, K, K, true) && s4_packed_scales(M)))) {
+                    // the 256 x 256 LDS-DMA kernel reads scale words [K/128][N]
                     const size_t n2 = (size_t)N * (K / LTX_GROUP);
                     LtxPairArgs pa{scales, sc.pairs, N, K / LTX_GROUP, scale_f16 ? 0 : 1};
                     c->launch("ltx_scale_pairs", (unsigned)((n2 + 255) / 256), 1, 1, 256, &pa, st);
@@ -1083,12 +1097,13 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
             }
         }
         // 16-bit modes: split-K partial sums (not captured: then no split)
-        if (const size_t np = ltx::linear_aligned(a, q, bias, y) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0)
+        const bool packed = ltx::linear_packed(a, q, scales, scale_f16, bias, y, K);
+        if (const size_t np = packed ? ltx::linear_part_bytes(c, M, N, K, mode) : 0)
             used = (sc.part = c->op_scratch.take(np, st)) != nullptr;
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
             // scratch owned by the context, grown as needed
             const size_t nq = (size_t)N * K, np = (size_t)N * (K / LTX_GROUP) * 4;
-            if (!ltx::linear_aligned(a, q, bias, y) && c->op_q.bytes < nq) c->op_q.alloc(nq);
+            if (!packed && c->op_q.bytes < nq) c->op_q.alloc(nq);
             if (c->op_pairs.bytes < np) c->op_pairs.alloc(np);
             sc.q = (uint32_t*)c->op_q.p;
             sc.pairs = (uint32_t*)c->op_pairs.p;

@@ -215,9 +215,13 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
 bool f3_shape(const ltx_ctx* c, int M, int N, int K);
 size_t f3_planes_bytes(int M, int K);
 size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K);
-// Bytes of split-K partial sums of the isolated int8 GEMM in the 16-bit modes
-// (0: no split, or operands that are not 16-byte aligned).
+// The isolated int8 GEMM: 16-byte aligned operands; in the 16-bit modes also
+// whether the kernels take the weights and scales as packed (f16 scales: an even
+// number of groups); and the bytes of its split-K partial sums, used with the
+// latter (0: no split).
 bool linear_aligned(const void* a, const void* q, const void* bias, const void* y);
+bool linear_packed(const void* a, const void* q, const void* scales, int scale_f16, const void* bias, const void* y,
+                   int K);
 size_t linear_part_bytes(const ltx_ctx* c, int M, int N, int K, int mode);
 // Shape and mode checks of the isolated int8 GEMM (throws Error), made before
 // any scratch is sized from N and K.

@@ -89,9 +89,9 @@ extern "C" int ltx_op_linear_q8_noalloc(ltx_ctx* c, const void* a, const int8_t*
             sc.plane_rows = rows;
             sc.part = part ? base + np : nullptr;
         }
-        if (const size_t part = ltx::linear_aligned(a, q, bias, y) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0) {
+        if (const size_t part = ltx::linear_packed(a, q, scales, scale_f16, bias, y, K) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0) {
             // beside the scale words; the room of the bytes q + 128 is free
-            // (aligned operands). At most 64 MiB: 256 tiles x slices of 256 KB
+            // (packed operands). At most 64 MiB: 256 tiles x slices of 256 KB
             const size_t np = ((size_t)N * (K / LTX_GROUP) * 4 + 255) & ~(size_t)255;
             if (np + part > LTX_NOALLOC_SCRATCH_BYTES)
                 throw ltx::Error("ltx_op_linear_q8_noalloc: scratch too small for the partial sums");  // (cannot happen)

@@ -247,10 +247,11 @@ def test_linear_q8_f32_mode(ctx, M, N, K, scale_f16, gelu):
 
 # int8 weights as packed (aligned operands) against the pass that lays them out
 # first (weights 4 bytes past alignment), and both against the oracle: split K on
-# the small-grid and the 256 x 256 kernels, no split, and the dequantising path
+# the small-grid and the 256 x 256 kernels, no split, the dequantising path, and
+# odd numbers of scale groups (three; five in a split of ten)
 @pytest.mark.parametrize("mode,scale_f16", [("f16", True), ("bf16", False)])
 @pytest.mark.parametrize("M,N,K", [(16, 512, 1024), (129, 4096, 2048), (40, 1024, 16384), (3000, 4096, 256),
-                                   (4100, 4096, 384)])
+                                   (4100, 4096, 384), (200, 512, 384), (70, 256, 1280)])
 def test_linear_q8_packed_weights(ctx, mode, scale_f16, M, N, K):
     say(f"linear_q8 packed weights mode={mode} scale_f16={scale_f16} M={M} N={N} K={K}")
     m, dt = MODES[mode]
