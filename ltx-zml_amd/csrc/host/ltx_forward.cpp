@@ -89,8 +89,11 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
     // split-K reduce (the context k|v projection, the 4096-wide projections
     // below 4,096 rows). With 16-bit weights, or K = 16,384, its 128 x 128
     // tiles (half the flops per byte moved) measured slower than the split
-    // 256 x 256 kernels; with no split (q|k|v at 1,024 rows) slower too.
-    return q8 && M < 4096 && K <= 4096 && gemm_ksplit(c->num_cu, M, N, K) > 1;
+    // 256 x 256 kernels; with no split (q|k|v at 1,024 rows) slower too. Up to
+    // 256 rows it takes K = 16,384 as well, half or all of whose 256-row tiles
+    // would be padding: 16 x 4,096 x 16,384 34 against 57 us, 128 rows 37 : 58,
+    // 256 rows 55 : 58; 400 rows 90 : 82.
+    return q8 && M < 4096 && (K <= 4096 || M <= 256) && gemm_ksplit(c->num_cu, M, N, K) > 1;
 }
 
 // Whether the f32 GEMM on bf16 MFMAs takes an M x N x K product (shape and
@@ -426,6 +429,14 @@ static bool pad_pays(const ltx_ctx* c, int lq, int lkv) {
     return nt >= (lkv % 8 == 0 ? 28 : 5);
 }
 
+// Whether the streaming attention takes 128-query workgroups: where they fit the
+// chip in one round (up to 1,024 queries), so that 256-query ones would leave half
+// of it idle. A workgroup of 128 takes three quarters of the other's time (the
+// same K and V^T fragments for half the MFMAs). Measured, 128 against 256, us:
+// 256 x 1,024 18 : 26, 512 x 512 12 : 17, 1,024 x 1,024 23 : 28, 1,024 x 128
+// 8.1 : 9.7.
+static bool attn_q128(const ltx_ctx* c, int lq) { return (lq + 127) / 128 * LTX_H <= c->num_cu; }
+
 // The attention's exponent scale: softmax scale 1/sqrt(128) times log2(e).
 static const float kAttnC = (float)(1.4426950408889634 / 11.313708498984761);
 
@@ -475,7 +486,12 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
     }
     if (c->attn_pp && whole && nt >= 2) {
         // ping-pong kernel: at least two 64-key tiles
-        std::snprintf(name, sizeof(name), "ltx_attn_%s_pp%s", msuffix(mode), q_scaled ? "" : "_uq");
+        const char* v = "pp";
+        if (attn_q128(c, lq)) {
+            a.q_tiles = (lq + 127) / 128;
+            v = "pp1";
+        }
+        std::snprintf(name, sizeof(name), "ltx_attn_%s_%s%s", msuffix(mode), v, q_scaled ? "" : "_uq");
         c->launch(name, a.q_tiles * LTX_H, 1, 1, 512, &a, st, label);
         return;
     }

@@ -353,7 +353,9 @@ __device__ __forceinline__ uint8_t* app_v() {
 
 // PS: Q arrives multiplied by the exponent scale C = log2(e)/sqrt(128) (the
 // block's qk-norm kernel writes it so), so a score is already in exp2 units.
-template <typename T, bool PS>
+// NQ: 16-query column blocks per wave, 2 (256 queries a workgroup) or, for query
+// counts whose 256-query tiles leave CUs idle, 1 (128; streaming form).
+template <typename T, bool PS, int NQ = 2>
 struct AttnPP {
     typedef typename Op<T>::v8 v8;
     const LtxAttnArgs& a;
@@ -363,12 +365,12 @@ struct AttnPP {
     int lw;                 // this wave's 2 KB slice of a stage
     uint32_t ok[4];         // K fragment offsets per 32-dim step ks (kb adds 4096)
     uint32_t ov[2];         // V^T fragment offsets per 32-key step kc (db adds 2048)
-    v8 qf[2][4];            // Q^T operand [qb][ks]
-    f32x4 o[8][2];          // O^T [db][qb]
-    f32x4 s[4][2];          // S^T [kb][qb]
-    v8 pf[2][2];            // P^T operand [kc][qb]
+    v8 qf[NQ][4];           // Q^T operand [qb][ks]
+    f32x4 o[8][NQ];         // O^T [db][qb]
+    f32x4 s[4][NQ];         // S^T [kb][qb]
+    v8 pf[2][NQ];           // P^T operand [kc][qb]
     v8 vpre[4];             // V^T fragments kc = 0, db = 0..3 of the next PV, read in the softmax phase (resident form)
-    f32x4 sb[2];            // -m of the lane's query in block qb: the S MFMAs start from it
+    f32x4 sb[NQ];           // -m of the lane's query in block qb: the S MFMAs start from it
     f32x2 m, l;             // running max and partial sum per query block (vectors, not arrays: kept in registers)
     float C;
     int nt, g;
@@ -416,14 +418,14 @@ struct AttnPP {
                                       ? vpre[db & 3]
                                       : __builtin_bit_cast(v8, *(const u32x4*)(sv + ov[kc] + 2048 * db));
                     o[db][0] = Op<T>::mfma16(vf, pf[kc][0], o[db][0]);
-                    o[db][1] = Op<T>::mfma16(vf, pf[kc][1], o[db][1]);
+                    if (NQ > 1) o[db][NQ - 1] = Op<T>::mfma16(vf, pf[kc][NQ - 1], o[db][NQ - 1]);
                 }
         }
         if (ds) {
 #pragma unroll
             for (int kb = 0; kb < 4; kb++) {
                 s[kb][0] = sb[0];
-                s[kb][1] = sb[1];
+                s[kb][NQ - 1] = sb[NQ - 1];
             }
 #pragma unroll
             for (int ks = 0; ks < 4; ks++)
@@ -431,7 +433,7 @@ struct AttnPP {
                 for (int kb = 0; kb < 4; kb++) {
                     const v8 kf = __builtin_bit_cast(v8, *(const u32x4*)(sk + ok[ks] + 4096 * kb));
                     s[kb][0] = Op<T>::mfma16(kf, qf[0][ks], s[kb][0]);
-                    s[kb][1] = Op<T>::mfma16(kf, qf[1][ks], s[kb][1]);
+                    if (NQ > 1) s[kb][NQ - 1] = Op<T>::mfma16(kf, qf[NQ - 1][ks], s[kb][NQ - 1]);
                 }
         }
         // fragment reads eight MFMAs (four reads) ahead (masks: 0x100 DS
@@ -439,7 +441,7 @@ struct AttnPP {
         if (!PRE) __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
         for (int i = 0; i < 32; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, NQ, 0);
             if (i < 28) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
     }
@@ -461,7 +463,7 @@ struct AttnPP {
 #pragma unroll
         for (int kc = 0; kc < 2; kc++)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) {
+            for (int qb = 0; qb < NQ; qb++) {
                 float p[8];
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
@@ -499,13 +501,13 @@ struct AttnPP {
             for (int kb = 0; kb < 4; kb++)
 #pragma unroll
                 for (int r = 0; r < 4; r++)
-                    if (32 * (kb >> 1) + 4 * (kb & 1) + r >= left) s[kb][0][r] = s[kb][1][r] = -__builtin_inff();
+                    if (32 * (kb >> 1) + 4 * (kb & 1) + r >= left) s[kb][0][r] = s[kb][NQ - 1][r] = -__builtin_inff();
         }
         f32x2 ps = exps<false>(f32x2{0.f, 0.f});
-        if (first || __builtin_amdgcn_ballot_w64(!(ps[0] <= 256.0f) || !(ps[1] <= 256.0f)) != 0) {
-            f32x2 delta;
+        if (first || __builtin_amdgcn_ballot_w64(!(ps[0] <= 256.0f) || !(ps[NQ - 1] <= 256.0f)) != 0) {
+            f32x2 delta = {0.f, 0.f};
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) {
+            for (int qb = 0; qb < NQ; qb++) {
                 float mx = s[0][qb][0];
 #pragma unroll
                 for (int kb = 0; kb < 4; kb++)
@@ -610,11 +612,11 @@ struct AttnPP {
 
     // Q^T operands of the wave's queries q0 .. q0 + 31 of head h (rows past
     // lq read row lq - 1)
-    __device__ __forceinline__ void load_q(v8 (&dst)[2][4], int h, int q0, int lane) const {
+    __device__ __forceinline__ void load_q(v8 (&dst)[NQ][4], int h, int q0, int lane) const {
         const uint16_t* Q = (const uint16_t*)a.q + (size_t)h * a.q_hs;
         const int j = lane >> 4, r = lane & 15;
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < NQ; qb++) {
             const int q = min(q0 + 16 * qb + r, a.lq - 1);
 #pragma unroll
             for (int ks = 0; ks < 4; ks++)
@@ -624,9 +626,9 @@ struct AttnPP {
 
     __device__ __forceinline__ void reset() {
 #pragma unroll
-        for (int db = 0; db < 8; db++) o[db][0] = o[db][1] = f32x4{0};
+        for (int db = 0; db < 8; db++) o[db][0] = o[db][NQ - 1] = f32x4{0};
         m = f32x2{0.f, 0.f};
-        sb[0] = sb[1] = f32x4{0};
+        sb[0] = sb[NQ - 1] = f32x4{0};
         l = f32x2{0.f, 0.f};
     }
 
@@ -635,7 +637,7 @@ struct AttnPP {
     __device__ __forceinline__ void load_glog(float (&gl)[2], int h, int q0, int lane) const {
         if (a.glog)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++)
+            for (int qb = 0; qb < NQ; qb++)
                 gl[qb] = a.glog[(size_t)min(q0 + 16 * qb + (lane & 15), a.lq - 1) * LTX_H + h];
     }
 
@@ -647,10 +649,10 @@ struct AttnPP {
                                               unsigned& bad) const {
         constexpr int LD = DPP + 8, LPR = DPP / 8, RPI = 64 / LPR;  // lanes per row, rows per instruction
         const int j = lane >> 4, r = lane & 15;
-        float sc[2];
-        bool qok[2];
+        float sc[NQ];
+        bool qok[NQ];
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < NQ; qb++) {
             float lt = l[qb] + __shfl_xor(l[qb], 16, 64);
             lt += __shfl_xor(lt, 32, 64);
             qok[qb] = q0 + 16 * qb + r < a.lq;
@@ -664,7 +666,7 @@ struct AttnPP {
             for (int dbh = 0; dbh < DPP / 16; dbh++) {
                 const int db = (DPP / 16) * part + dbh;
 #pragma unroll
-                for (int qb = 0; qb < 2; qb++) {
+                for (int qb = 0; qb < NQ; qb++) {
                     const f32x4 v = o[db][qb] * sc[qb];
                     *(u32x2*)(patch + (16 * qb + r) * LD + 16 * dbh + 4 * j) =
                         u32x2{Op<T>::cvt2(v[0], v[1]), Op<T>::cvt2(v[2], v[3])};
@@ -674,7 +676,7 @@ struct AttnPP {
                 }
             }
 #pragma unroll
-            for (int it = 0; it < 32 / RPI; it++) {
+            for (int it = 0; it < 16 * NQ / RPI; it++) {
                 const int row = RPI * it + lane / LPR, c = lane % LPR;  // LPR lanes x 16 B per row
                 const u32x4 v = *(const u32x4*)(patch + row * LD + 8 * c);
                 const int q = q0 + row;
@@ -691,7 +693,7 @@ struct AttnPP {
         int t = blockIdx.x;
         if ((nblk & 7) == 0) t = (t & 7) * (nblk >> 3) + (t >> 3);
         const int h = t / a.q_tiles, qt = t - h * a.q_tiles;
-        const int q0 = qt * 256 + w * 32;
+        const int q0 = (qt * 8 + w) * 16 * NQ;
         setup(h, w, lane);
         load_q(qf, h, q0, lane);
         reset();
@@ -735,9 +737,9 @@ struct AttnPP {
 #pragma unroll
         for (int kc = 0; kc < 2; kc++)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) asm volatile("" ::"v"(__builtin_bit_cast(u32x4, pf[kc][qb])));
+            for (int qb = 0; qb < NQ; qb++) asm volatile("" ::"v"(__builtin_bit_cast(u32x4, pf[kc][qb])));
         asm volatile("" ::"v"(l), "v"(m));
-        asm volatile("" ::"v"(sb[0]), "v"(sb[1]));
+        asm volatile("" ::"v"(sb[0]), "v"(sb[NQ - 1]));
     }
 
     // as pin_softmax, and the prefetched V^T fragments of the next PV
@@ -749,11 +751,11 @@ struct AttnPP {
 
     // after the last softmax of a query tile: the next MFMA phase starts the
     // next tile (S(0) from a zero max, with its Q)
-    __device__ __forceinline__ void next_tile(const v8 (&qn)[2][4]) {
+    __device__ __forceinline__ void next_tile(const v8 (&qn)[NQ][4]) {
         m = f32x2{0.f, 0.f};
-        sb[0] = sb[1] = f32x4{0};
+        sb[0] = sb[NQ - 1] = f32x4{0};
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++)
+        for (int qb = 0; qb < NQ; qb++)
 #pragma unroll
             for (int ks = 0; ks < 4; ks++) qf[qb][ks] = qn[qb][ks];
     }
@@ -779,6 +781,7 @@ struct AttnPP {
     // Every query tile takes 2 nt barriers in both groups (group 1 keeps its
     // one-phase lag), plus one after the final PV.
     __device__ __forceinline__ void run_resident(uint8_t* kres, uint8_t* vres, uint16_t* patches) {
+        static_assert(NQ == 2, "256-query tiles");
         const int tid = threadIdx.x, lane = tid & 63;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
         g = w >> 2;
@@ -812,7 +815,7 @@ struct AttnPP {
         if (g == 1) __builtin_amdgcn_s_barrier();
         uint16_t* patch = patches + 1280 * w;  // [32 q][40]: 32 dims per pass
         unsigned bad = 0;  // 16-bit outputs out of range (range guard)
-        v8 qn[2][4];       // the next tile's Q^T operands
+        v8 qn[NQ][4];      // the next tile's Q^T operands
         for (int qt = qt0; qt < a.q_tiles; qt += wph) {
             const bool prev = qt > qt0;
             // t = 0: PV of the previous tile's last key tile, S(0); then the
@@ -875,6 +878,24 @@ extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_f16_pp_uq(const Lt
 }
 extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_bf16_pp_uq(const LtxAttnArgs a) {
     AttnPP<__bf16, false> k(a);
+    k.run();
+}
+
+// _pp1[_uq]: 128 queries a workgroup
+extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_f16_pp1(const LtxAttnArgs a) {
+    AttnPP<_Float16, true, 1> k(a);
+    k.run();
+}
+extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_bf16_pp1(const LtxAttnArgs a) {
+    AttnPP<__bf16, true, 1> k(a);
+    k.run();
+}
+extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_f16_pp1_uq(const LtxAttnArgs a) {
+    AttnPP<_Float16, false, 1> k(a);
+    k.run();
+}
+extern "C" __global__ void __launch_bounds__(512, 1) ltx_attn_bf16_pp1_uq(const LtxAttnArgs a) {
+    AttnPP<__bf16, false, 1> k(a);
     k.run();
 }
 

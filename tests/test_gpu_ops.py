@@ -451,6 +451,13 @@ def test_attention_ragged_keys(ctx, mode, q_scaled, lq, lkv):
     assert oracle.rel_rms(f64(out), want) <= (2e-3 if mode == "f16" else 1e-2)
 
 
+@pytest.mark.parametrize("lq,lkv", [(16, 128), (127, 192), (129, 320), (1024, 200), (1025, 320)])
+def test_attention_query_tiles(ctx, lq, lkv):
+    """128-query workgroups (up to 1,024 queries) at the edges of a tile and of
+    a wave, and the first query count on 256-query ones."""
+    test_attention(ctx, "f16", lq, lkv, True, True)
+
+
 def test_attention_ragged_keys_captured(ctx):
     """Under capture no scratch is taken (the any-length kernel runs); eager
     calls between the replays take the padded path."""
