@@ -202,11 +202,16 @@ int ltx_range_count(ltx_ctx* ctx, void* stream, uint64_t* count, int reset);
  * scales [N][K/128] f32 or f16 (f32: finite, magnitude below 2^100, not
  * checked here); y f32 (out_f32) or 16-bit. Mirrors linQ
  * (ltx/block.zig:473-477). In the 16-bit modes with N a multiple of 256 the
- * call first lays the weights out as bytes q + 128 and the scales as words
- * [K/128][N] in scratch the context owns (allocated on first use, grown as
- * needed) and then runs the GEMM, all on `stream`: two calls of one context on
- * different streams may overwrite each other's scratch, so keep one context's
- * calls on one stream. A shape with M, N or K not positive or K not a
+ * GEMM uses scratch the context owns (allocated on first use, grown as needed):
+ * scale words, weights dequantised to the operand type or split-K partial sums,
+ * and for operands that are not 16-byte aligned (scales 4-byte; f16 scales: K an
+ * odd multiple of 128) the weights as bytes q + 128. Two calls of one context on
+ * different streams may overwrite that scratch, so keep one context's calls on
+ * one stream. Mode F32 with N a multiple of 128 splits a into three bf16 planes
+ * in context scratch; calls on different streams are ordered behind each other's
+ * use of it. A call being captured takes no scratch for planes or partial sums:
+ * it runs the kernels that need none (the same products summed in another
+ * order). A shape with M, N or K not positive or K not a
  * multiple of 128, or an unknown mode, is refused (status 0, ltx_last_error)
  * before any scratch is sized or allocated. */
 int ltx_op_linear_q8(ltx_ctx* ctx, const void* a, const int8_t* q, const void* scales, int scale_f16,
@@ -216,10 +221,12 @@ int ltx_op_linear_q8(ltx_ctx* ctx, const void* a, const int8_t* q, const void* s
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): ltx_op_linear_q8 with the same arguments and results,
- * calling no hipMalloc / hipFree. Its scratch (the weights as bytes q + 128,
- * N * K bytes rounded up to 256, then the scale words, 4 N K / 128 bytes,
- * and for the shapes ltx_op_linear_q8 runs on the four-wave GEMM, from 4,096
- * rows, the weights dequantised to the operand type, 2 N K bytes) is
+ * calling no hipMalloc / hipFree. Its scratch (room for the weights as bytes
+ * q + 128, N * K bytes rounded up to 256, then the scale words, 4 N K / 128
+ * bytes, and for the shapes ltx_op_linear_q8 runs on the four-wave GEMM, from
+ * 4,096 rows, the weights dequantised to the operand type, 2 N K bytes; split-K
+ * partial sums take the place of the bytes q + 128, and mode F32 runs the planes
+ * of as many rows at a time as fit) is
  * a static device array of LTX_NOALLOC_SCRATCH_BYTES on each GPU the library
  * runs on, held until the process ends; a shape needing more is refused with
  * an error. The kernels write all of the scratch they read on each call, so
@@ -234,6 +241,10 @@ int ltx_op_linear_q8_noalloc(ltx_ctx* ctx, const void* a, const int8_t* q, const
 /* Attention with per-(token, head) gate (gate logits glog [Lq][32] f32, or
  * NULL for no gate). F16/BF16: q, k [32][L][128] 16-bit, vt [32][128][Lkv]
  * 16-bit, out [Lq][4096] 16-bit. F32: q, k, v, out [L][4096] f32.
+ * 16-bit modes with Lkv no multiple of 64, where it pays: V^T is first copied,
+ * padded to whole 64-key tiles, into context scratch (calls on different streams
+ * are ordered behind each other's use of it; a call being captured runs the
+ * any-length kernel instead).
  * mode | LTX_ATTN_Q_SCALED (16-bit modes): q already holds
  * q * log2(e) / sqrt(128), as the block's qk-norm writes it (LTX_ST_Q1). */
 #define LTX_ATTN_Q_SCALED 0x100
