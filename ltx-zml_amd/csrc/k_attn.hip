@@ -361,6 +361,7 @@ struct AttnPP {
     const LtxAttnArgs& a;
     __amdgpu_buffer_rsrc_t rk, rv;
     uint32_t gk[2], gv[2];  // per-lane DMA source offsets in tile 0
+    uint32_t gm[2];         // gk's upper bounds: the same chunk of the last K row
     uint32_t kr;            // bytes between consecutive K rows
     int lw;                 // this wave's 2 KB slice of a stage
     uint32_t ok[4];         // K fragment offsets per 32-dim step ks (kb adds 4096)
@@ -380,15 +381,23 @@ struct AttnPP {
     // Group 0 (waves 0-3) issues every DMA: wave w fills its own 2 KB slice
     // of a stage and that of wave w + 4 (8 KB further, K rows + 32 = keys
     // + 32, V^T rows + 64), 4 instructions per K or V tile.
-    template <int S>
+    // K rows past the last repeat it where the tile may be the last one (CLAMP;
+    // the scalar offset takes no part in the buffer's range check).
+    template <bool CLAMP>
+    __device__ __forceinline__ void dma_k1(uint8_t* d, int t, int h, int i) {
+        const uint32_t o = (uint32_t)(64 * t + 32 * h) * kr;
+        if (CLAMP)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (attn_lds_ptr)d, 16, min(gk[i] + o, gm[i]), 0, 0, 0);
+        else
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (attn_lds_ptr)d, 16, gk[i], o, 0, 0);
+    }
+    template <int S, bool CLAMP>
     __device__ __forceinline__ void dma_k(int t) {
         uint8_t* d = app_k<S>() + lw;
 #pragma unroll
         for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (attn_lds_ptr)(d + 8192 * h + 1024 * i), 16, gk[i],
-                                                         (uint32_t)(64 * t + 32 * h) * kr, 0, 0);
+            for (int i = 0; i < 2; i++) dma_k1<CLAMP>(d + 8192 * h + 1024 * i, t, h, i);
     }
     template <int S>
     __device__ __forceinline__ void dma_v(int t) {
@@ -537,7 +546,7 @@ struct AttnPP {
 
     // MFMA phase t then softmax phase t (T4 = t mod 4); returns after the
     // softmax phase's barrier (or after the MFMA phase's when t == nt).
-    // FULL: 1 <= t and t + 2 < nt, every operation present. The wave in its
+    // FULL: 1 <= t and t + 3 < nt, every operation present, the tile t + 2 whole. The wave in its
     // MFMA phase takes issue priority over the other wave of its SIMD.
     //
     // K and V^T both run two tiles ahead in four stages each: the softmax
@@ -560,7 +569,7 @@ struct AttnPP {
         __builtin_amdgcn_sched_barrier(0);
         const bool dkv = FULL || t + 2 < nt;
         if (g == 0 && dkv) {
-            dma_k<(T4 + 2) % 4>(t + 2);
+            dma_k<(T4 + 2) % 4, !FULL>(t + 2);
             dma_v<(T4 + 2) % 4>(t + 2);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -585,8 +594,6 @@ struct AttnPP {
         kr = 2u * (uint32_t)a.k_rs;
         rk = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)a.k + (size_t)h * a.k_hs), 0,
                                                (int)((uint32_t)(lkv - 1) * kr + 2u * LTX_HD), ASP_RSRC_W3);
-        // (K rows past lkv lie past this end: the buffer's range check reads
-        // them as zeros, and their scores are masked)
         rv = __builtin_amdgcn_make_buffer_rsrc((void*)((const uint16_t*)a.vt + (size_t)h * LTX_HD * a.v_rs), 0,
                                                a.v_rs * LTX_HD * 2, ASP_RSRC_W3);
         lw = 2048 * w;
@@ -599,6 +606,7 @@ struct AttnPP {
             const int key = (r & 3) | ((r & 16) >> 2) | ((r & 4) << 1) | ((r & 8) << 1);
             const int c = (lane & 15) ^ (r & 15);
             gk[i] = (uint32_t)key * kr + 16u * c;
+            gm[i] = (uint32_t)(lkv - 1) * kr + 16u * c;
             const int d = 8 * (2 * w + i) + (lane >> 3);
             const int cv = (lane & 7) ^ ((d >> 1) & 7);
             gv[i] = (uint32_t)d * (uint32_t)a.v_rs * 2u + 16u * cv;
@@ -698,9 +706,9 @@ struct AttnPP {
         load_q(qf, h, q0, lane);
         reset();
         if (g == 0) {  // K(0) and V(0) complete, K(1) and V(1) in flight
-            dma_k<0>(0);
+            dma_k<0, true>(0);
             dma_v<0>(0);
-            dma_k<1>(1);
+            dma_k<1, true>(1);
             dma_v<1>(1);
             __builtin_amdgcn_s_waitcnt(ASP_WAIT_VM(8));
         }
@@ -708,7 +716,7 @@ struct AttnPP {
         if (g == 1) __builtin_amdgcn_s_barrier();
         step<0, false>(0);
         int u = 1;
-        for (; u + 5 < nt; u += 4) {
+        for (; u + 6 < nt; u += 4) {
             step<1, true>(u);
             step<2, true>(u + 1);
             step<3, true>(u + 2);
@@ -796,9 +804,7 @@ struct AttnPP {
                 for (int hh = 0; hh < 2; hh++)
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
-                        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                            rk, (attn_lds_ptr)(kres + 16384 * t + lw + 8192 * hh + 1024 * i), 16, gk[i],
-                            (uint32_t)(64 * t + 32 * hh) * kr, 0, 0);
+                        dma_k1<true>(kres + 16384 * t + lw + 8192 * hh + 1024 * i, t, hh, i);
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(
                             rv, (attn_lds_ptr)(vres + 16384 * t + lw + 8192 * hh + 1024 * i), 16, gv[i],
                             t * 128 + 128 * a.v_rs * hh, 0, 0);
