@@ -1,7 +1,7 @@
 // Parts around the blocks (ltx/core_parts.zig), the distilled scheduler
 // (ltx/scheduler.zig) and the denoising loop that drives a stack of resident
 // blocks (ltx/e2e_denoise.zig:218-336). Everything here is f32, as in the
-// reference; the linear layers use the f32 GEMM kernel with bf16 weights.
+// reference; the weights are bf16.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
