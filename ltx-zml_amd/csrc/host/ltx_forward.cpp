@@ -174,6 +174,7 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
 struct Ws32 {
     void *n_msa, *q, *k, *v, *glog1, *o1, *x_sa, *attn_in, *q2, *enc, *k2, *v2, *glog2, *o2, *x_ca, *ff_in, *h;
     void *planes, *part;  // the f3 GEMMs' split of the current A (three bf16 planes) and split-K partial sums
+    size_t planes_bytes;
 };
 
 static void carve32(Carve& c, Ws32& w, size_t T, size_t S, const ltx_ctx* ctx) {
@@ -205,6 +206,7 @@ static void carve32(Carve& c, Ws32& w, size_t T, size_t S, const ltx_ctx* ctx) {
         part = std::max(part, f3_part_bytes(ctx, sh[0], sh[1], sh[2]));
     }
     if (planes) w.planes = c.take(planes);
+    w.planes_bytes = planes;
     if (part) w.part = c.take(part);
 }
 
@@ -500,8 +502,10 @@ static void attn16(ltx_ctx* c, int mode, const void* q, const void* k, const voi
     c->launch(name, a.q_tiles * LTX_H, 1, 1, 512, &a, st, label);
 }
 
-// Splits A [M][K] into the three bf16 planes at `planes` (f3_planes_bytes).
-static void split3(ltx_ctx* c, const float* A, int M, int K, void* planes, hipStream_t st) {
+// Splits A [M][K] into the three bf16 planes at `planes`, of `bytes` (at least
+// f3_planes_bytes).
+static void split3(ltx_ctx* c, const float* A, int M, int K, void* planes, size_t bytes, hipStream_t st) {
+    if (f3_planes_bytes(M, K) > bytes) throw Error("split3: the planes exceed their buffer");
     const size_t n = (size_t)M * K, ps = al(n * 2);
     char* p = (char*)planes;
     LtxSplit3Args a{A, (uint16_t*)p, (uint16_t*)(p + ps), (uint16_t*)(p + 2 * ps), n};
@@ -638,13 +642,15 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         // self-attention (ltx/block.zig:546-547, qAttn1 520-530)
         norm_mod(c, mode, x, b.n_msa, ada, T, 0, 1, st,
              mode == LTX_MODE_F16 ? (const unsigned long long*)w->f16_over.p : nullptr);
-        // the GEMMs' A operands are split into bf16 planes as they are formed
+        // the GEMMs' A operands are split into bf16 planes as they are formed,
+        // where the GEMM that follows (N columns) takes planes: not every
+        // projection does at every token count (f3_shape)
         const void* pl = nullptr;
-        auto split = [&](const void* A, int rows, int K) {
-            pl = b.planes;
-            if (pl) split3(c, (const float*)A, rows, K, b.planes, st);
+        auto split = [&](const void* A, int rows, int N, int K) {
+            pl = b.planes && f3_shape(c, rows, N, K) ? b.planes : nullptr;
+            if (pl) split3(c, (const float*)A, rows, K, b.planes, b.planes_bytes, st);
         };
-        split(b.n_msa, T, LTX_D);
+        split(b.n_msa, T, LTX_D, LTX_D);
         gemm32(c, w->qkv1, 0, LTX_D, (const float*)b.n_msa, T, (float*)b.q, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
         gemm32(c, w->qkv1, LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.k, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
         gemm32(c, w->qkv1, 2 * LTX_D, LTX_D, (const float*)b.n_msa, T, (float*)b.v, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:qkv1", pl, b.part);
@@ -652,28 +658,28 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         qknorm32(c, (float*)b.q, w->qn1.p, cs, sn, T, st);
         qknorm32(c, (float*)b.k, w->kn1.p, cs, sn, T, st);
         attn32(c, (const float*)b.q, (const float*)b.k, (const float*)b.v, (const float*)b.glog1, (float*)b.o1, T, T, st, "attn:self");
-        split(b.o1, T, LTX_D);
+        split(b.o1, T, LTX_D, LTX_D);
         gemm32(c, w->o1, 0, LTX_D, (const float*)b.o1, T, (float*)b.x_sa, LTX_EPI_RESID_GATE, x, ada, 2, 0, st, "gemm:o1", pl, b.part);
         // cross-attention (ltx/block.zig:548-568)
         norm_mod(c, mode, (const float*)b.x_sa, b.attn_in, ada, T, 6, 7, st);
         LtxEncArgs ea{ctxv, (const float*)w->psst.p, pts2, b.enc, S};
         c->launch("ltx_enc_f32", S, 1, 1, 256, &ea, st);
-        split(b.attn_in, T, LTX_D);
+        split(b.attn_in, T, LTX_D, LTX_D);
         gemm32(c, w->q2, 0, LTX_D, (const float*)b.attn_in, T, (float*)b.q2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:q2", pl, b.part);
-        split(b.enc, S, LTX_D);
+        split(b.enc, S, LTX_D, LTX_D);
         gemm32(c, w->kv2, 0, LTX_D, (const float*)b.enc, S, (float*)b.k2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
         gemm32(c, w->kv2, LTX_D, LTX_D, (const float*)b.enc, S, (float*)b.v2, LTX_EPI_STORE, nullptr, ada, 0, 0, st, "gemm:kv2", pl, b.part);
         gate32(c, w->g2, (const float*)b.attn_in, T, (float*)b.glog2, st, "ltx_gate:2");
         qknorm32(c, (float*)b.q2, w->qn2.p, nullptr, nullptr, T, st);
         qknorm32(c, (float*)b.k2, w->kn2.p, nullptr, nullptr, S, st);
         attn32(c, (const float*)b.q2, (const float*)b.k2, (const float*)b.v2, (const float*)b.glog2, (float*)b.o2, T, S, st, "attn:cross");
-        split(b.o2, T, LTX_D);
+        split(b.o2, T, LTX_D, LTX_D);
         gemm32(c, w->o2, 0, LTX_D, (const float*)b.o2, T, (float*)b.x_ca, LTX_EPI_RESID_GATE, (const float*)b.x_sa, ada, 8, 0, st, "gemm:o2", pl, b.part);
         // feed-forward (ltx/block.zig:569-573)
         norm_mod(c, mode, (const float*)b.x_ca, b.ff_in, ada, T, 3, 4, st);
-        split(b.ff_in, T, LTX_D);
+        split(b.ff_in, T, LTX_FF, LTX_D);
         gemm32(c, w->f1, 0, LTX_FF, (const float*)b.ff_in, T, (float*)b.h, LTX_EPI_STORE, nullptr, ada, 0, 1, st, "gemm:ff1", pl, b.part);
-        split(b.h, T, LTX_FF);
+        split(b.h, T, LTX_D, LTX_FF);
         gemm32(c, w->f2, 0, LTX_D, (const float*)b.h, T, y, LTX_EPI_RESID_GATE, (const float*)b.x_ca, ada, 5, 0, st, "gemm:ff2", pl, b.part);
         set_stage(c, LTX_ST_NORM_MSA, b.n_msa, TD * 4);
         set_stage(c, LTX_ST_Q1, b.q, TD * 4);
@@ -933,7 +939,7 @@ void linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, i
             for (int r = 0; r < M; r += step) {
                 const int m = std::min(step, M - r);
                 const float* ar = (const float*)a + (size_t)r * K;
-                if (f3) split3(c, ar, m, K, sc.planes, st);
+                if (f3) split3(c, ar, m, K, sc.planes, f3_planes_bytes(sc.plane_rows, K), st);
                 gemm32(c, p, 0, N, ar, m, (float*)y + (size_t)r * N, LTX_EPI_STORE, nullptr, ada, 0, gelu, st, nullptr,
                        f3 ? sc.planes : nullptr, sc.part, ks);
             }

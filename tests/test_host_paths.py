@@ -1,0 +1,32 @@
+"""The host code on a recording stand-in for the HIP runtime
+(tests/host/fake_hip.hpp): the sizes, routes and orders of what a call
+allocates and launches, at shapes and in situations that need no GPU."""
+import pathlib
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parent.parent
+PKG = ROOT / "ltx-zml_amd"
+
+
+@pytest.fixture(scope="session")
+def host_paths(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("host") / "host_paths"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-Wno-unused-result", "-rdynamic",
+                    "-I/opt/rocm/include", f"-I{ROOT / 'include'}", f"-I{PKG / 'csrc'}", f"-I{PKG / 'csrc' / 'host'}",
+                    str(ROOT / "tests" / "host" / "host_paths.cpp"), "-o", str(exe), str(PKG / "libltx_amd.so"),
+                    f"-Wl,-rpath,{PKG}", "-Wl,--allow-shlib-undefined", "-pthread"], check=True)
+
+    def run(*args):
+        r = subprocess.run([str(exe), *map(str, args)], capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0 and r.stdout.endswith("ok\n"), r.stdout + r.stderr
+        return r.stdout
+    return run
+
+
+@pytest.mark.parametrize("T,S", [(1024, 128), (65535, 128), (65536, 128), (262143, 77), (262144, 128), (64, 262144)])
+def test_f32_block_planes_fit_their_room(host_paths, T, S):
+    """Token counts on both sides of where the GEMM on planes stops taking the
+    K = 16,384 projection (65,536) and the K = 4,096 ones (262,144)."""
+    host_paths("f32_planes", T, S)
