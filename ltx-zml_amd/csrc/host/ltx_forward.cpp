@@ -1109,11 +1109,10 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         ltx::LinearScratch sc{};
         hipStream_t st = (hipStream_t)stream;
         // mode F32 splits A into planes (not captured: then the f32 MFMA kernel)
-        bool used = false;  // c->op_scratch
+        ltx::ScratchUse use(c->op_scratch, st);
         if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
             const size_t np = ltx::f3_planes_bytes(M, K), need = np + ltx::f3_part_bytes(c, M, N, K);
-            if ((sc.planes = c->op_scratch.take(need, st))) {
-                used = true;
+            if ((sc.planes = use.take(need))) {
                 sc.plane_rows = M;
                 sc.part = need > np ? (char*)sc.planes + np : nullptr;
             }
@@ -1121,7 +1120,7 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         // 16-bit modes: split-K partial sums (not captured: then no split)
         const bool packed = ltx::linear_packed(a, q, scales, scale_f16, bias, y, K);
         if (const size_t np = packed ? ltx::linear_part_bytes(c, M, N, K, mode) : 0)
-            used = (sc.part = c->op_scratch.take(np, st)) != nullptr;
+            sc.part = use.take(np);
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
             // scratch owned by the context, grown as needed
             const size_t nq = (size_t)N * K, np = (size_t)N * (K / LTX_GROUP) * 4;
@@ -1135,7 +1134,6 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
             }
         }
         ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, st);
-        if (used) c->op_scratch.done(st);
     })
 }
 
@@ -1157,12 +1155,12 @@ int ltx_op_attention(ltx_ctx* c, const void* q, const void* k, const void* v, co
         // captured: then the any-length kernel)
         const int vld = ltx::vt_ld(lkv);
         void* pad = nullptr;
-        if (vld != lkv && c->attn_pp && ltx::pad_pays(c, lq, lkv) && (pad = c->op_scratch.take((size_t)LTX_D * vld * 2, st))) {
+        ltx::ScratchUse use(c->op_scratch, st);
+        if (vld != lkv && c->attn_pp && ltx::pad_pays(c, lq, lkv) && (pad = use.take((size_t)LTX_D * vld * 2))) {
             LtxVtPadArgs pa{(const uint16_t*)v, (uint16_t*)pad, lkv, vld};
             c->launch("ltx_vt_pad", (vld + 511) / 512, LTX_D / 4, 1, 256, &pa, st);
         }
         ltx::attn16(c, mode, q, k, pad ? pad : v, pad ? vld : lkv, glog, out, lq, lkv, q_scaled, st);
-        if (pad) c->op_scratch.done(st);
     })
 }
 

@@ -42,20 +42,36 @@ struct DevBuf {
 
 // Scratch of the isolated operators that needed none before they had it: one
 // buffer per context, kept and grown. Calls on different streams stay
-// independent for the caller: take() makes the stream wait for the last use on
-// another one (done()). It returns NULL to a call that is being captured, whose
-// replays nothing here could order and which may not allocate; the caller then
-// runs the kernel that needs no scratch.
+// independent for the caller: take() makes the stream wait for the last use
+// (done()). On the same stream too, where the wait costs nothing: a handle does
+// not identify a stream (the per-thread stream has one for every thread, and a
+// destroyed stream's may come back while its work is in flight). It returns NULL
+// to a call that is being captured, whose replays nothing here could order and
+// which may not allocate; the caller then runs the kernel that needs no scratch.
 struct StreamScratch {
     DevBuf buf;
     hipEvent_t ev = nullptr;
-    hipStream_t last = nullptr;
     bool used = false;
     void* take(size_t bytes, hipStream_t st);
-    void done(hipStream_t st);
+    void done(hipStream_t st) noexcept;
     ~StreamScratch() {
         if (ev) (void)hipEventDestroy(ev);
     }
+};
+
+// One call's use of the scratch: recorded when the scope ends, also when the
+// call fails with part of its work enqueued.
+struct ScratchUse {
+    StreamScratch& s;
+    hipStream_t st;
+    void* p = nullptr;
+    ScratchUse(StreamScratch& scratch, hipStream_t stream) : s(scratch), st(stream) {}
+    void* take(size_t bytes) { return p = s.take(bytes, st); }
+    ~ScratchUse() {
+        if (p) s.done(st);
+    }
+    ScratchUse(const ScratchUse&) = delete;
+    ScratchUse& operator=(const ScratchUse&) = delete;
 };
 
 struct ProfRec {

@@ -59,14 +59,15 @@ void* StreamScratch::take(size_t bytes, hipStream_t st) {
     if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
     if (!ev) HIPC(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (buf.bytes < bytes) buf.alloc(bytes);  // (hipFree of the old one waits for the device)
-    if (used && last != st) HIPC(hipStreamWaitEvent(st, ev, 0));
+    if (used) HIPC(hipStreamWaitEvent(st, ev, 0));
     return buf.p;
 }
 
-void StreamScratch::done(hipStream_t st) {
-    HIPC(hipEventRecord(ev, st));
-    last = st;
-    used = true;
+void StreamScratch::done(hipStream_t st) noexcept {
+    if (hipEventRecord(ev, st) == hipSuccess)
+        used = true;
+    else
+        (void)hipStreamSynchronize(st);  // nothing to wait for later
 }
 
 uint16_t f32_to_f16_bits(float f) {  // round to nearest even, IEEE binary16

@@ -81,12 +81,65 @@ static void f32_planes(int T, int S) {
     std::printf("%d splits\n", splits);
 }
 
+static bool linear(ltx_ctx* c, int M, int N, int K, int mode, hipStream_t st, bool noalloc = false, size_t off = 0) {
+    auto f = noalloc ? ltx_op_linear_q8_noalloc : ltx_op_linear_q8;
+    return f(c, ptr(0), (const int8_t*)ptr(1) + off, ptr(2), 1, nullptr, ptr(3), mode == LTX_MODE_F32, M, N, K, 0, mode,
+             st);
+}
+static bool attention(ltx_ctx* c, int lq, int lkv, hipStream_t st) {
+    return ltx_op_attention(c, ptr(0), ptr(1), ptr(2), nullptr, ptr(3), lq, lkv, LTX_MODE_F16, st);
+}
+
+// The uses of one shared scratch follow each other, whatever the stream's
+// handle (the per-thread stream has one handle for all threads, and a destroyed
+// stream's may come back): between two uses lies a record behind the first and a
+// wait for it before the second. A call that fails half-way counts as a use.
+// `scratch` names the kernels that write it, `call` makes one call on a stream.
+template <class Call>
+static void scratch_order(const char* scratch, const char* reader, Call call) {
+    const hipStream_t s1 = (hipStream_t)0x10, s2 = (hipStream_t)0x20;
+    CHECK(call(s1), "%s", ltx_last_error(nullptr));
+    fake::log.clear();
+    int n = 0;
+    auto uses = [&]() {  // checks the calls logged so far
+        hipEvent_t behind = nullptr;  // recorded behind the last use, and waited for
+        bool recorded = false, waited = false;
+        n = 0;
+        for (const fake::Op& o : fake::log) {
+            if (o.what == "record") behind = o.event, recorded = true, waited = false;
+            if (o.what == "wait" && recorded && o.event == behind) waited = true;
+            if (o.what == "launch" && o.name.rfind(scratch, 0) == 0) {
+                CHECK(!n || (recorded && waited), "use %d: %s%s", n + 1, recorded ? "recorded " : "not recorded ",
+                      waited ? "waited" : "not waited");
+                recorded = waited = false;
+                n++;
+            }
+        }
+    };
+    for (hipStream_t s : {s1, s1, s2, s1}) CHECK(call(s), "%s", ltx_last_error(nullptr));
+    uses();
+    CHECK(n == 4, "%d uses", n);
+    fake::fail_launch = reader;
+    CHECK(!call(s1), "a failed launch went unnoticed");
+    fake::fail_launch.clear();
+    CHECK(call(s2), "%s", ltx_last_error(nullptr));
+    uses();
+    CHECK(n == 6, "%d uses", n);
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
     if (cmd == "f32_planes")
         f32_planes(arg(2), arg(3));
-    else
+    else if (cmd == "scratch_order_planes") {
+        ltx_ctx* c = make_ctx();
+        scratch_order("ltx_split3", "ltx_gemm_f3_i8f16_store",
+                      [&](hipStream_t st) { return linear(c, 1000, 4096, 512, LTX_MODE_F32, st); });
+    } else if (cmd == "scratch_order_vt") {
+        ltx_ctx* c = make_ctx();
+        scratch_order("ltx_vt_pad", "ltx_attn_f16_pp_uq", [&](hipStream_t st) { return attention(c, 2970, 2970, st); });
+    } else
         CHECK(false, "unknown command %s", cmd.c_str());
     std::printf("ok\n");
     std::fflush(stdout);

@@ -30,3 +30,11 @@ def test_f32_block_planes_fit_their_room(host_paths, T, S):
     """Token counts on both sides of where the GEMM on planes stops taking the
     K = 16,384 projection (65,536) and the K = 4,096 ones (262,144)."""
     host_paths("f32_planes", T, S)
+
+
+@pytest.mark.parametrize("scratch", ["planes", "vt"])
+def test_operator_scratch_is_ordered(host_paths, scratch):
+    """Calls that share a context's operator scratch (mode F32's planes, the
+    attention's padded V^T) follow each other: on one stream handle, on two, and
+    behind a call that failed between its launches."""
+    host_paths(f"scratch_order_{scratch}")
