@@ -209,10 +209,15 @@ int ltx_range_count(ltx_ctx* ctx, void* stream, uint64_t* count, int reset);
  * different streams may overwrite that scratch, so keep one context's calls on
  * one stream. Mode F32 with N a multiple of 128 splits a into three bf16 planes
  * in context scratch; calls on different streams are ordered behind each other's
- * use of it. A call being captured takes no scratch for planes or partial sums:
- * it runs the kernels that need none (the same products summed in another
- * order). A shape with M, N or K not positive or K not a
- * multiple of 128, or an unknown mode, is refused (status 0, ltx_last_error)
+ * use of it. A call being captured, or one that finds no memory for it, takes no
+ * scratch for planes or partial sums. In the 16-bit modes it then sums the same
+ * products in another order (no split of K); in mode F32 it runs the f32 MFMA
+ * kernel, which rounds every scaled weight to f32 (at 1,024 x 12,288 x 4,096 an
+ * error of 1.1e-6 against 64 bits instead of 1.6e-7) and takes three times as
+ * long. Growing the planes' and partial sums' scratch is allowed beside a
+ * capture on another stream, in any capture mode. A shape with M, N or K not
+ * positive or K not a multiple of 128, or an unknown mode, is refused (status 0,
+ * ltx_last_error)
  * before any scratch is sized or allocated. */
 int ltx_op_linear_q8(ltx_ctx* ctx, const void* a, const int8_t* q, const void* scales, int scale_f16,
                      const float* bias, void* y, int out_f32, int M, int N, int K, int gelu, int mode,
@@ -242,9 +247,10 @@ int ltx_op_linear_q8_noalloc(ltx_ctx* ctx, const void* a, const int8_t* q, const
  * NULL for no gate). F16/BF16: q, k [32][L][128] 16-bit, vt [32][128][Lkv]
  * 16-bit, out [Lq][4096] 16-bit. F32: q, k, v, out [L][4096] f32.
  * 16-bit modes with Lkv no multiple of 64, where it pays: V^T is first copied,
- * padded to whole 64-key tiles, into context scratch (calls on different streams
- * are ordered behind each other's use of it; a call being captured runs the
- * any-length kernel instead).
+ * padded to whole 64-key tiles, into context scratch of V's size (calls on
+ * different streams are ordered behind each other's use of it, and it may grow
+ * beside a capture on another stream; a call being captured, or one that finds
+ * no memory for it, runs the any-length kernel instead, at about half the speed).
  * mode | LTX_ATTN_Q_SCALED (16-bit modes): q already holds
  * q * log2(e) / sqrt(128), as the block's qk-norm writes it (LTX_ST_Q1). */
 #define LTX_ATTN_Q_SCALED 0x100

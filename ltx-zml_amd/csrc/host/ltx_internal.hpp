@@ -33,6 +33,7 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0;
     void alloc(size_t n);
+    bool try_grow(size_t n);
     void free_();
     ~DevBuf() { free_(); }
     DevBuf() = default;
@@ -47,7 +48,8 @@ struct DevBuf {
 // not identify a stream (the per-thread stream has one for every thread, and a
 // destroyed stream's may come back while its work is in flight). It returns NULL
 // to a call that is being captured, whose replays nothing here could order and
-// which may not allocate; the caller then runs the kernel that needs no scratch.
+// which may not allocate, and where there is no memory; the caller then runs the
+// kernel that needs no scratch.
 struct StreamScratch {
     DevBuf buf;
     hipEvent_t ev = nullptr;

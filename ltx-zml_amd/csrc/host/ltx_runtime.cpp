@@ -54,11 +54,39 @@ void DevBuf::free_() {
     bytes = 0;
 }
 
-void* StreamScratch::take(size_t bytes, hipStream_t st) {
+// Room of at least n bytes, or false: no memory, also without the old room.
+// Freeing that waits for the device.
+bool DevBuf::try_grow(size_t n) {
+    if (bytes >= n) return true;
+    // A caller may be capturing another stream in the global mode, which forbids
+    // hipMalloc and hipFree to every thread that has not opted out; nothing here
+    // touches that stream.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* q = nullptr;
+    bool ok = hipMalloc(&q, n) == hipSuccess;
+    if (p) {
+        free_();
+        if (!ok) ok = hipMalloc(&q, n) == hipSuccess;
+    }
+    if (ok) {
+        p = q;
+        bytes = n;
+    }
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) (void)hipGetLastError();  // handled here: clear it for later callers
+    return ok;
+}
+
+void* StreamScratch::take(size_t n, hipStream_t st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) return nullptr;
+    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
     if (!ev) HIPC(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    if (buf.bytes < bytes) buf.alloc(bytes);  // (hipFree of the old one waits for the device)
+    if (!buf.try_grow(n)) return nullptr;
     if (used) HIPC(hipStreamWaitEvent(st, ev, 0));
     return buf.p;
 }

@@ -127,6 +127,44 @@ static void scratch_order(const char* scratch, const char* reader, Call call) {
     CHECK(n == 6, "%d uses", n);
 }
 
+static int launches(const std::string& prefix) {
+    int n = 0;
+    for (const fake::Op& o : fake::log) n += o.what == "launch" && o.name.rfind(prefix, 0) == 0;
+    return n;
+}
+
+// The scratch grows for a call beside a stream that is being captured in global
+// mode: the call runs as it always does and the capture stays whole.
+static void scratch_capture() {
+    ltx_ctx* c = make_ctx();
+    const hipStream_t s1 = (hipStream_t)0x10, other = (hipStream_t)0x20;
+    CHECK(attention(c, 2970, 70, s1) && linear(c, 200, 256, 256, LTX_MODE_F32, s1), "%s", ltx_last_error(c));
+    fake::capturing.insert(other);
+    fake::log.clear();
+    CHECK(attention(c, 2970, 2970, s1), "attention: %s", ltx_last_error(c));
+    CHECK(launches("ltx_vt_pad") == 1, "%d paddings", launches("ltx_vt_pad"));
+    CHECK(linear(c, 8000, 4096, 4096, LTX_MODE_F32, s1), "linear: %s", ltx_last_error(c));
+    CHECK(launches("ltx_split3") == 1, "%d splits", launches("ltx_split3"));
+    CHECK(!fake::broken_capture, "the other stream's capture is broken");
+    CHECK(fake::thread_mode == hipStreamCaptureModeGlobal, "the thread's capture mode is changed");
+}
+
+// No memory for scratch: the calls run on the kernels that need none, and take
+// the scratch again when there is memory.
+static void scratch_memory() {
+    ltx_ctx* c = make_ctx();
+    const hipStream_t s1 = (hipStream_t)0x10;
+    CHECK(attention(c, 2970, 70, s1), "%s", ltx_last_error(c));
+    fake::limit = fake::in_use + (1 << 20);
+    fake::log.clear();
+    CHECK(attention(c, 2970, 2970, s1), "attention: %s", ltx_last_error(c));
+    CHECK(launches("ltx_attn_f16_w8") == 1 && !launches("ltx_vt_pad"), "not the any-length kernel");
+    CHECK(linear(c, 2000, 4096, 4096, LTX_MODE_F32, s1), "linear: %s", ltx_last_error(c));
+    CHECK(launches("ltx_gemm_f32") == 1 && !launches("ltx_split3"), "not the f32 MFMA kernel");
+    fake::limit = ~0ull;
+    CHECK(attention(c, 2970, 2970, s1) && launches("ltx_vt_pad") == 1, "%s", ltx_last_error(c));
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -139,7 +177,11 @@ int main(int argc, char** argv) {
     } else if (cmd == "scratch_order_vt") {
         ltx_ctx* c = make_ctx();
         scratch_order("ltx_vt_pad", "ltx_attn_f16_pp_uq", [&](hipStream_t st) { return attention(c, 2970, 2970, st); });
-    } else
+    } else if (cmd == "scratch_capture")
+        scratch_capture();
+    else if (cmd == "scratch_memory")
+        scratch_memory();
+    else
         CHECK(false, "unknown command %s", cmd.c_str());
     std::printf("ok\n");
     std::fflush(stdout);

@@ -479,6 +479,34 @@ def test_attention_ragged_keys_captured(ctx):
         assert oracle.rel_rms(f64(out), f64(eager)) <= 2e-3, i
 
 
+def test_operator_scratch_grows_beside_a_capture(ctx):
+    """An eager call whose scratch grows while another stream is captured in the
+    global mode: it runs, and the capture is whole."""
+    say("operator scratch grows beside a capture")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn(32, n, d, generator=g, device="cuda").half() for n, d in ((2100, 128), (2100, 128), (128, 2100)))
+    out, want = (torch.empty(2100, 4096, dtype=torch.float16, device="cuda") for _ in range(2))
+    ctx.attention(q, k, v, None, want, 2100, 2100)
+    c, other, x = rt.Context(0), torch.cuda.Stream(), torch.zeros(1024, device="cuda")
+    try:
+        # the same kernels on less scratch first
+        c.attention(q, k, v[:, :, :130].contiguous(), None, out, 2100, 130)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, capture_error_mode="global"):
+            x.add_(1)
+            c.attention(q, k, v, None, out, 2100, 2100, stream=other)
+            x.add_(1)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        for _ in range(3):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert (x == 6).all()
+    finally:
+        c.close()
+
+
 @pytest.mark.parametrize("lq,lkv", [(130, 70), (1000, 1000), (257, 193), (64, 1)])
 def test_attention_f32_mode(ctx, lq, lkv):
     say(f"attention mode=f32 lq={lq} lkv={lkv}")

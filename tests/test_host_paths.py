@@ -38,3 +38,11 @@ def test_operator_scratch_is_ordered(host_paths, scratch):
     attention's padded V^T) follow each other: on one stream handle, on two, and
     behind a call that failed between its launches."""
     host_paths(f"scratch_order_{scratch}")
+
+
+def test_operator_scratch_grows_beside_a_capture(host_paths):
+    host_paths("scratch_capture")
+
+
+def test_operator_scratch_without_memory(host_paths):
+    host_paths("scratch_memory")
