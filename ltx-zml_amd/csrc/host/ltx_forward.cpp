@@ -741,10 +741,13 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     // then the context side (K/V modulation, k|v GEMM with its own partial sums,
     // k norm), and later the cross-attention's gate logits beside the q2 GEMM
     // (1,024 tokens: 653 us; with the gate logits on the main stream 667, with
-    // the context side from the start 669). Where that GEMM fills the chip, side
-    // work beside it would wait for its end and then slow the q and k norms: the
-    // context side starts with the forward, beside the first norm, and the gate
-    // logits run on the main stream (2,970 tokens: 1,613 against 1,645 us).
+    // the context side from the start 669). So also beside the 16-bit-weight GEMM
+    // (256 x 128 tiles), full or not: the gate logits fit its CUs (2,048 tokens,
+    // unquantised: 1,030 us; 1,090 with them on the main stream). Where another
+    // GEMM fills the chip, side work beside it would wait for its end and then
+    // slow the q and k norms: the context side starts with the forward, beside
+    // the first norm, and the gate logits run on the main stream (2,970 tokens:
+    // 1,613 against 1,645 us).
     // Large T: side work starts only after the persistent GEMMs, whose
     // one-workgroup-per-CU grids it would otherwise hold back, and ends before
     // the attentions, which it would slow as much as it gains.
@@ -756,7 +759,8 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     };
     if (early) {
         const int tr = tile_rows(c, T, 3 * LTX_D), last = (T + tr - 1) / tr * (3 * LTX_D / 256) % c->num_cu;
-        side_gates = last > 0 && last <= c->num_cu - c->num_cu / 8;
+        const bool w16 = !w->qkv1.q8 && !x4_shape(c, mode, T, 3 * LTX_D, LTX_D, LTX_D, true);  // 256 x 128 tiles
+        side_gates = w16 || (last > 0 && last <= c->num_cu - c->num_cu / 8);
         if (!side_gates) {
             stream_after(sd, st, c->side_ev[0]);
             fail_check();

@@ -252,11 +252,14 @@ extern "C" __global__ void __launch_bounds__(256) ltx_gemm_dq16_bf16_s32(const L
 // Bound by reading a. A workgroup of 8 waves takes 16 rows, each wave 512 of
 // the 4,096 channels (its 48 operand loads straight from global memory, all in
 // flight before its 32 MFMAs: the 32 x 4,096 weight stays in L2), and the
-// waves' sums meet in LDS.
+// waves' sums meet in the first. Its 14 KB of LDS and 64 registers a lane fit
+// beside a workgroup of the 16-bit-weight GEMM (256 x 128 tiles: 144 KB, two
+// waves of 192 registers a SIMD; LDS goes in pieces of 1,280 B), so beside that
+// GEMM the logits cost nothing.
 template <typename T>
 __device__ void gate_body(const LtxGateArgs& a) {
     typedef typename Op<T>::v8 v8;
-    __shared__ float part[8][16][LTX_H + 1];
+    __shared__ f32x4 part[7][2][64];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int lr = lane & 15, lg = lane >> 4;
     const int m0 = blockIdx.x * 16, c0 = 512 * w + 8 * lg;
@@ -272,14 +275,20 @@ __device__ void gate_body(const LtxGateArgs& a) {
     }
 #pragma unroll
     for (int nb = 0; nb < 2; nb++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) part[w][4 * lg + i][16 * nb + lr] = acc[nb][i];
+        if (w) part[w - 1][nb][lane] = acc[nb];
     __syncthreads();
-    const int row = tid >> 5, h = tid & 31;
-    float o = 0.f;
+    if (w) return;
 #pragma unroll
-    for (int i = 0; i < 8; i++) o += part[i][row][h];
-    if (m0 + row < a.M) a.out[(size_t)(m0 + row) * LTX_H + h] = o + a.gb[h];
+    for (int nb = 0; nb < 2; nb++) {
+#pragma unroll
+        for (int i = 0; i < 7; i++) acc[nb] += part[i][nb][lane];  // in wave order
+        const float gb = a.gb[16 * nb + lr];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int m = m0 + 4 * lg + i;
+            if (m < a.M) a.out[(size_t)m * LTX_H + 16 * nb + lr] = acc[nb][i] + gb;
+        }
+    }
 }
 
 extern "C" __global__ void __launch_bounds__(512) ltx_gate_f16(const LtxGateArgs a) { gate_body<_Float16>(a); }

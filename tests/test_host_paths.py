@@ -2,6 +2,7 @@
 (tests/host/fake_hip.hpp): the sizes, routes and orders of what a call
 allocates and launches, at shapes and in situations that need no GPU."""
 import pathlib
+import re
 import subprocess
 
 import pytest
@@ -46,3 +47,27 @@ def test_operator_scratch_grows_beside_a_capture(host_paths):
 
 def test_operator_scratch_without_memory(host_paths):
     host_paths("scratch_memory")
+
+
+def test_gate_logits_fit_beside_the_16_bit_gemm(tmp_path):
+    """The gate logits run on the second stream beside the 16-bit-weight GEMM
+    (unquantised blocks up to 2,048 tokens): a workgroup of theirs has to fit
+    what that GEMM leaves of a CU. 160 KB of LDS in pieces of 1,280 bytes; 512
+    registers a lane of a SIMD, in eights, for two waves of each."""
+    bundle = PKG / "_build" / "k_gemm.hsaco"
+    llvm = pathlib.Path("/opt/rocm/llvm/bin")
+    if not bundle.exists() or not (llvm / "llvm-readelf").exists():
+        pytest.skip("no built code object, or no LLVM tools to read it")
+    co = tmp_path / "k_gemm.co"
+    subprocess.run([llvm / "clang-offload-bundler", "--type=o", "--unbundle",
+                    "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--input={bundle}", f"--output={co}"], check=True)
+    notes = subprocess.run([llvm / "llvm-readelf", "--notes", co], capture_output=True, text=True, check=True).stdout
+    kernels = {}
+    for entry in re.split(r"\n  - \.agpr_count", notes)[1:]:
+        get = lambda key: re.search(rf"\.{key}:\s+(\S+)", entry)[1]  # noqa: E731
+        kernels[get("name")] = (int(get("group_segment_fixed_size")), int(get("vgpr_count")))
+    for dt in ("f16", "bf16"):
+        gate = kernels[f"ltx_gate_{dt}"]
+        for gemm in (kernels[f"ltx_gemm_w16dma_{dt}_qkv"], kernels[f"ltx_gemm_w16dma_{dt}_store"]):
+            assert sum(-(-lds // 1280) * 1280 for lds, _ in (gate, gemm)) <= 160 * 1024
+            assert sum(2 * -(-regs // 8) * 8 for _, regs in (gate, gemm)) <= 512
