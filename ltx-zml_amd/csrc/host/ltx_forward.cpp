@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
+#include <numeric>
 
 #include "ltx_internal.hpp"
 
@@ -110,6 +111,17 @@ size_t f3_planes_bytes(int M, int K) { return 3 * al((size_t)M * K * 2); }
 size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K) {
     const int s = gemm_ksplit(c->num_cu, M, N, K, 128, 128);
     return s > 1 ? (size_t)s * M * N * 4 : 0;
+}
+
+int f3_rows(const ltx_ctx* c, int M, int N, int K, size_t room) {
+    const size_t row = 3 * (size_t)K * 2 + f3_part_bytes(c, M, N, K) / M, pad = 3 * 256;  // al() of three planes
+    if (room < pad) return 0;
+    const size_t most = (room - pad) / row;
+    if (most >= (size_t)M) return M;
+    // whole rounds of one tile a CU, or a pass's last round idles (28,672 x 4,096
+    // x 16,384 in six even passes 12.1 ms, in whole rounds and in one pass 11.4)
+    const int tiles = (int)(most / 128), q = c->num_cu / std::gcd(N / 128, c->num_cu);
+    return (tiles >= q ? tiles / q * q : tiles) * 128;
 }
 
 // Whether the small-grid kernel gathers the isolated GEMM's scales as packed
@@ -1104,6 +1116,10 @@ void ltx_block_graph_destroy(ltx_block_graph* g) {
     delete g;
 }
 
+// Mode F32's planes (and partial sums) take at most this of the operator
+// scratch, which the context keeps: operands of more rows go in passes.
+static constexpr size_t kPlanesMax = 512u << 20;
+
 int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* scales, int scale_f16, const float* bias,
                      void* y, int out_f32, int M, int N, int K, int gelu, int mode, void* stream) {
     LTX_GUARD(c, {
@@ -1115,10 +1131,11 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         // mode F32 splits A into planes (not captured: then the f32 MFMA kernel)
         ltx::ScratchUse use(c->op_scratch, st);
         if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
-            const size_t np = ltx::f3_planes_bytes(M, K), need = np + ltx::f3_part_bytes(c, M, N, K);
-            if ((sc.planes = use.take(need))) {
-                sc.plane_rows = M;
-                sc.part = need > np ? (char*)sc.planes + np : nullptr;
+            const int rows = ltx::f3_rows(c, M, N, K, kPlanesMax);
+            const size_t part = ltx::f3_part_bytes(c, M, N, K) / M * rows, np = ltx::f3_planes_bytes(rows, K);
+            if (rows && (sc.planes = use.take(np + part))) {
+                sc.plane_rows = rows;
+                sc.part = part ? (char*)sc.planes + np : nullptr;
             }
         }
         // 16-bit modes: split-K partial sums (not captured: then no split)

@@ -233,6 +233,9 @@ bool s4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool q8)
 bool f3_shape(const ltx_ctx* c, int M, int N, int K);
 size_t f3_planes_bytes(int M, int K);
 size_t f3_part_bytes(const ltx_ctx* c, int M, int N, int K);
+// The rows of a pass whose planes and partial sums fit `room`: M, or whole
+// 128-row tiles, or 0 (not one tile fits).
+int f3_rows(const ltx_ctx* c, int M, int N, int K, size_t room);
 // The isolated int8 GEMM: 16-byte aligned operands; in the 16-bit modes also
 // whether the kernels take the weights and scales as packed (f16 scales: an even
 // number of groups); and the bytes of its split-K partial sums, used with the

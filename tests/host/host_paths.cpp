@@ -165,6 +165,43 @@ static void scratch_memory() {
     CHECK(attention(c, 2970, 2970, s1) && launches("ltx_vt_pad") == 1, "%s", ltx_last_error(c));
 }
 
+// Mode F32's planes stay below 512 MiB: larger operands go in passes of whole
+// 128-row tiles, each on planes and partial sums inside the scratch, and
+// together all of the rows with one split of K.
+static void planes_bound(int M, int N, int K, bool noalloc) {
+    ltx_ctx* c = make_ctx();
+    fake::log.clear();
+    CHECK(linear(c, M, N, K, LTX_MODE_F32, nullptr, noalloc), "%s", ltx_last_error(c));
+    CHECK(c->op_scratch.buf.bytes <= (512u << 20), "%zu bytes kept", c->op_scratch.buf.bytes);
+    size_t row = 0;
+    const fake::Op* split = nullptr;
+    int ks = 0;
+    for (const fake::Op& o : fake::log) {
+        if (o.name == "ltx_split3") {
+            split = &o;
+            CHECK(o.split.x == ptr(0) + row * K, "a pass starts elsewhere than at row %zu", row);
+            for (uint16_t* p : {o.split.p0, o.split.p1, o.split.p2})
+                CHECK(fake::inside(p, 2 * o.split.n), "planes of %zu values outside the scratch", o.split.n);
+        }
+        if (o.name.rfind("ltx_gemm_f3_", 0) == 0) {
+            const LtxGemmArgs& g = o.f3.g;
+            CHECK(split && g.a == split->split.p0 && o.f3.a2 == split->split.p2, "not the planes just split");
+            CHECK((size_t)g.M * K == split->split.n && g.out == (char*)ptr(3) + row * N * 4, "not the rows just split");
+            CHECK(!ks || g.ksplit == ks, "split of K %d, then %d", ks, g.ksplit);
+            ks = g.ksplit;
+            if (ks > 1)
+                CHECK(g.part >= (const float*)((const char*)split->split.p2 + 2 * split->split.n) &&
+                          fake::inside(g.part, (size_t)ks * g.M * N * 4),
+                      "partial sums outside the scratch");
+            row += g.M;
+            CHECK(row == (size_t)M || g.M % 128 == 0, "a pass of %d rows", g.M);
+            split = nullptr;
+        }
+    }
+    CHECK(row == (size_t)M, "%zu of %d rows", row, M);
+    std::printf("%d passes, %zu bytes\n", launches("ltx_split3"), c->op_scratch.buf.bytes);
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -181,6 +218,8 @@ int main(int argc, char** argv) {
         scratch_capture();
     else if (cmd == "scratch_memory")
         scratch_memory();
+    else if (cmd == "planes_bound")
+        planes_bound(arg(2), arg(3), arg(4), false);
     else
         CHECK(false, "unknown command %s", cmd.c_str());
     std::printf("ok\n");

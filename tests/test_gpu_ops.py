@@ -375,6 +375,23 @@ def test_linear_q8_f32_planes_nonfinite_and_streams(ctx):
         assert torch.equal(o, w)
 
 
+def test_linear_q8_f32_planes_in_passes(ctx):
+    """6,000 rows of K = 16,384 exceed the planes' 512 MiB: two passes, the bits
+    of two calls of one pass each (no split of K in either)."""
+    say("linear_q8 f32 planes in passes")
+    M, N, K = 6000, 2048, 16384
+    g = torch.Generator(device="cuda").manual_seed(6)
+    a = torch.randn(M, K, generator=g, device="cuda")
+    q = torch.randint(-128, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+    s = torch.rand(N, K // 128, generator=g, device="cuda") * 0.01
+    y, halves = (torch.full((M, N), float("nan"), device="cuda") for _ in range(2))
+    ctx.linear_q8(a, q, s, None, y, mode=rt.MODE_F32)
+    for h in (slice(0, 3000), slice(3000, M)):
+        ctx.linear_q8(a[h], q, s, None, halves[h], mode=rt.MODE_F32)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y).all() and torch.equal(y, halves)
+
+
 def _heads(x, L):  # [L, D] -> [H, L, 128]
     return np.ascontiguousarray(x.reshape(L, 32, 128).transpose(1, 0, 2))
 

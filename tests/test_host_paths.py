@@ -49,6 +49,12 @@ def test_operator_scratch_without_memory(host_paths):
     host_paths("scratch_memory")
 
 
+@pytest.mark.parametrize("M,N,K", [(1024, 12288, 4096), (1, 128, 128), (300, 256, 4096), (28672, 4096, 16384),
+                                   (5377, 4096, 16384), (65535, 128, 16384), (200000, 128, 4096), (129, 128, 32768)])
+def test_f32_linear_planes_are_bounded(host_paths, M, N, K):
+    host_paths("planes_bound", M, N, K)
+
+
 def test_gate_logits_fit_beside_the_16_bit_gemm(tmp_path):
     """The gate logits run on the second stream beside the 16-bit-weight GEMM
     (unquantised blocks up to 2,048 tokens): a workgroup of theirs has to fit
