@@ -431,16 +431,26 @@ static void gate16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
 // Whether ltx_op_attention pads V^T (lkv no multiple of 64) for the LDS-DMA
 // kernels. The padding launch costs 7 to 9 us; the any-length kernel takes about
 // twice as long a round of workgroups and key tile, less where 8 divides lkv
-// (it then loads V^T in 16-byte vectors). Measured, padded against any-length,
-// us (lq x lkv): four or more rounds 7,001 x 16 38 : 54, 7,001 x 200 55 : 67;
-// two 2,970 x 50 27 : 22, 2,970 x 77 27 : 27, 2,970 x 129 29 : 33, 2,970 x
-// 2,970 154 : 278; one 1,000 x 200 20 : 15, 1,000 x 255 20 : 21, 1,000 x 500
-// 25 : 30, 1,000 x 1,000 (8 divides) 38 : 34.
+// (it then loads V^T in 16-byte vectors) and where its last round has few
+// workgroups (they have their CUs to themselves). Measured, padded against
+// any-length, us, by rounds and the last one's share of the CUs (lq x lkv, f16):
+// four or more: 6,145 x 16 37 : 40, 7,001 x 200 56 : 67;
+// three, an eighth: 4,200 x 72 35 : 34, x 200 45 : 44, x 264 48 : 48, x 328 52 :
+// 54, x 65 35 : 38; more: 5,000 x 72 37 : 37, 6,144 x 72 37 : 46, 5,000 x 50
+// 33 : 33;
+// two, an eighth: 2,100 x 77 26 : 22, x 130 29 : 28, x 250 32 : 34; 8 divides:
+// x 72 26 : 20, x 712 54 : 54, x 968 66 : 68; up to half: 2,400 x 77 26 : 26, x
+// 130 30 : 32, x 200 32 : 30, x 328 38 : 37, x 392 40 : 41; more: 4,096 x 65
+// 30 : 31, x 200 38 : 35, x 264 39 : 39, x 328 42 : 43;
+// one: 1,000 x 200 20 : 15, x 255 20 : 21, x 500 25 : 30.
 static bool pad_pays(const ltx_ctx* c, int lq, int lkv) {
-    const int nt = (lkv + 63) / 64, rounds = ((lq + 255) / 256 * LTX_H + c->num_cu - 1) / c->num_cu;
+    const int nt = (lkv + 63) / 64, wgs = (lq + 255) / 256 * LTX_H;
+    const int rounds = (wgs + c->num_cu - 1) / c->num_cu, last = wgs - (rounds - 1) * c->num_cu;
+    const bool few = last <= c->num_cu / 8, v8 = lkv % 8 == 0;
     if (rounds >= 4) return true;
-    if (rounds >= 2) return nt >= 2;
-    return nt >= (lkv % 8 == 0 ? 28 : 5);
+    if (rounds == 3) return nt >= (v8 && few ? 5 : 2);
+    if (rounds == 2) return nt >= (v8 ? few ? 13 : last <= c->num_cu / 2 ? 6 : 5 : few ? 4 : 2);
+    return nt >= (v8 ? 28 : 5);
 }
 
 // Whether the streaming attention takes 128-query workgroups: where they fit the

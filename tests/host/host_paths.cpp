@@ -220,7 +220,14 @@ int main(int argc, char** argv) {
         scratch_memory();
     else if (cmd == "planes_bound")
         planes_bound(arg(2), arg(3), arg(4), false);
-    else
+    else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv
+        ltx_ctx* c = make_ctx();
+        for (int i = 2; i + 1 < argc; i += 2) {
+            fake::log.clear();
+            CHECK(attention(c, arg(i), arg(i + 1), nullptr), "%s", ltx_last_error(c));
+            std::printf("%d ", launches("ltx_vt_pad"));
+        }
+    } else
         CHECK(false, "unknown command %s", cmd.c_str());
     std::printf("ok\n");
     std::fflush(stdout);

@@ -55,6 +55,17 @@ def test_f32_linear_planes_are_bounded(host_paths, M, N, K):
     host_paths("planes_bound", M, N, K)
 
 
+def test_attention_pads_where_it_pays(host_paths):
+    """(queries, keys) on both sides of each line of the padding rule: the calls
+    measured faster on the any-length kernel stay on it."""
+    any_length = [(200, 16), (1000, 255), (2048, 264), (2049, 72), (2100, 77), (2100, 130), (2304, 712), (2305, 264),
+                  (2500, 200), (3000, 50), (3000, 264), (4000, 200), (4096, 63), (4097, 200), (4200, 72), (5000, 50)]
+    padded = [(200, 300), (1025, 450), (2100, 250), (2304, 776), (2305, 65), (2500, 328), (3000, 130), (3500, 264),
+              (4096, 264), (4097, 65), (4200, 264), (4353, 72), (5000, 200), (6145, 1), (8200, 16)]
+    out = host_paths("attn_padded", *(n for pair in any_length + padded for n in pair)).split()[:-1]
+    assert [p for p, o in zip(any_length + padded, out) if (o == "1") != (p in padded)] == []
+
+
 def test_gate_logits_fit_beside_the_16_bit_gemm(tmp_path):
     """The gate logits run on the second stream beside the 16-bit-weight GEMM
     (unquantised blocks up to 2,048 tokens): a workgroup of theirs has to fit
