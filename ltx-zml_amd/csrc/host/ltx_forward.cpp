@@ -54,16 +54,25 @@ static int gemm_ksplit(int num_cu, int M, int N, int K, int tn = 256, int tm = 2
 
 // Rows of a persistent GEMM's 256-column tiles, 256 or 192: the height whose
 // whole rounds of one tile a CU are the fewest rows, a row of the lower tiles
-// counted 1.05 times (they read more LDS and move more operand bytes per MFMA).
+// counted 1.08 times, past K = 4,096 1.2 times (they read more LDS, move more
+// operand bytes and dequantise more weights per MFMA).
 // Measured, 192 against 256 rows, us (rows x N x K, the dequantisation
-// included): 4,100 x 4,096 x 4,096 147 : 182, 2,970 x 12,288 x 4,096 271 : 303,
-// 1,600 x 12,288 x 4,096 164 : 192, 4,100 x 4,096 x 16,384 588 : 685; where the
-// rule stays at 256: 4,095 x 4,096 x 4,096 150 : 120, 8,000 x 4,096 x 4,096 229
-// : 211, 2,048 x 16,384 x 4,096 254 : 231. Tiles of 128 rows lost everywhere.
-static int tile_rows(const ltx_ctx* c, int M, int N) {
+// included; rounds of each):
+// equal rounds 4,100 x 4,096 x 4,096 151 : 187, 2,970 x 12,288 x 4,096 284 :
+// 313, 1,600 x 12,288 x 4,096 170 : 193, 4,100 x 4,096 x 16,384 604 : 683, 9,216
+// x 4,096 x 16,384 1,131 : 1,246;
+// six to five 5,400 x 12,288 x 4,096 458 : 483, 18,432 x 4,096 x 4,096 462 :
+// 470, 17,000 x 4,096 x 16,384 2,176 : 2,009; eleven to nine 16,500 x 8,192 x
+// 4,096 834 : 855; five to four 4,100 x 12,288 x 4,096 383 : 390, 15,360 x 4,096
+// x 4,096 388 : 384, 3,500 x 16,384 x 4,096 434 : 421, 13,000 x 4,096 x 16,384
+// 1,822 : 1,632; fifteen to twelve 15,000 x 12,288 x 4,096 1,165 : 1,156;
+// one round of the W8A16 kernel with f32 scales 2,100 x 4,096 x 4,096 82 : 86,
+// 2,500 94 : 91, yet in a block, between other kernels, the lower tiles win there
+// (bf16, 2,304 tokens 1,308 : 1,356, 2,500 tokens 1,424 : 1,438).
+static int tile_rows(const ltx_ctx* c, int M, int N, int K) {
     if (c->gemm_rows == 192 || c->gemm_rows == 256) return c->gemm_rows;
     auto rounds = [&](int rows) { return (((M + rows - 1) / rows) * (N / 256) + c->num_cu - 1) / c->num_cu; };
-    return rounds(192) * 192 * 1.05f < rounds(256) * 256 ? 192 : 256;
+    return rounds(192) * 192 * (K <= 4096 ? 1.08f : 1.2f) < rounds(256) * 256 ? 192 : 256;
 }
 
 bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool w16) {
@@ -306,7 +315,7 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
             g.ksplit = 1;
             std::snprintf(name, sizeof(name), "ltx_gemm_x4_%s_%s%s%s", msuffix(mode), es,
                           epi == LTX_EPI_STORE && g.out_f32 ? "32" : "", epi == LTX_EPI_STORE && g.gelu ? "_gelu" : "");
-            const int tr = tile_rows(c, M, p.N);
+            const int tr = tile_rows(c, M, p.N, p.K);
             if (tr != 256) std::snprintf(name + std::strlen(name), sizeof(name) - std::strlen(name), "_h%d", tr);
             g.tiles_m = (M + tr - 1) / tr;
             const int nitems = g.tiles_m * g.tiles_n;
@@ -350,7 +359,7 @@ static void gemm16(ltx_ctx* c, int mode, const LtxProj& p, const void* A, int M,
         // few output tiles: split K over more workgroups (when the caller
         // gave a buffer for the partial sums), then reduce + epilogue
         g.ksplit = g.part ? gemm_ksplit(c->num_cu, M, p.N, p.K) : 1;
-        const int tr = g.ksplit > 1 ? 256 : tile_rows(c, M, p.N);
+        const int tr = g.ksplit > 1 ? 256 : tile_rows(c, M, p.N, p.K);
         if (tr != 256) std::snprintf(name + std::strlen(name), sizeof(name) - std::strlen(name), "_h%d", tr);
         g.tiles_m = (M + tr - 1) / tr;
         const int nitems = g.tiles_m * g.tiles_n * g.ksplit;
@@ -780,7 +789,8 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         qknorm16(c, mode, b.k2_16, LTX_D, w->kn2.p, nullptr, nullptr, b.kh2, S, 1.0f, sd);
     };
     if (early) {
-        const int tr = tile_rows(c, T, 3 * LTX_D), last = (T + tr - 1) / tr * (3 * LTX_D / 256) % c->num_cu;
+        const int tr = tile_rows(c, T, 3 * LTX_D, LTX_D);
+        const int last = (T + tr - 1) / tr * (3 * LTX_D / 256) % c->num_cu;
         const bool w16 = !w->qkv1.q8 && !x4_shape(c, mode, T, 3 * LTX_D, LTX_D, LTX_D, true);  // 256 x 128 tiles
         side_gates = w16 || (last > 0 && last <= c->num_cu - c->num_cu / 8);
         if (!side_gates) {

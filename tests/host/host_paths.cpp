@@ -81,9 +81,9 @@ static void f32_planes(int T, int S) {
     std::printf("%d splits\n", splits);
 }
 
-static bool linear(ltx_ctx* c, int M, int N, int K, int mode, hipStream_t st, bool noalloc = false, size_t off = 0) {
+static bool linear(ltx_ctx* c, int M, int N, int K, int mode, hipStream_t st, bool noalloc = false, int scale_f16 = 1) {
     auto f = noalloc ? ltx_op_linear_q8_noalloc : ltx_op_linear_q8;
-    return f(c, ptr(0), (const int8_t*)ptr(1) + off, ptr(2), 1, nullptr, ptr(3), mode == LTX_MODE_F32, M, N, K, 0, mode,
+    return f(c, ptr(0), (const int8_t*)ptr(1), ptr(2), scale_f16, nullptr, ptr(3), mode == LTX_MODE_F32, M, N, K, 0, mode,
              st);
 }
 static bool attention(ltx_ctx* c, int lq, int lkv, hipStream_t st) {
@@ -226,6 +226,16 @@ int main(int argc, char** argv) {
             fake::log.clear();
             CHECK(attention(c, arg(i), arg(i + 1), nullptr), "%s", ltx_last_error(c));
             std::printf("%d ", launches("ltx_vt_pad"));
+        }
+    } else if (cmd == "tile_rows") {  // prints whether tiles of 192 rows run, for quadruples M N K scale_f16
+        ltx_ctx* c = make_ctx();
+        for (int i = 2; i + 3 < argc; i += 4) {
+            fake::log.clear();
+            CHECK(linear(c, arg(i), arg(i + 1), arg(i + 2), LTX_MODE_BF16, nullptr, false, arg(i + 3)), "%s",
+                  ltx_last_error(c));
+            int h = 0;
+            for (const fake::Op& o : fake::log) h += o.name.find("_h192") != std::string::npos;
+            std::printf("%d ", h);
         }
     } else
         CHECK(false, "unknown command %s", cmd.c_str());

@@ -66,6 +66,18 @@ def test_attention_pads_where_it_pays(host_paths):
     assert [p for p, o in zip(any_length + padded, out) if (o == "1") != (p in padded)] == []
 
 
+def test_gemm_tile_heights(host_paths):
+    """(M, N, K, f16 scales) on both sides of each line of the rule for tiles of
+    192 rows: the calls measured faster on 256 rows stay there."""
+    r256 = [(3500, 16384, 4096, 0), (3500, 16384, 4096, 1), (15360, 4096, 4096, 1), (13000, 4096, 16384, 1),
+            (17000, 4096, 16384, 0), (21000, 4096, 16384, 0), (15000, 12288, 4096, 1), (28672, 4096, 4096, 1),
+            (4095, 4096, 4096, 1), (2970, 16384, 4096, 0)]
+    r192 = [(4100, 4096, 4096, 0), (9216, 4096, 16384, 1), (2970, 12288, 4096, 0), (5400, 12288, 4096, 1),
+            (16500, 8192, 4096, 1), (18432, 4096, 4096, 0), (2100, 4096, 4096, 0), (2500, 4096, 4096, 0)]
+    out = host_paths("tile_rows", *(n for shape in r256 + r192 for n in shape)).split()[:-1]
+    assert [s for s, o in zip(r256 + r192, out) if (o == "1") != (s in r192)] == []
+
+
 def test_gate_logits_fit_beside_the_16_bit_gemm(tmp_path):
     """The gate logits run on the second stream beside the 16-bit-weight GEMM
     (unquantised blocks up to 2,048 tokens): a workgroup of theirs has to fit
