@@ -226,18 +226,21 @@ int ltx_op_linear_q8(ltx_ctx* ctx, const void* a, const int8_t* q, const void* s
 /* No counterpart in the reference. For callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc): ltx_op_linear_q8 with the same arguments and results,
- * calling no hipMalloc / hipFree. Its scratch (room for the weights as bytes
- * q + 128, N * K bytes rounded up to 256, then the scale words, 4 N K / 128
- * bytes, and for the shapes ltx_op_linear_q8 runs on the four-wave GEMM, from
- * 4,096 rows, the weights dequantised to the operand type, 2 N K bytes; split-K
- * partial sums take the place of the bytes q + 128, and mode F32 runs the planes
- * of as many rows at a time as fit) is
- * a static device array of LTX_NOALLOC_SCRATCH_BYTES on each GPU the library
- * runs on, held until the process ends; a shape needing more is refused with
- * an error. The kernels write all of the scratch they read on each call, so
- * nothing carries over between calls, but every call on one GPU shares the
- * array: calls that overlap on one GPU (other streams, contexts or threads)
- * race. */
+ * calling no hipMalloc / hipFree. Its scratch is static device arrays of
+ * LTX_NOALLOC_SCRATCH_BYTES on each GPU the library runs on, held until the
+ * process ends; a shape needing more is refused with an error. The kernels write
+ * all of the scratch they read on each call, so nothing carries over between
+ * calls.
+ * The 16-bit modes use one array: room for the weights as bytes q + 128 (N * K
+ * bytes rounded up to 256; split-K partial sums may take their place), then the
+ * scale words, 4 N K / 128 bytes, and for the shapes ltx_op_linear_q8 runs on
+ * the four-wave GEMM, from 4,096 rows, the weights dequantised to the operand
+ * type, 2 N K bytes. Every such call on one GPU shares it: calls that overlap on
+ * one GPU (other streams, contexts or threads) race.
+ * Mode F32 has an array of its own for the planes and partial sums of as many
+ * rows at a time as fit. Its calls may overlap any others: they are ordered
+ * behind each other's use of the array, and a call being captured uses none (the
+ * f32 MFMA kernel, as in ltx_op_linear_q8). */
 #define LTX_NOALLOC_SCRATCH_BYTES (66u << 20)
 int ltx_op_linear_q8_noalloc(ltx_ctx* ctx, const void* a, const int8_t* q, const void* scales, int scale_f16,
                              const float* bias, void* y, int out_f32, int M, int N, int K, int gelu, int mode,

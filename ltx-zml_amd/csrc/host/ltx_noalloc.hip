@@ -20,11 +20,50 @@
 #include "ltx_internal.hpp"
 
 static __device__ __align__(256) unsigned char scratch[LTX_NOALLOC_SCRATCH_BYTES];
+// Mode F32's planes and partial sums, an array of their own: its calls use none
+// of the above and may overlap calls that do.
+static __device__ __align__(256) unsigned char planes[LTX_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
-void* g_scratch[kMaxDevices] = {};
+struct Device {
+    void* scratch = nullptr;
+    void* planes = nullptr;
+    // the last use of planes: calls of every context and thread follow each other
+    std::mutex mu;
+    hipEvent_t ev = nullptr;
+    bool used = false;
+} g_dev[kMaxDevices];
+
+// One call's use of the planes, ordered behind the last one and recorded when
+// the scope ends. Not for a call that is being captured: nothing here could
+// order its replays.
+struct PlanesUse {
+    Device* d = nullptr;
+    std::unique_lock<std::mutex> lk;
+    hipStream_t st;
+    explicit PlanesUse(hipStream_t stream) : st(stream) {}
+    void* take(Device& dev) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (cap != hipStreamCaptureStatusNone) return nullptr;
+        lk = std::unique_lock<std::mutex>(dev.mu);
+        if (dev.used) HIPC(hipStreamWaitEvent(st, dev.ev, 0));
+        d = &dev;
+        return dev.planes;
+    }
+    ~PlanesUse() {
+        if (!d) return;
+        if (hipEventRecord(d->ev, st) == hipSuccess)
+            d->used = true;
+        else
+            (void)hipStreamSynchronize(st);  // nothing to wait for later
+    }
+};
 }  // namespace
 
 namespace ltx {
@@ -32,16 +71,20 @@ namespace ltx {
 void noalloc_setup(int device) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (device < 0 || device >= kMaxDevices) throw Error("noalloc: device index beyond the supported 64");
-    if (g_scratch[device]) return;
-    void* p = nullptr;
+    Device& d = g_dev[device];
+    if (d.ev) return;
+    void *p = nullptr, *q = nullptr;
     HIPC(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    if (!p) throw Error("noalloc: hipGetSymbolAddress returned no address for the scratch array");
-    g_scratch[device] = p;
+    HIPC(hipGetSymbolAddress(&q, HIP_SYMBOL(planes)));
+    if (!p || !q) throw Error("noalloc: hipGetSymbolAddress returned no address for the scratch array");
+    HIPC(hipEventCreateWithFlags(&d.ev, hipEventDisableTiming));
+    d.scratch = p;
+    d.planes = q;
 }
 
 void* noalloc_scratch(int device) {
     std::lock_guard<std::mutex> lk(g_mu);
-    return device >= 0 && device < kMaxDevices ? g_scratch[device] : nullptr;
+    return device >= 0 && device < kMaxDevices ? g_dev[device].scratch : nullptr;
 }
 
 }  // namespace ltx
@@ -73,21 +116,19 @@ extern "C" int ltx_op_linear_q8_noalloc(ltx_ctx* c, const void* a, const int8_t*
             sc.w16 = nw ? base + nq + np : nullptr;
         }
         char* base = (char*)ltx::noalloc_scratch(c->device);
+        HIPC(hipSetDevice(c->device));
+        PlanesUse use((hipStream_t)stream);
         if (mode == LTX_MODE_F32 && ltx::f3_shape(c, M, N, K)) {
             // the planes of as many rows of A as fit, with their partial sums;
             // at least 128: a split has at most 256 tiles x slices of 64 KB,
             // and K is at most 32,768
-            const size_t part = ltx::f3_part_bytes(c, M, N, K);
-            int rows = M;
-            while (rows > 128 && ltx::f3_planes_bytes(rows, K) + (part ? part / M * rows : 0) > LTX_NOALLOC_SCRATCH_BYTES)
-                rows = (rows / 2 + 127) / 128 * 128;
-            const size_t np = ltx::f3_planes_bytes(rows, K);
+            const int rows = ltx::f3_rows(c, M, N, K, LTX_NOALLOC_SCRATCH_BYTES);
             if (!base) throw ltx::Error("ltx_op_linear_q8_noalloc: scratch not set up on this device");
-            if (np + (part ? part / M * rows : 0) > LTX_NOALLOC_SCRATCH_BYTES)
-                throw ltx::Error("ltx_op_linear_q8_noalloc: scratch too small for 128 rows");  // (cannot happen)
-            sc.planes = base;
-            sc.plane_rows = rows;
-            sc.part = part ? base + np : nullptr;
+            if (!rows) throw ltx::Error("ltx_op_linear_q8_noalloc: scratch too small for 128 rows");  // (cannot happen)
+            if ((sc.planes = use.take(g_dev[c->device]))) {
+                sc.plane_rows = rows;
+                sc.part = ltx::f3_part_bytes(c, M, N, K) ? (char*)sc.planes + ltx::f3_planes_bytes(rows, K) : nullptr;
+            }
         }
         if (const size_t part = ltx::linear_packed(a, q, scales, scale_f16, bias, y, K) ? ltx::linear_part_bytes(c, M, N, K, mode) : 0) {
             // beside the scale words; the room of the bytes q + 128 is free
@@ -98,7 +139,6 @@ extern "C" int ltx_op_linear_q8_noalloc(ltx_ctx* c, const void* a, const int8_t*
             sc.pairs = (uint32_t*)base;
             sc.part = base + np;
         }
-        HIPC(hipSetDevice(c->device));
         ltx::linear_q8(c, a, q, scales, scale_f16, bias, y, out_f32, M, N, K, gelu, mode, sc, (hipStream_t)stream);
     })
 }

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "ltx_args.h"
+#include "ltx_block.h"
 
 namespace fake {
 
@@ -105,7 +106,7 @@ hipError_t hipDeviceSynchronize() {
 }
 hipError_t hipGetSymbolAddress(void** p, const void*) {
     *p = (void*)(fake::next_addr);
-    fake::mem[fake::next_addr] = 1ull << 30;
+    fake::mem[fake::next_addr] = LTX_NOALLOC_SCRATCH_BYTES;
     fake::next_addr += 1ull << 30;
     return hipSuccess;
 }

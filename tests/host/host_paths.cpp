@@ -202,6 +202,27 @@ static void planes_bound(int M, int N, int K, bool noalloc) {
     std::printf("%d passes, %zu bytes\n", launches("ltx_split3"), c->op_scratch.buf.bytes);
 }
 
+// Mode F32 without allocations: eager calls follow each other, whatever their
+// stream and context, and use none of the scratch that the 16-bit modes share;
+// a captured call, whose replays may overlap anything, uses no scratch at all.
+static void noalloc_f32() {
+    ltx_ctx *c1 = make_ctx(), *c2 = make_ctx();
+    const hipStream_t cap = (hipStream_t)0x30;
+    int i = 0;
+    scratch_order("ltx_split3", "ltx_gemm_f3_i8f16_store",
+                  [&](hipStream_t st) { return linear(i++ % 2 ? c1 : c2, 1000, 4096, 512, LTX_MODE_F32, st, true); });
+    uint64_t lo = ~0ull, hi = 0;
+    for (const fake::Op& o : fake::log)
+        if (o.name == "ltx_split3") lo = std::min(lo, (uint64_t)o.split.p0), hi = std::max(hi, (uint64_t)o.split.p2);
+    const uint64_t s = (uint64_t)ltx::noalloc_scratch(0);
+    CHECK(s && (hi < s || lo >= s + LTX_NOALLOC_SCRATCH_BYTES), "planes in the shared scratch");
+    fake::capturing.insert(cap);
+    fake::log.clear();
+    CHECK(linear(c1, 1000, 4096, 512, LTX_MODE_F32, cap, true), "%s", ltx_last_error(c1));
+    CHECK(launches("") == 1 && launches("ltx_gemm_f32") == 1, "%d launches", launches(""));
+    for (const fake::Op& o : fake::log) CHECK(o.what == "launch", "%s in a capture", o.what.c_str());
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -220,6 +241,10 @@ int main(int argc, char** argv) {
         scratch_memory();
     else if (cmd == "planes_bound")
         planes_bound(arg(2), arg(3), arg(4), false);
+    else if (cmd == "noalloc_f32")
+        noalloc_f32();
+    else if (cmd == "planes_bound_noalloc")
+        planes_bound(arg(2), arg(3), arg(4), true);
     else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv
         ltx_ctx* c = make_ctx();
         for (int i = 2; i + 1 < argc; i += 2) {

@@ -55,6 +55,16 @@ def test_f32_linear_planes_are_bounded(host_paths, M, N, K):
     host_paths("planes_bound", M, N, K)
 
 
+def test_noalloc_f32_calls_are_independent(host_paths):
+    host_paths("noalloc_f32")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (300, 256, 4096), (3000, 128, 4096), (28672, 4096, 16384),
+                                   (1000, 4096, 32768), (129, 128, 32768)])
+def test_noalloc_f32_planes_fit_the_array(host_paths, M, N, K):
+    host_paths("planes_bound_noalloc", M, N, K)
+
+
 def test_attention_pads_where_it_pays(host_paths):
     """(queries, keys) on both sides of each line of the padding rule: the calls
     measured faster on the any-length kernel stay on it."""

@@ -5,8 +5,9 @@ library's static device array, so its output must equal the allocating entry
 point's bit for bit. Two calls in a row, the second with a smaller input (so a
 stale first-call scratch would show), from a shape on the four-wave GEMM
 (weights dequantised into the scratch) down to ones on the W8A16 kernel, in
-both 16-bit modes with f16 and f32 scales; the F32 mode (no scratch); and a shape whose scratch exceeds the
-array is refused.
+both 16-bit modes with f16 and f32 scales; the F32 mode (an array of its own,
+its calls ordered behind each other); and a shape whose scratch exceeds the array
+is refused.
 """
 import numpy as np
 import pytest
@@ -59,8 +60,8 @@ def test_noalloc_equals_linear_q8(ctx, mode, scale_f16):
 
 
 def test_noalloc_without_scratch_paths(ctx):
-    """F32 mode uses no scratch; its results still equal the allocating
-    entry point's. A shape both entry points refuse (N not a multiple of 256
+    """F32 mode uses none of the shared scratch; its results still equal the
+    allocating entry point's. A shape both entry points refuse (N not a multiple of 256
     in a 16-bit mode) is refused by both with the same error."""
     M, N, K = 130, 384, 1024
     say(f"linear_q8_noalloc without scratch mode=f32 M={M} N={N} K={K}")
@@ -113,3 +114,36 @@ def test_noalloc_split_and_planes(ctx, mode, M, N, K, scale_f16):
     y0, y1 = _both(ctx, mode, M, N, K, 3, scale_f16, False, mode == rt.MODE_F32)
     assert torch.isfinite(y0).all().item()
     assert torch.equal(y0, y1)
+
+
+def test_noalloc_f32_overlapping_calls(ctx):
+    """Mode F32 calls of two contexts on two streams, and one captured between
+    them: each gives what it gives alone."""
+    M, N, K = 1000, 4096, 1024
+    say(f"linear_q8_noalloc f32 overlapping M={M} N={N} K={K}")
+    other = rt.Context(0)
+    try:
+        args, alone, ys = [], [], []
+        for i in range(2):
+            a, q, s, b = _case(M, N, K, 20 + i, 1)
+            args.append([torch.from_numpy(x).cuda() for x in (a, q, s, b)])
+            alone.append(torch.empty((M, N), device="cuda"))
+            ys.append(torch.empty_like(alone[0]))
+            ctx.linear_q8(*args[i], alone[i], mode=rt.MODE_F32)
+        cap, graph = torch.empty_like(ys[0]), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            ctx.linear_q8(*args[0], cap, mode=rt.MODE_F32, noalloc=True)
+        streams = [torch.cuda.Stream() for _ in range(3)]
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for c, st, x, y in zip((ctx, other), streams, args, ys):
+                c.linear_q8(*x, y, mode=rt.MODE_F32, noalloc=True, stream=st)
+            with torch.cuda.stream(streams[2]):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, w) for y, w in zip(ys, alone))
+        # two kernels: each rounds K / 4 = 256 running sums to f32, as a random
+        # walk 2^-24 sqrt(256) = 1e-6 of the result
+        assert ((cap - alone[0]).norm() / alone[0].norm()).item() <= 1e-6
+    finally:
+        other.close()
