@@ -28,6 +28,14 @@
 // step before the one that uses them. A group's partial sums are folded into
 // the accumulators between the first 16 MFMAs of the next group, which restart
 // them from zero.
+//
+// A group's sum of a q may leave f32's range (from |a| = 2^114 on) where y does
+// not. A tile with a sum that is not finite is therefore formed once more with
+// the int8 weights times 2^-14 and the scales times 2^14 (exact): the range is
+// that of A and y, and an infinity or NaN in A stays one. Doing so always cost
+// 8 % (one subtraction for two weights: the VALU has no room beside these
+// MFMAs). At the other end the lowest plane ends at bf16's smallest subnormal:
+// values keep all of their bits from 2^-110 on.
 #pragma once
 #include "gemm_s4.h"
 
@@ -35,6 +43,7 @@ __shared__ __attribute__((aligned(1024))) uint8_t f3q_st0[57344];
 __shared__ __attribute__((aligned(1024))) uint8_t f3q_st1[57344];
 __shared__ __attribute__((aligned(1024))) uint8_t f3w_st0[65536];
 __shared__ __attribute__((aligned(1024))) uint8_t f3w_st1[65536];
+__shared__ int f3_redo;  // 1 + the tile (and slice) to form once more
 
 template <bool Q, int S>
 __device__ __forceinline__ uint8_t* f3_stage() {
@@ -91,7 +100,10 @@ struct F3Gemm {
         return *(const u32x4*)(f3_stage<Q, S>() + offa[STEP] + 16384 * (i >> 2) + 2048 * (i & 3));
     }
 
-    // 8 weights as a bf16 operand: an int8 is exact in the upper half of its f32
+    // 8 weights as a bf16 operand: an int8 is exact in the upper half of its f32.
+    // X: times 2^-14, 14 off the exponents of a pair (a zero's stays zero: the
+    // subtraction saturates).
+    template <bool X>
     __device__ __forceinline__ bf16x8 operand(const WF& w) {
         if constexpr (Q) {
             u32x4 o;
@@ -101,8 +113,13 @@ struct F3Gemm {
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const float lo = (float)(int8_t)(x >> (16 * e)), hi = (float)(int8_t)(x >> (16 * e + 8));
-                    o[2 * d + e] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi),
-                                                         __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+                    uint32_t b = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, hi),
+                                                       __builtin_bit_cast(uint32_t, lo), 0x07060302u);
+                    if (X) {
+                        const u16x2 m = __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, b), (u16x2)(14 << 7));
+                        b = __builtin_bit_cast(uint32_t, m);
+                    }
+                    o[2 * d + e] = b;
                 }
             }
             return __builtin_bit_cast(bf16x8, o);
@@ -111,6 +128,7 @@ struct F3Gemm {
         }
     }
 
+    template <bool X>
     __device__ __forceinline__ void load_scales(int g) {
         if constexpr (Q) {
             const size_t G = a.K / LTX_GROUP;
@@ -120,6 +138,7 @@ struct F3Gemm {
                     s[j] = f16_bits_to_f32(((const uint16_t*)sc)[16 * j * G + g]);
                 else
                     s[j] = ((const float*)sc)[16 * j * G + g];
+                if (X) s[j] *= 16384.0f;
             }
         }
     }
@@ -146,7 +165,7 @@ struct F3Gemm {
     // One step's 48 MFMAs (xa, xb), with the 16 fragment reads of step STEP of
     // stage RS (W first), the conversion of its W fragments, and, when DMA,
     // the DMA of tile kd into stage DS.
-    template <int RS, int STEP, int DS, bool DMA, bool FIRST>
+    template <int RS, int STEP, int DS, bool DMA, bool FIRST, bool X>
     __device__ __forceinline__ void region(const u32x4 (&xa)[12], const bf16x8 (&xb)[4], u32x4 (&ya)[12],
                                            bf16x8 (&yb)[4], int kd) {
         WF yw[4];
@@ -163,7 +182,7 @@ struct F3Gemm {
                 if (DMA && g < 12 + NDB) dma1<DS>(g, kd);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (m >= 24 && (m - 24) % 6 == 0) yb[(m - 24) / 6] = operand(yw[(m - 24) / 6]);
+            if (m >= 24 && (m - 24) % 6 == 0) yb[(m - 24) / 6] = operand<X>(yw[(m - 24) / 6]);
         }
     }
 
@@ -178,13 +197,52 @@ struct F3Gemm {
     // Entered after a barrier: tile k in stage S (k % 2) with its step-1
     // fragments in fa1/fb1, tile k + 1 landed in the other stage, no DMA
     // pending, stage S read by every wave. A group is tiles k, k + 1 of an even k.
-    template <int S, bool DMA>
+    template <int S, bool DMA, bool X>
     __device__ __forceinline__ void pair(int k) {
-        if (S == 0) load_scales(k >> 1);
-        region<S ^ 1, 0, S, DMA, false>(fa1, fb1, fa0, fb0, k + 2);
+        if (S == 0) load_scales<X>(k >> 1);
+        region<S ^ 1, 0, S, DMA, false, X>(fa1, fb1, fa0, fb0, k + 2);
         __builtin_amdgcn_sched_barrier(0);
-        region<S ^ 1, 1, S, false, S == 1>(fa0, fb0, fa1, fb1, 0);
+        region<S ^ 1, 1, S, false, S == 1, X>(fa0, fb0, fa1, fb1, 0);
         meet();
+    }
+
+    // acc = A . W^T of the tile over nk K-tiles (the stages free on entry; the
+    // last tile's reads are not waited for)
+    template <bool X>
+    __device__ __forceinline__ void product(int nk) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0, 0, 0, 0};
+        dma<0>(0);
+        __builtin_amdgcn_s_waitcnt(Q8_WAIT_VM(0));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        dma<1>(1);
+        {
+            WF w0[4], w1[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) w0[j] = read_w<0, 0>(j), w1[j] = read_w<0, 1>(j);
+#pragma unroll
+            for (int i = 0; i < 12; i++) fa0[i] = read_a<0, 0>(i), fa1[i] = read_a<0, 1>(i);
+#pragma unroll
+            for (int j = 0; j < 4; j++) fb0[j] = operand<X>(w0[j]), fb1[j] = operand<X>(w1[j]);
+        }
+#pragma unroll
+        for (int m = 0; m < 48; m++) mfma1<true, false>(m, fa0, fb0);  // tile 0, step 0
+        meet();
+        for (int k = 0; k < nk - 2; k += 2) {
+            pair<0, true, X>(k);
+            pair<1, true, X>(k + 1);
+        }
+        pair<0, false, X>(nk - 2);
+#pragma unroll
+        for (int m = 0; m < 48; m++) mfma1<false, false>(m, fa1, fb1);  // tile nk - 1, step 1
+        if constexpr (Q)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) fold(i, j);
     }
 
     __device__ __forceinline__ void run(const LtxGemmF3Args& args) {
@@ -218,6 +276,7 @@ struct F3Gemm {
         // epilogue patches (32 rows of 72 floats, 9 KB): two waves in each stage
         uint8_t* patch = (w & 1 ? f3_stage<Q, 1>() : f3_stage<Q, 0>()) + 16384 * (w >> 1);
         const int nitems = a.tiles_m * a.tiles_n * ks_n;
+        if (Q && tid == 0) f3_redo = 0;  // (before the first tile's barriers)
         for (int item = blockIdx.x; item < nitems; item += gridDim.x) {
             const int ks = item % ks_n;
             const TileIdx ti = tile_of(item / ks_n, a.tiles_m, a.tiles_n);
@@ -241,40 +300,29 @@ struct F3Gemm {
                 const size_t so = (size_t)(n0 + wn + (lane & 15)) * (a.K / LTX_GROUP) + k0 / LTX_GROUP;
                 sc = (const char*)a.scales + so * (BK == LTX_B_I8_F16S ? 2 : 4);
             }
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0, 0, 0, 0};
-            dma<0>(0);
-            __builtin_amdgcn_s_waitcnt(Q8_WAIT_VM(0));
-            __builtin_amdgcn_s_barrier();
-            __builtin_amdgcn_sched_barrier(0);
-            dma<1>(1);
-            {
-                WF w0[4], w1[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) w0[j] = read_w<0, 0>(j), w1[j] = read_w<0, 1>(j);
-#pragma unroll
-                for (int i = 0; i < 12; i++) fa0[i] = read_a<0, 0>(i), fa1[i] = read_a<0, 1>(i);
-#pragma unroll
-                for (int j = 0; j < 4; j++) fb0[j] = operand(w0[j]), fb1[j] = operand(w1[j]);
-            }
-#pragma unroll
-            for (int m = 0; m < 48; m++) mfma1<true, false>(m, fa0, fb0);  // tile 0, step 0
-            meet();
-            for (int k = 0; k < nk - 2; k += 2) {
-                pair<0, true>(k);
-                pair<1, true>(k + 1);
-            }
-            pair<0, false>(nk - 2);
-#pragma unroll
-            for (int m = 0; m < 48; m++) mfma1<false, false>(m, fa1, fb1);  // tile nk - 1, step 1
-            if constexpr (Q)
+            product<false>(nk);
+            if constexpr (Q) {
+                float mx = 0.f;  // NaN wins over everything
 #pragma unroll
                 for (int i = 0; i < 4; i++)
 #pragma unroll
-                    for (int j = 0; j < 4; j++) fold(i, j);
+                    for (int j = 0; j < 4; j++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            mx = __builtin_elementwise_maximum(mx, __builtin_fabsf(acc[i][j][e]));
+                if (!(mx <= 3.402823466e38f)) f3_redo = item + 1;
+                // (the barrier alone does not keep the compiler from answering the
+                // read below with this wave's own store)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            }
             meet();
+            if constexpr (Q) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+                if (__builtin_amdgcn_readfirstlane(f3_redo) == item + 1) {  // the same in every wave
+                    product<true>(nk);
+                    meet();
+                }
+            }
             // every wave has passed the last barrier: the stages are free
             const int el = opaque_tid() & 63;
             auto fill = [&](int b, float* p, int LD) {

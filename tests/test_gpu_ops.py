@@ -375,6 +375,28 @@ def test_linear_q8_f32_planes_nonfinite_and_streams(ctx):
         assert torch.equal(o, w)
 
 
+@pytest.mark.parametrize("M,scale_f16", [(200, True), (130, False)])
+def test_linear_q8_f32_planes_range(ctx, M, scale_f16):
+    """Values of A up to the largest floats: a group's sum of a q passes f32's
+    range long before y does. And down to 2^-110, below which the lowest plane's
+    bits fall under bf16's smallest subnormal, 2^-133."""
+    say(f"linear_q8 f32 planes range M={M} scale_f16={scale_f16}")
+    N, K = 256, 512
+    a, q, s, _ = _gemm_case(M, N, K, seed=11, scale_f16=scale_f16)
+    a /= np.abs(a).max()
+    a = a.astype(np.float64) * 2.0 ** np.linspace(-106, 126.5, M)[:, None]
+    a = a.astype(np.float32)
+    y = torch.full((M, N), float("nan"), dtype=torch.float32, device="cuda")
+    ctx.linear_q8(torch.from_numpy(a).cuda(), torch.from_numpy(q).cuda(), torch.from_numpy(s).cuda(), None, y,
+                  mode=rt.MODE_F32)
+    torch.cuda.synchronize()
+    want = a.astype(np.float64) @ oracle.dequant(q, s).astype(np.float64).T
+    assert np.abs(want).max() < 3e38
+    row = 2.0 ** -np.linspace(-106, 126.5, M)[:, None]  # each row by itself
+    # as test_linear_q8_f32_mode
+    assert oracle.rel_rms(f64(y) * row, want * row) <= 1e-6
+
+
 def test_linear_q8_f32_planes_in_passes(ctx):
     """6,000 rows of K = 16,384 exceed the planes' 512 MiB: two passes, the bits
     of two calls of one pass each (no split of K in either)."""
