@@ -154,7 +154,10 @@ void ltx_block_graph_destroy(ltx_block_graph* g);
  * (the staged methods of ltx/block.zig:248-338), and the velocity of the last
  * ltx_denoise step (ltx/e2e_denoise.zig:314 gates it per step). Device
  * pointer + bytes, valid until the next forward on this context; a stage the
- * last call did not produce reads NULL / 0. */
+ * last call did not produce reads NULL / 0. The address stays the same while the
+ * token counts and the mode do. LTX_ST_V1 and LTX_ST_V2 in the 16-bit modes, T or
+ * S no multiple of 64: a context's first question waits for the forward (later
+ * forwards, and any captured one, form them as they run). */
 enum {
     LTX_ST_NORM_MSA,    /* s1NormMsa: modulated norm, operand dtype [T][4096] */
     LTX_ST_Q1,          /* normed+roped q times log2(e)/sqrt(128), [T][4096] (f32 mode: unscaled) */

@@ -34,6 +34,7 @@ struct Carve {
 struct Ws16 {
     void *n_msa, *qk16, *vt1, *qh1, *kh1, *glog1, *o1, *x_sa, *attn_in, *q2_16, *glog2, *enc, *k2_16, *vt2, *qh2,
         *kh2, *o2, *x_ca, *ff_in, *h, *part, *part2;
+    void *v1, *v2;  // the stages of V: V^T's rows without padding (vt1, vt2 themselves where they have none)
     void* dq[6];  // 16-bit weights of qkv1, o1, q2, o2, ff1, ff2 for the four-wave GEMM (NULL: not used)
 };
 
@@ -152,6 +153,7 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
     w.n_msa = c.take(T * D * 2);
     w.qk16 = c.take(T * 2 * D * 2);
     w.vt1 = c.take((size_t)vt_ld(T) * D * 2);
+    w.v1 = (size_t)vt_ld(T) != T ? c.take(T * D * 2) : w.vt1;
     w.qh1 = c.take(T * D * 2);
     w.kh1 = c.take(T * D * 2);
     w.glog1 = c.take(T * LTX_H * 4);
@@ -163,6 +165,7 @@ static void carve16(Carve& c, Ws16& w, size_t T, size_t S, const ltx_ctx* ctx, i
     w.enc = c.take(S * D * 2);
     w.k2_16 = c.take(S * D * 2);
     w.vt2 = c.take((size_t)vt_ld(S) * D * 2);
+    w.v2 = (size_t)vt_ld(S) != S ? c.take(S * D * 2) : w.vt2;
     w.qh2 = c.take(T * D * 2);
     w.kh2 = c.take(S * D * 2);
     w.o2 = c.take(T * D * 2);
@@ -642,19 +645,24 @@ static void stream_after(hipStream_t to, hipStream_t from, hipEvent_t e) {
     HIPC(hipStreamWaitEvent(to, e, 0));
 }
 
-// vld: V^T's row stride (ltx_block_stage hands out its rows without the padding)
-static void set_stage(ltx_ctx* c, int id, void* p, size_t bytes, int vld = 0) {
+static void set_stage(ltx_ctx* c, int id, void* p, size_t bytes) {
     c->stage_ptr[id] = p;
     c->stage_bytes[id] = bytes;
-    if (id == LTX_ST_V1) c->stage_vld[0] = vld;
-    if (id == LTX_ST_V2) c->stage_vld[1] = vld;
+}
+
+// Fills stage V1 (i = 0) or V2 (1) of the last forward, if it has padded rows.
+void fill_stage_v(ltx_ctx* c, int i, hipStream_t st) {
+    const StageV& s = c->stage_v;
+    if (!s.vt[i]) return;
+    LtxVtPadArgs a{(const uint16_t*)s.vt[i], (uint16_t*)s.v[i], s.n[i], vt_ld(s.n[i])};
+    c->launch("ltx_vt_unpad", (s.n[i] + 511) / 512, LTX_D / 4, 1, 256, &a, st);
 }
 
 // ---- the block ------------------------------------------------------------
 
 void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const float* tstab, int K,
                    const int32_t* tidx, const float* ctxv, int S, const float* pts2, const float* cs, const float* sn,
-                   int T, float* y, int mode, hipStream_t st) {
+                   int T, float* y, int mode, hipStream_t st, bool own_graph) {
     if (!w) throw Error("NULL weights");
     if (T <= 0 || S <= 0 || K <= 0) throw Error("T, S and K must be positive");
     if (!x || !tstab || !tidx || !ctxv || !pts2 || !cs || !sn || !y) throw Error("NULL tensor argument");
@@ -663,6 +671,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     HIPC(hipSetDevice(c->device));
     ensure_ws(c, (size_t)T, (size_t)S, mode);
     std::memset(c->stage_ptr, 0, sizeof(c->stage_ptr));
+    c->stage_v = StageV{};
     const size_t TD = (size_t)T * LTX_D, SD = (size_t)S * LTX_D;
     LtxAda ada = make_ada(w, tstab, tidx, K);
     Carve cv{(char*)c->ws.p, 0, 0, false};
@@ -752,6 +761,15 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
                 throw Error("injected failure inside a graph capture, after the second stream joined it [LTX_FAIL_CAPTURE]");
         }
     };
+    // The stages of V at ragged token counts (StageV), where this forward fills
+    // them, on the second stream: V1 started just behind the attention, whose
+    // workgroups leave registers for it (2,970 tokens: 5 us of 1,660; ahead of the
+    // q and k norms 9), or where that stream forks again anyway, behind the second
+    // gate logits.
+    StageV& sv = c->stage_v;
+    if (b.v1 != b.vt1) sv.vt[0] = b.vt1, sv.v[0] = b.v1, sv.n[0] = T;
+    if (b.v2 != b.vt2) sv.vt[1] = b.vt2, sv.v[1] = b.v2, sv.n[1] = S;
+    sv.filled = c->stage_v_wanted || (!own_graph && is_capturing(st));
     // The context side of the cross-attention: K/V modulation, fused k|v
     // GEMM (split-K partial sums in `part`), on stream s.
     auto ctx_side = [&](hipStream_t s, void* part) {
@@ -765,6 +783,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         gk.sat = sat;
         gk.part = (float*)part;
         gemm16(c, mode, w->kv2, b.enc, S, LTX_D, LTX_EPI_QKV, gk, s, "gemm:kv2");
+        if (sv.filled) fill_stage_v(c, 1, s);
     };
     // Small T (early): the side stream fills the CUs that the main chain leaves
     // idle. Where the last round of the q|k|v GEMM's tiles leaves an eighth of
@@ -833,7 +852,11 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
         c->launch(mode == LTX_MODE_BF16 ? "ltx_qknorm2_bf16" : "ltx_qknorm2_f16", T, 1, 1, 256, &qa, st);
     }
     if (side_gates) HIPC(hipStreamWaitEvent(st, c->side_ev[1], 0));
+    const bool late_v1 = early && side_gates;
+    const bool fill_v1 = sv.filled && sv.vt[0];
+    if (fill_v1 && !late_v1) stream_after(sd, st, c->side_ev[4]);
     attn16(c, mode, b.qh1, b.kh1, b.vt1, vt_ld(T), (const float*)b.glog1, b.o1, T, T, true, st, "attn:self", sat, true);
+    if (fill_v1 && !late_v1) fill_stage_v(c, 0, sd);
     g = LtxGemmArgs{};
     g.out = b.x_sa;
     g.resid = x;
@@ -847,6 +870,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     if (early) {
         if (side_gates) stream_after(sd, st, c->side_ev[2]);
         gate16(c, mode, w->g2, b.attn_in, T, (float*)b.glog2, side_gates ? sd : st);
+        if (fill_v1 && late_v1) fill_stage_v(c, 0, sd);
     }
     g = LtxGemmArgs{};
     g.out = b.q2_16;
@@ -903,7 +927,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     set_stage(c, LTX_ST_NORM_MSA, b.n_msa, TD * 2);
     set_stage(c, LTX_ST_Q1, b.qh1, TD * 2);
     set_stage(c, LTX_ST_K1, b.kh1, TD * 2);
-    set_stage(c, LTX_ST_V1, b.vt1, TD * 2, vt_ld(T));
+    set_stage(c, LTX_ST_V1, b.v1, TD * 2);
     set_stage(c, LTX_ST_GLOG1, b.glog1, (size_t)T * LTX_H * 4);
     set_stage(c, LTX_ST_ATTN1, b.o1, TD * 2);
     set_stage(c, LTX_ST_X_SA, b.x_sa, TD * 4);
@@ -915,7 +939,8 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     set_stage(c, LTX_ST_GLOG2, b.glog2, (size_t)T * LTX_H * 4);
     set_stage(c, LTX_ST_Q2, b.qh2, TD * 2);
     set_stage(c, LTX_ST_K2, b.kh2, SD * 2);
-    set_stage(c, LTX_ST_V2, b.vt2, SD * 2, vt_ld(S));
+    set_stage(c, LTX_ST_V2, b.v2, SD * 2);
+    if (!sv.filled && !own_graph && (sv.vt[0] || sv.vt[1])) HIPC(hipEventRecord(c->stage_ev, st));
 }
 
 bool linear_q8_needs_scratch(const ltx_ctx* c, int N, int K, int mode) {
@@ -1046,7 +1071,7 @@ struct ltx_block_graph {
     // every launch
     void* stage_ptr[LTX_ST_COUNT] = {};
     uint64_t stage_bytes[LTX_ST_COUNT] = {};
-    int stage_vld[2] = {};
+    ltx::StageV stage_v;
 };
 
 int ltx_block_graph_create(ltx_ctx* c, const ltx_block_weights* w, const float* x, const float* tstab, int K,
@@ -1071,7 +1096,7 @@ int ltx_block_graph_create(ltx_ctx* c, const ltx_block_weights* w, const float* 
             throw ltx::Error(std::string("graph capture could not start: ") + hipGetErrorString(eb));
         }
         try {
-            ltx::block_forward(c, w, x, tstab, K, tidx, ctx_tokens, S, pts2, cos, sin, T, y, mode, cs);
+            ltx::block_forward(c, w, x, tstab, K, tidx, ctx_tokens, S, pts2, cos, sin, T, y, mode, cs, true);
         } catch (...) {
             // A throw after the forward forked the context's second stream
             // into the capture leaves that stream capturing: join it back
@@ -1109,7 +1134,7 @@ int ltx_block_graph_create(ltx_ctx* c, const ltx_block_weights* w, const float* 
         g->exec = exec;
         std::memcpy(g->stage_ptr, c->stage_ptr, sizeof(g->stage_ptr));
         std::memcpy(g->stage_bytes, c->stage_bytes, sizeof(g->stage_bytes));
-        std::memcpy(g->stage_vld, c->stage_vld, sizeof(g->stage_vld));
+        g->stage_v = c->stage_v;
         c->ws_pins++;
         *out = g;
     })
@@ -1123,7 +1148,12 @@ int ltx_block_graph_launch(ltx_block_graph* g, void* stream) {
         HIPC(hipGraphLaunch(g->exec, (hipStream_t)stream));
         std::memcpy(c->stage_ptr, g->stage_ptr, sizeof(c->stage_ptr));
         std::memcpy(c->stage_bytes, g->stage_bytes, sizeof(c->stage_bytes));
-        std::memcpy(c->stage_vld, g->stage_vld, sizeof(c->stage_vld));
+        ltx::StageV& sv = c->stage_v = g->stage_v;
+        if (!sv.filled && (sv.vt[0] || sv.vt[1])) {
+            sv.filled = c->stage_v_wanted || ltx::is_capturing((hipStream_t)stream);
+            if (!sv.filled) HIPC(hipEventRecord(c->stage_ev, (hipStream_t)stream));
+            for (int i = 0; i < 2 && sv.filled; i++) ltx::fill_stage_v(c, i, (hipStream_t)stream);
+        }
     })
 }
 

@@ -28,6 +28,20 @@ void hip_check(hipError_t e, const char* what);
 bool fail_in_capture();
 #define HIPC(x) ::ltx::hip_check((x), #x)
 
+// Lets this thread make calls that a capture of another stream, in the global
+// mode, forbids to all threads (allocations, waits); nothing here touches that
+// stream.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    RelaxedCapture() = default;
+    ~RelaxedCapture() {
+        if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+};
+
 // A device allocation owned by the runtime.
 struct DevBuf {
     void* p = nullptr;
@@ -74,6 +88,18 @@ struct ScratchUse {
     }
     ScratchUse(const ScratchUse&) = delete;
     ScratchUse& operator=(const ScratchUse&) = delete;
+};
+
+// The stages V1 and V2 of a 16-bit forward at ragged token counts: v, in the
+// workspace, is vt without the padding of its rows. A forward being captured
+// fills them, and every forward (or graph launch) of a context that has been
+// asked for one; else ltx_block_stage does, when asked the first time. (Filling
+// takes 5 us of a 1,600 us forward at 2,970 tokens.)
+struct StageV {
+    void* vt[2] = {};  // NULL: nothing to fill
+    void* v[2] = {};
+    int n[2] = {};
+    bool filled = false;
 };
 
 struct ProfRec {
@@ -175,8 +201,9 @@ struct ltx_ctx {
     int ws_pins = 0;  // live block graphs: their kernels hold workspace addresses
     void* stage_ptr[LTX_ST_COUNT] = {};
     uint64_t stage_bytes[LTX_ST_COUNT] = {};
-    int stage_vld[2] = {};     // row stride of the V^T stages V1, V2 (0: mode F32)
-    ltx::DevBuf stage_vt[2];   // their rows without the padding (ltx_block_stage)
+    ltx::StageV stage_v;
+    bool stage_v_wanted = false;  // the stages of V have been asked for: forwards fill them
+    hipEvent_t stage_ev = nullptr;  // behind the last forward that left them unfilled
     // profiling
     bool prof = false;
     std::vector<ltx::ProfRec> prof_recs;
@@ -207,7 +234,9 @@ constexpr int kEarlySideRows = 4096;
 void set_thread_error(const std::string& e);
 void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const float* tstab, int K,
                    const int32_t* tidx, const float* ctxv, int S, const float* pts2, const float* cs,
-                   const float* sn, int T, float* y, int mode, hipStream_t st);
+                   const float* sn, int T, float* y, int mode, hipStream_t st, bool own_graph = false);
+void fill_stage_v(ltx_ctx* c, int i, hipStream_t st);
+bool is_capturing(hipStream_t st);
 uint16_t f32_to_f16_bits(float f);
 float bf16_bits_to_f32(uint16_t b);
 float f16_bits_to_f32(uint16_t h);

@@ -45,12 +45,7 @@ struct PlanesUse {
     hipStream_t st;
     explicit PlanesUse(hipStream_t stream) : st(stream) {}
     void* take(Device& dev) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        if (cap != hipStreamCaptureStatusNone) return nullptr;
+        if (ltx::is_capturing(st)) return nullptr;
         lk = std::unique_lock<std::mutex>(dev.mu);
         if (dev.used) HIPC(hipStreamWaitEvent(st, dev.ev, 0));
         d = &dev;

@@ -58,11 +58,7 @@ void DevBuf::free_() {
 // Freeing that waits for the device.
 bool DevBuf::try_grow(size_t n) {
     if (bytes >= n) return true;
-    // A caller may be capturing another stream in the global mode, which forbids
-    // hipMalloc and hipFree to every thread that has not opted out; nothing here
-    // touches that stream.
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    RelaxedCapture relaxed;
     void* q = nullptr;
     bool ok = hipMalloc(&q, n) == hipSuccess;
     if (p) {
@@ -73,18 +69,19 @@ bool DevBuf::try_grow(size_t n) {
         p = q;
         bytes = n;
     }
-    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (!ok) (void)hipGetLastError();  // handled here: clear it for later callers
     return ok;
 }
 
-void* StreamScratch::take(size_t n, hipStream_t st) {
+bool is_capturing(hipStream_t st) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // the legacy stream beside a capture
+    return true;
+}
+
+void* StreamScratch::take(size_t n, hipStream_t st) {
+    if (is_capturing(st)) return nullptr;
     if (!ev) HIPC(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     if (!buf.try_grow(n)) return nullptr;
     if (used) HIPC(hipStreamWaitEvent(st, ev, 0));
@@ -247,6 +244,7 @@ int ltx_init(int device, ltx_ctx** out) {
         }
         HIPC(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));  // default priority
         for (auto& e : c->side_ev) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        HIPC(hipEventCreateWithFlags(&c->stage_ev, hipEventDisableTiming | hipEventDisableSystemFence));
         for (auto& e : c->marks) HIPC(hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventDisableSystemFence));
         for (const unsigned char* co :
              {ltx_co_k_gemm, ltx_co_k_gemm_s4, ltx_co_k_gemm_f3, ltx_co_k_gemm_x4h, ltx_co_k_gemm_q8h, ltx_co_k_attn,
@@ -277,6 +275,7 @@ void ltx_destroy(ltx_ctx* c) {
         if (e) (void)hipEventDestroy(e);
     for (auto e : c->marks)
         if (e) (void)hipEventDestroy(e);
+    if (c->stage_ev) (void)hipEventDestroy(c->stage_ev);
     if (c->side) (void)hipStreamDestroy(c->side);
     c->ws.free_();
     c->op_pairs.free_();
@@ -345,21 +344,16 @@ int ltx_block_stage(ltx_ctx* c, int stage, void** dev_ptr, uint64_t* bytes) {
         if (!c) throw ltx::Error("NULL context");
         if (stage < 0 || stage >= LTX_ST_COUNT) throw ltx::Error("stage id out of range");
         if (!c->stage_ptr[stage]) throw ltx::Error("stage not available (no forward yet, or not in this mode)");
-        void* p = c->stage_ptr[stage];
-        // V^T is kept with rows padded to whole key tiles: hand out [32][128][n]
-        if (stage == LTX_ST_V1 || stage == LTX_ST_V2) {
-            const int i = stage == LTX_ST_V2;
-            const size_t n = c->stage_bytes[stage] / (LTX_D * 2), vld = (size_t)c->stage_vld[i];
-            if (vld && vld != n) {
-                HIPC(hipSetDevice(c->device));
-                HIPC(hipDeviceSynchronize());
-                if (c->stage_vt[i].bytes < c->stage_bytes[stage]) c->stage_vt[i].alloc(c->stage_bytes[stage]);
-                HIPC(hipMemcpy2D(c->stage_vt[i].p, n * 2, p, vld * 2, n * 2, LTX_D, hipMemcpyDeviceToDevice));
-                HIPC(hipDeviceSynchronize());
-                p = c->stage_vt[i].p;
-            }
+        ltx::StageV& sv = c->stage_v;
+        if ((stage == LTX_ST_V1 || stage == LTX_ST_V2) && !sv.filled && (sv.vt[0] || sv.vt[1])) {
+            ltx::RelaxedCapture relaxed;
+            HIPC(hipSetDevice(c->device));
+            HIPC(hipStreamWaitEvent(c->side, c->stage_ev, 0));  // (a device-wide wait would break such a capture)
+            for (int i = 0; i < 2; i++) ltx::fill_stage_v(c, i, c->side);
+            HIPC(hipStreamSynchronize(c->side));
+            sv.filled = c->stage_v_wanted = true;
         }
-        if (dev_ptr) *dev_ptr = p;
+        if (dev_ptr) *dev_ptr = c->stage_ptr[stage];
         if (bytes) *bytes = c->stage_bytes[stage];
     })
 }

@@ -943,3 +943,20 @@ extern "C" __global__ void __launch_bounds__(256) ltx_vt_pad(const LtxVtPadArgs 
     __builtin_memcpy(&v, e, 16);
     *(u32x4*)(a.y + (size_t)d * a.ld + c) = v;
 }
+
+// The other way, for the block's V^T: its rows without the padding (the stages
+// of V that ltx_block_stage hands out).
+extern "C" __global__ void __launch_bounds__(256) ltx_vt_unpad(const LtxVtPadArgs a) {
+    const int c = 8 * (blockIdx.x * 64 + (threadIdx.x & 63)), d = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (c >= a.n) return;
+    const u32x4 v = *(const u32x4*)(a.v + (size_t)d * a.ld + c);
+    uint16_t* dst = a.y + (size_t)d * a.n + c;
+    if (c + 8 <= a.n) {
+        __builtin_memcpy(dst, &v, 16);
+    } else {
+        uint16_t e[8];
+        __builtin_memcpy(e, &v, 16);
+        for (int j = 0; j < 8; j++)
+            if (c + j < a.n) dst[j] = e[j];
+    }
+}

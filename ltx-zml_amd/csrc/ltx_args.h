@@ -178,7 +178,8 @@ typedef struct {
 } LtxAttnArgs;
 
 // V^T rows [LTX_D][n] -> [LTX_D][ld], ld = n rounded up to 64, zeros from
-// column n on (ltx_op_attention, key counts that are no multiple of 64).
+// column n on (ltx_op_attention, key counts that are no multiple of 64); or,
+// ltx_vt_unpad, [LTX_D][ld] -> [LTX_D][n].
 typedef struct {
     const uint16_t* v;
     uint16_t* y;

@@ -30,9 +30,12 @@ struct Op {
     LtxGemmArgs gemm{};
     LtxAttnArgs attn{};
     LtxVtPadArgs vt{};
+    std::map<hipStream_t, uint64_t> clock;  // launch: what of each stream precedes it, itself included
 };
 
 inline std::vector<Op> log;
+inline std::map<hipStream_t, std::map<hipStream_t, uint64_t>> streams;  // each stream's clock
+inline std::map<hipEvent_t, std::map<hipStream_t, uint64_t>> events;    // and each event's, as recorded
 inline std::map<uint64_t, uint64_t> mem;   // live allocations
 inline uint64_t next_addr = 1ull << 40, in_use = 0, limit = ~0ull;
 inline std::set<hipStream_t> capturing;    // streams being captured, in global mode
@@ -52,6 +55,11 @@ inline bool inside(uint64_t p, uint64_t n) {
     if (it == mem.begin()) return false;
     --it;
     return p >= it->first && p + n <= it->first + it->second;
+}
+// a is done before b starts
+inline bool before(const Op& a, const Op& b) {
+    auto it = b.clock.find(a.stream);
+    return it != b.clock.end() && it->second >= a.clock.at(a.stream) && &a != &b;
 }
 inline bool inside(const void* p, uint64_t n) { return inside((uint64_t)p, n); }
 
@@ -102,7 +110,13 @@ hipError_t hipMemcpy2D(void*, size_t, const void*, size_t, size_t, size_t, hipMe
 hipError_t hipMemset(void*, int, size_t) { return fake::forbidden(); }
 hipError_t hipDeviceSynchronize() {
     fake::log.push_back({"sync"});
-    return fake::forbidden();
+    if (fake::capturing.empty()) return hipSuccess;
+    fake::broken_capture = true;  // also for a thread that has opted out
+    return hipErrorStreamCaptureUnsupported;
+}
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    fake::log.push_back({"sync"});
+    return fake::capturing.count(s) ? hipErrorStreamCaptureUnsupported : hipSuccess;
 }
 hipError_t hipGetSymbolAddress(void** p, const void*) {
     *p = (void*)(fake::next_addr);
@@ -118,6 +132,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
     o.event = e;
     o.stream = s;
     fake::log.push_back(o);
+    fake::events[e] = fake::streams[s];
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
@@ -125,6 +140,7 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
     o.event = e;
     o.stream = s;
     fake::log.push_back(o);
+    for (auto& [stream, n] : fake::events[e]) fake::streams[s][stream] = std::max(fake::streams[s][stream], n);
     return hipSuccess;
 }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
@@ -152,6 +168,8 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned, unsigned, unsigned, 
     o.name = (const char*)f;
     o.stream = s;
     if (o.name == fake::fail_launch) return hipErrorUnknown;
+    fake::streams[s][s]++;
+    o.clock = fake::streams[s];
     auto is = [&](const char* prefix) { return o.name.rfind(prefix, 0) == 0; };
     if (is("ltx_split3")) o.split = *(LtxSplit3Args*)params[0];
     if (is("ltx_gemm_f3_")) o.f3 = *(LtxGemmF3Args*)params[0];

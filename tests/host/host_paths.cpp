@@ -223,6 +223,77 @@ static void noalloc_f32() {
     for (const fake::Op& o : fake::log) CHECK(o.what == "launch", "%s in a capture", o.what.c_str());
 }
 
+// The stages of V at ragged token counts: addresses of the workspace, like all
+// others. The first question after an eager forward may wait for it and fill them
+// (allocating nothing, and beside a capture on another stream); from then on, and
+// in a captured forward, they are filled between the GEMM that forms V and the
+// end of the forward, and asking does nothing.
+static void stage_v(int T, int S, int mode, bool captured) {
+    ltx_ctx* c = make_ctx();
+    ltx_block_weights w;
+    fill(w, mode != LTX_MODE_BF16);
+    w.f16_max = 1.0f;
+    const hipStream_t st = (hipStream_t)0x10, other = (hipStream_t)0x20;
+    void* first[2] = {};
+    if (captured) {
+        forward(c, w, T, S, mode, st);  // (sizes the workspace)
+        fake::capturing.insert(st);
+    }
+    for (int pass = 0; pass < 2; pass++) {
+        fake::log.clear();
+        forward(c, w, T, S, mode, st);
+        const std::vector<fake::Op> ops = fake::log;
+        const bool asking = !captured && !pass;
+        fake::capturing.insert(other);
+        fake::log.clear();
+        for (int i = 0; i < 2; i++) {
+            const int n = i ? S : T;
+            void* p = nullptr;
+            uint64_t bytes = 0;
+            CHECK(ltx_block_stage(c, i ? LTX_ST_V2 : LTX_ST_V1, &p, &bytes), "%s", ltx_last_error(c));
+            for (const fake::Op& o : fake::log)
+                CHECK(asking && (o.what == "sync" || o.what == "wait" || (o.name == "ltx_vt_unpad" && o.stream == c->side)),
+                      "%s %s on asking for stage V%d", o.what.c_str(), o.name.c_str(), i + 1);
+            CHECK(bytes == (uint64_t)n * LTX_D * 2, "%zu bytes", (size_t)bytes);
+            CHECK((uint64_t)p >= (uint64_t)c->ws.p && (uint64_t)p + bytes <= (uint64_t)c->ws.p + c->ws.bytes,
+                  "stage V%d outside the workspace", i + 1);
+            if (!first[i]) first[i] = p;
+            CHECK(p == first[i], "stage V%d moved", i + 1);
+            // the attention over n keys reads V at v; p is v itself or filled from it
+            const fake::Op *attn = nullptr, *copy = nullptr, *gemm = nullptr;
+            for (const fake::Op& o : ops)
+                if (o.name.rfind("ltx_attn", 0) == 0 && (!attn || i)) attn = &o;
+            for (const fake::Op& o : ops) {
+                if (o.name == "ltx_vt_unpad" && o.vt.y == p) copy = &o;
+                if (o.gemm.out2 == attn->attn.vt && o.gemm.out2) gemm = &o;
+            }
+            CHECK(gemm, "no GEMM forms V%d", i + 1);
+            CHECK(fake::before(*gemm, *attn), "the attention does not wait for V%d", i + 1);
+            if (asking) {
+                if (p != attn->attn.vt) {
+                    int fills = 0;
+                    for (const fake::Op& o : fake::log)
+                        if (o.name == "ltx_vt_unpad" && o.vt.y == p) {
+                            fills++;
+                            CHECK(fake::before(*gemm, o), "stage V%d is filled before V is formed", i + 1);
+                        }
+                    CHECK(!copy && fills == 1 && fake::log.back().what == "sync", "stage V%d filled %d times", i + 1,
+                          fills);
+                }
+            } else if (p != attn->attn.vt) {
+                CHECK(copy && copy->vt.v == attn->attn.vt && copy->vt.n == n && copy->vt.ld == attn->attn.v_rs,
+                      "nothing fills stage V%d", i + 1);
+                CHECK(fake::before(*gemm, *copy), "stage V%d is filled before V is formed", i + 1);
+                CHECK(fake::before(*copy, ops.back()), "the forward does not wait for stage V%d", i + 1);
+            } else {
+                CHECK(n == attn->attn.v_rs, "stage V%d has padded rows", i + 1);
+            }
+        }
+        CHECK(!fake::broken_capture, "a capture is broken");
+        fake::capturing.erase(other);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -245,6 +316,8 @@ int main(int argc, char** argv) {
         noalloc_f32();
     else if (cmd == "planes_bound_noalloc")
         planes_bound(arg(2), arg(3), arg(4), true);
+    else if (cmd == "stage_v")
+        stage_v(arg(2), arg(3), arg(4), arg(5));
     else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv
         ltx_ctx* c = make_ctx();
         for (int i = 2; i + 1 < argc; i += 2) {

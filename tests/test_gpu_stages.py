@@ -27,6 +27,8 @@ independently of the oracle, and the int8 recipe's own error against the
 unquantised block with the reference's pre-registered budgets
 (ltx/block_conformance.zig:466-494).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -332,3 +334,89 @@ def test_block_tile_rows(monkeypatch, block0, block0_w16, mode, x4, T, S, weight
     assert np.isfinite(ys[0]).all()
     assert oracle.rel_rms(*ys) <= (2.0 ** -11 if mode == "f16" else 2.0 ** -8)
     assert all(np.array_equal(*x) for x in zip(*xs))
+
+
+class _Memory:
+    """Device memory at an address, as torch.as_tensor takes it."""
+
+    def __init__(self, ptr, shape):
+        self.__cuda_array_interface__ = dict(data=(ptr, False), shape=shape, typestr="<i2", version=3)
+
+
+def _stage_v(c, T, S):
+    """The stages V1 and V2 in place (16-bit words)."""
+    views = []
+    for name, n in (("v1", T), ("v2", S)):
+        p, b = C.c_void_p(), C.c_uint64()
+        assert rt.lib().ltx_block_stage(c.handle, rt.STAGES.index(name), C.byref(p), C.byref(b))
+        assert b.value == H * HD * n * 2
+        views.append(torch.as_tensor(_Memory(p.value, (H, HD, n)), device="cuda"))
+    return views
+
+
+def test_stages_of_v_follow_forwards(block0):
+    """V's stages at ragged token counts, whose attention reads padded rows: of an
+    eager forward, first asked for beside a capture; then in place after the next
+    forward without asking again; of a block graph; and in a caller's own graph of
+    a context that was never asked before."""
+    T, S = 250, 40
+    say(f"stages of V follow forwards T={T} S={S}")
+    inps = [synth.make_inputs(T, S, seed=i, sigma=0.7) for i in range(2)]
+    cos, sin = rt.rope_tables(inps[0]["grid"])
+    bufs = [torch.empty_like(dev(inps[0][n])) for n in ("x", "tstab", "tidx", "ctx", "pts2")]
+    y = torch.empty((T, D), dtype=torch.float32, device="cuda")
+
+    def put(i):
+        for b, n in zip(bufs, ("x", "tstab", "tidx", "ctx", "pts2")):
+            b.copy_(dev(inps[i][n]))
+    dcos, dsin = dev(cos), dev(sin)
+    ctxs = [rt.Context(0) for _ in range(3)]
+    try:
+        ws = [c.upload(block0) for c in ctxs]
+        args = lambda w: (w, *bufs, dcos, dsin, y)  # noqa: E731
+        # eager; the first question while another stream is captured
+        c, w = ctxs[0], ws[0]
+        put(0)
+        c.forward(*args(w), mode=rt.MODE_F16)
+        spare, graph = torch.zeros(64, device="cuda"), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, capture_error_mode="global"):
+            spare.add_(1)
+            views = _stage_v(c, T, S)
+        want = [[v.clone() for v in views]]
+        graph.replay()
+        put(1)
+        c.forward(*args(w), mode=rt.MODE_F16)
+        want.append([v.clone() for v in views])
+        torch.cuda.synchronize()
+        assert (spare == 1).all() and not torch.equal(want[0][0], want[1][0])
+        v = oracle.rel_rms(want[1][0].view(torch.float16).float().cpu().numpy(),
+                           c.stage("v1").view(torch.float16).reshape(H, HD, T).float().cpu().numpy())
+        assert v == 0 and torch.isfinite(want[1][0].view(torch.float16)).all()
+        # a block graph
+        c, w = ctxs[1], ws[1]
+        g = c.block_graph(*args(w), mode=rt.MODE_F16)
+        for i in (0, 1, 0):
+            put(i)
+            g.launch()
+            if not i:
+                views = _stage_v(c, T, S)
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(views, want[i])), i
+        g.free()
+        # a caller's graph
+        c, w = ctxs[2], ws[2]
+        c.forward(*args(w), mode=rt.MODE_F16)
+        torch.cuda.synchronize()
+        outs, graph = [torch.empty_like(v) for v in want[0]], torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            c.forward(*args(w), mode=rt.MODE_F16)
+            for o, v in zip(outs, _stage_v(c, T, S)):
+                o.copy_(v)
+        for i in (1, 0, 1):
+            put(i)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(outs, want[i])), i
+    finally:
+        for c in ctxs:
+            c.close()

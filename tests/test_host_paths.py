@@ -55,6 +55,15 @@ def test_f32_linear_planes_are_bounded(host_paths, M, N, K):
     host_paths("planes_bound", M, N, K)
 
 
+@pytest.mark.parametrize("captured", [0, 1])
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("T,S", [(250, 40), (256, 64), (1024, 77), (2970, 128), (2970, 100), (4100, 1), (8200, 300)])
+def test_stages_of_v_stay_in_the_workspace(host_paths, T, S, mode, captured):
+    """Whole and ragged token counts on every schedule of the second stream, int8
+    and (mode 1) unquantised weights."""
+    host_paths("stage_v", T, S, mode, captured)
+
+
 def test_noalloc_f32_calls_are_independent(host_paths):
     host_paths("noalloc_f32")
 
