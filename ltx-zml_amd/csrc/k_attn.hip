@@ -838,6 +838,10 @@ struct AttnPP {
             if (prev) {
                 store_out<32>(patch, h, q0 - 256 * wph, lane, gl, bad);
                 load_glog(gl, h, q0, lane);
+                // (softmax(first) scales by 0, which would keep a NaN)
+#pragma unroll
+                for (int db = 0; db < 8; db++) o[db][0] = o[db][1] = f32x4{0};
+                l = f32x2{0.f, 0.f};
             }
             softmax(true, nt == 1);
             if (nt == 1) next_tile(qn);

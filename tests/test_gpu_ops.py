@@ -490,6 +490,26 @@ def test_attention_ragged_keys(ctx, mode, q_scaled, lq, lkv):
     assert oracle.rel_rms(f64(out), want) <= (2e-3 if mode == "f16" else 1e-2)
 
 
+@pytest.mark.parametrize("lq,lkv", [(4200, 100), (4200, 192), (8200, 40), (2100, 250), (300, 450)])
+def test_attention_nan_query_stays_in_its_row(ctx, lq, lkv):
+    """Resident K/V, several query tiles a workgroup one after the other, and the
+    streaming forms: a query of NaN makes its own row NaN and no other."""
+    say(f"attention NaN query lq={lq} lkv={lkv}")
+    g = torch.Generator(device="cuda").manual_seed(lq + lkv)
+    q, k, v = (torch.randn(32, n, d, generator=g, device="cuda").half() for n, d in ((lq, 128), (lkv, 128), (128, lkv)))
+    out, want = (torch.full((lq, 4096), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    ctx.attention(q, k, v, None, want, lq, lkv)
+    q[:, 5] = float("nan")
+    ctx.attention(q, k, v, None, out, lq, lkv)
+    torch.cuda.synchronize()
+    assert torch.isnan(out[5]).all() and torch.isfinite(want).all()
+    rest = torch.arange(lq, device="cuda") != 5
+    assert torch.isfinite(out[rest]).all()
+    # the NaN's wave moves its maxima at every tile: P and the output, each
+    # rounded once to f16, as test_attention
+    assert oracle.rel_rms(f64(out[rest]), f64(want[rest])) <= 2e-3
+
+
 @pytest.mark.parametrize("lq,lkv", [(16, 128), (127, 192), (129, 320), (1024, 200), (1025, 320)])
 def test_attention_query_tiles(ctx, lq, lkv):
     """128-query workgroups (up to 1,024 queries) at the edges of a tile and of
