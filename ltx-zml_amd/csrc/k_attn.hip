@@ -374,6 +374,7 @@ struct AttnPP {
     f32x4 sb[NQ];           // -m of the lane's query in block qb: the S MFMAs start from it
     f32x2 m, l;             // running max and partial sum per query block (vectors, not arrays: kept in registers)
     float C;
+    float most;  // largest row sum of a tile that keeps the max: 256, or -1 (see softmax)
     int nt, g;
 
     __device__ __forceinline__ AttnPP(const LtxAttnArgs& args) : a(args) {}
@@ -499,7 +500,9 @@ struct AttnPP {
     // to inf) is the tile max taken (over the query's four lanes), the max
     // moved, the output and row sum rescaled (after PV(t-1), before PV(t))
     // and the weights formed again. The first tile always takes that path
-    // and sets m to its max.
+    // and sets m to its max; where a query of the wave has had no score above
+    // -inf yet, its m stays 0 and the wave's next tile takes the path too, as its
+    // first (most = -1: a flag beside the test cost 2 %).
     // LAST: this may be the last tile, whose keys past lkv get no weight.
     template <bool LAST = true>
     __device__ __forceinline__ void softmax(bool first, bool last) {
@@ -513,8 +516,9 @@ struct AttnPP {
                     if (32 * (kb >> 1) + 4 * (kb & 1) + r >= left) s[kb][0][r] = s[kb][NQ - 1][r] = -__builtin_inff();
         }
         f32x2 ps = exps<false>(f32x2{0.f, 0.f});
-        if (first || __builtin_amdgcn_ballot_w64(!(ps[0] <= 256.0f) || !(ps[NQ - 1] <= 256.0f)) != 0) {
+        if (first || __builtin_amdgcn_ballot_w64(!(ps[0] <= most) || !(ps[NQ - 1] <= most)) != 0) {
             f32x2 delta = {0.f, 0.f};
+            bool none = false;
 #pragma unroll
             for (int qb = 0; qb < NQ; qb++) {
                 float mx = s[0][qb][0];
@@ -523,9 +527,10 @@ struct AttnPP {
 #pragma unroll
                     for (int r = 0; r < 4; r++) mx = fmaxf(mx, s[kb][qb][r]);
                 mx = asp_quad_max(mx);  // tile max relative to m
-                // (a first tile with no finite score keeps m = 0)
-                delta[qb] = first ? (mx == -__builtin_inff() ? 0.f : mx) : fmaxf(mx, 0.f);
-                const float corr = first ? 0.f : __builtin_amdgcn_exp2f(PS ? -delta[qb] : -delta[qb] * C);
+                const bool start = first || (most < 0.f && asp_quad_max(l[qb]) == 0.f), inf = mx == -__builtin_inff();
+                none |= start && inf;
+                delta[qb] = start ? (inf ? 0.f : mx) : fmaxf(mx, 0.f);
+                const float corr = start ? 0.f : __builtin_amdgcn_exp2f(PS ? -delta[qb] : -delta[qb] * C);
                 m[qb] += delta[qb];
                 l[qb] *= corr;
 #pragma unroll
@@ -533,6 +538,7 @@ struct AttnPP {
                 sb[qb] = f32x4{0} - m[qb];
             }
             ps = exps<true>(delta);
+            most = __builtin_amdgcn_ballot_w64(none) != 0 ? -1.0f : 256.0f;
         }
         l += ps;
     }
@@ -638,6 +644,7 @@ struct AttnPP {
         m = f32x2{0.f, 0.f};
         sb[0] = sb[NQ - 1] = f32x4{0};
         l = f32x2{0.f, 0.f};
+        most = 256.0f;
     }
 
     // gate logits glog[q][h] of the lane's two queries (rows past lq read

@@ -510,6 +510,36 @@ def test_attention_nan_query_stays_in_its_row(ctx, lq, lkv):
     assert oracle.rel_rms(f64(out[rest]), f64(want[rest])) <= 2e-3
 
 
+@pytest.mark.parametrize("mode,q_scaled", [("f16", False), ("bf16", True)])
+@pytest.mark.parametrize("lq,lkv", [(300, 450), (2100, 450), (4200, 130), (8200, 250), (300, 320)])
+def test_attention_keys_without_weight_first(ctx, mode, q_scaled, lq, lkv):
+    """The first 64 keys score -inf (NaN for every second query) and the others far below
+    0: nothing of the first tile may set the scale of the ones behind it."""
+    say(f"attention first keys -inf mode={mode} lq={lq} lkv={lkv}")
+    m, dt = MODES[mode]
+    cq = np.float32(rt.ATTN_C if q_scaled else 1.0)
+    rng = np.random.default_rng(lq + lkv)
+    q, k, v = (rng.standard_normal((n, 4096)).astype(np.float32) for n in (lq, lkv, lkv))
+    q, k = q.reshape(lq, 32, 128), k.reshape(lkv, 32, 128)
+    q[:, :, 0], k[:, :, 0] = 1.0, 0.0
+    k[:64, :, 0] = -np.inf
+    q[:, :, 1], k[:, :, 1] = 30.0, -30.0  # scores around -80
+    q[1::2, :, 0] = 0.0
+    k[64:, :, 2:] *= 0.5
+    dq, dk = to16(_heads((q * cq).reshape(lq, 4096), lq), dt), to16(_heads(k.reshape(lkv, 4096), lkv), dt)
+    dv = to16(np.ascontiguousarray(v.reshape(lkv, 32, 128).transpose(1, 2, 0)), dt)
+    out = torch.full((lq, 4096), float("nan"), dtype=dt, device="cuda")
+    ctx.attention(dq.cuda(), dk.cuda(), dv.cuda(), None, out, lq, lkv, mode=m, q_scaled=q_scaled)
+    torch.cuda.synchronize()
+    rows = slice(0, lq, 2)  # (0 times -inf: the other rows are NaN)
+    assert torch.isnan(out[1::2]).all()
+    want = oracle.sdpa(f64(dq)[:, rows].transpose(1, 0, 2).reshape(-1, 4096) / cq,
+                       f64(dk)[:, 64:].transpose(1, 0, 2).reshape(lkv - 64, 4096),
+                       f64(dv)[:, :, 64:].transpose(2, 0, 1).reshape(lkv - 64, 4096), chunk=0)
+    # as test_attention
+    assert oracle.rel_rms(f64(out[rows]), want) <= (2e-3 if mode == "f16" else 1e-2)
+
+
 @pytest.mark.parametrize("lq,lkv", [(16, 128), (127, 192), (129, 320), (1024, 200), (1025, 320)])
 def test_attention_query_tiles(ctx, lq, lkv):
     """128-query workgroups (up to 1,024 queries) at the edges of a tile and of
