@@ -1223,11 +1223,13 @@ int ltx_op_attention(ltx_ctx* c, const void* q, const void* k, const void* v, co
             return LTX_OK;
         }
         // V^T's rows padded to whole key tiles for the LDS-DMA kernels (not
-        // captured: then the any-length kernel)
+        // captured, or with K's rows off the DMA's 16 bytes: then the any-length
+        // kernel)
         const int vld = ltx::vt_ld(lkv);
         void* pad = nullptr;
         ltx::ScratchUse use(c->op_scratch, st);
-        if (vld != lkv && c->attn_pp && ltx::pad_pays(c, lq, lkv) && (pad = use.take((size_t)LTX_D * vld * 2))) {
+        if (vld != lkv && c->attn_pp && ((uintptr_t)k & 15) == 0 && ltx::pad_pays(c, lq, lkv) &&
+            (pad = use.take((size_t)LTX_D * vld * 2))) {
             LtxVtPadArgs pa{(const uint16_t*)v, (uint16_t*)pad, lkv, vld};
             c->launch("ltx_vt_pad", (vld + 511) / 512, LTX_D / 4, 1, 256, &pa, st);
         }

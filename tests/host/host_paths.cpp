@@ -86,8 +86,8 @@ static bool linear(ltx_ctx* c, int M, int N, int K, int mode, hipStream_t st, bo
     return f(c, ptr(0), (const int8_t*)ptr(1), ptr(2), scale_f16, nullptr, ptr(3), mode == LTX_MODE_F32, M, N, K, 0, mode,
              st);
 }
-static bool attention(ltx_ctx* c, int lq, int lkv, hipStream_t st) {
-    return ltx_op_attention(c, ptr(0), ptr(1), ptr(2), nullptr, ptr(3), lq, lkv, LTX_MODE_F16, st);
+static bool attention(ltx_ctx* c, int lq, int lkv, hipStream_t st, size_t k_off = 0) {
+    return ltx_op_attention(c, ptr(0), (char*)ptr(1) + k_off, ptr(2), nullptr, ptr(3), lq, lkv, LTX_MODE_F16, st);
 }
 
 // The uses of one shared scratch follow each other, whatever the stream's
@@ -316,7 +316,15 @@ int main(int argc, char** argv) {
         noalloc_f32();
     else if (cmd == "planes_bound_noalloc")
         planes_bound(arg(2), arg(3), arg(4), true);
-    else if (cmd == "stage_v")
+    else if (cmd == "attn_misaligned") {
+        ltx_ctx* c = make_ctx();
+        for (size_t off : {2, 8}) {
+            fake::log.clear();
+            CHECK(attention(c, 2970, 2970, nullptr, off), "%s", ltx_last_error(c));
+            CHECK(launches("") == 1 && launches("ltx_attn_f16_w8") == 1, "K %zu bytes past alignment: %s", off,
+                  fake::log[0].name.c_str());
+        }
+    } else if (cmd == "stage_v")
         stage_v(arg(2), arg(3), arg(4), arg(5));
     else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv
         ltx_ctx* c = make_ctx();

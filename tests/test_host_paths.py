@@ -74,6 +74,11 @@ def test_noalloc_f32_planes_fit_the_array(host_paths, M, N, K):
     host_paths("planes_bound_noalloc", M, N, K)
 
 
+def test_attention_with_misaligned_keys_stays_any_length(host_paths):
+    """Ragged key counts with K off a 16-byte boundary: not for 16-byte LDS DMA."""
+    host_paths("attn_misaligned")
+
+
 def test_attention_pads_where_it_pays(host_paths):
     """(queries, keys) on both sides of each line of the padding rule: the calls
     measured faster on the any-length kernel stay on it."""
