@@ -1193,9 +1193,10 @@ int ltx_op_linear_q8(ltx_ctx* c, const void* a, const int8_t* q, const void* sca
         if (const size_t np = packed ? ltx::linear_part_bytes(c, M, N, K, mode) : 0)
             sc.part = use.take(np);
         if (ltx::linear_q8_needs_scratch(c, N, K, mode)) {
-            // scratch owned by the context, grown as needed
+            // scratch owned by the context, grown as needed; all that a call of
+            // this shape may use, so that one call warms up for every alignment
             const size_t nq = (size_t)N * K, np = (size_t)N * (K / LTX_GROUP) * 4;
-            if (!packed && c->op_q.bytes < nq) c->op_q.alloc(nq);
+            if (c->op_q.bytes < nq) c->op_q.alloc(nq);
             if (c->op_pairs.bytes < np) c->op_pairs.alloc(np);
             sc.q = (uint32_t*)c->op_q.p;
             sc.pairs = (uint32_t*)c->op_pairs.p;

@@ -294,6 +294,23 @@ static void stage_v(int T, int S, int mode, bool captured) {
     }
 }
 
+// After one call of a shape, calls of that shape on the same stream allocate
+// nothing, whatever the alignment of their operands: a program that warms up and
+// then captures.
+static void linear_warmed() {
+    for (int mode : {LTX_MODE_F16, LTX_MODE_BF16}) {
+        ltx_ctx* c = make_ctx();
+        CHECK(linear(c, 300, 4096, 4096, mode, nullptr), "%s", ltx_last_error(c));
+        const hipStream_t cap = (hipStream_t)0x30;
+        fake::capturing.insert(cap);
+        CHECK(ltx_op_linear_q8(c, ptr(0), (const int8_t*)ptr(1) + 4, ptr(2), 1, nullptr, ptr(3), 0, 300, 4096, 4096, 0, mode,
+                               cap),
+              "%s", ltx_last_error(c));
+        CHECK(!fake::broken_capture, "the capture is broken");
+        fake::capturing.clear();
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -324,7 +341,9 @@ int main(int argc, char** argv) {
             CHECK(launches("") == 1 && launches("ltx_attn_f16_w8") == 1, "K %zu bytes past alignment: %s", off,
                   fake::log[0].name.c_str());
         }
-    } else if (cmd == "stage_v")
+    } else if (cmd == "linear_warmed")
+        linear_warmed();
+    else if (cmd == "stage_v")
         stage_v(arg(2), arg(3), arg(4), arg(5));
     else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv
         ltx_ctx* c = make_ctx();

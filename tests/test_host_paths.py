@@ -79,6 +79,10 @@ def test_attention_with_misaligned_keys_stays_any_length(host_paths):
     host_paths("attn_misaligned")
 
 
+def test_linear_allocates_nothing_once_warmed(host_paths):
+    host_paths("linear_warmed")
+
+
 def test_attention_pads_where_it_pays(host_paths):
     """(queries, keys) on both sides of each line of the padding rule: the calls
     measured faster on the any-length kernel stay on it."""
