@@ -85,7 +85,9 @@ bool x4_shape(const ltx_ctx* c, int mode, int M, int N, int K, int lda, bool w16
     // where its 256 x 256 tiles fill the CUs: the sizes that need no split-K.
     // 16-bit weights (no dequantisation): as soon as the 256 x 128 tiles of the
     // other kernel need a second round for 4,096 columns (o1 and o2 at 2,970
-    // rows 84 against 120 us)
+    // rows 84 against 120 us; the whole unquantised block in bf16, before and
+    // with it: 2,049 tokens 1,592 : 1,290 us, 2,500 1,670 : 1,328, 2,970 1,883 :
+    // 1,572, 4,000 2,131 : 1,960; 2,048 tokens, on the other kernel, 1,030)
     return M >= (w16 ? 2049 : 4096) && gemm_ksplit(c->num_cu, M, N, K) == 1;
 }
 
@@ -138,7 +140,9 @@ int f3_rows(const ltx_ctx* c, int M, int N, int K, size_t room) {
 // instead of from the words that a launch of 5 us lays out: the gathers cost more
 // with more row tiles on the chip. Measured, packed against words, us (rows x N,
 // K = 4,096): 16 x 4,096 17.8 : 21.4, 128 x 4,096 24.2 : 27.4, 256 x 8,192 34.5 :
-// 36.3; 512 x 8,192 50.2 : 44.7, 1,024 x 4,096 49.4 : 45.2.
+// 36.3; 300 x 4,096 34.1 : 35.7, x 8,192 43.3 : 42.2, x 16,384 65.3 : 66.4; 448 x
+// 8,192 44.8 : 43.6, bf16 x 16,384 85.9 : 84.3; 512 x 8,192 45.4 : 44.6, 1,024 x
+// 4,096 49.4 : 45.2.
 static bool s4_packed_scales(int M) { return M <= 256; }
 
 // The small-T schedule of the block forward (side stream from the first
@@ -797,7 +801,9 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     // GEMM fills the chip, side work beside it would wait for its end and then
     // slow the q and k norms: the context side starts with the forward, beside
     // the first norm, and the gate logits run on the main stream (2,970 tokens:
-    // 1,613 against 1,645 us).
+    // 1,613 against 1,645 us). At 21 token counts from 300 to 4,095, f16 and bf16,
+    // that line chose the faster schedule or one within 1.3 % (a last round of 224
+    // tiles: the side stream faster by 1.2 to 2.3 %; of 240: no difference).
     // Large T: side work starts only after the persistent GEMMs, whose
     // one-workgroup-per-CU grids it would otherwise hold back, and ends before
     // the attentions, which it would slow as much as it gains.

@@ -228,7 +228,8 @@ struct MarkScope {
 };
 constexpr int kMarkRows = 8192;
 // below this many tokens the block's GEMM and attention grids leave CUs idle:
-// the side stream starts at the first RMSNorm + modulate (block_forward)
+// the side stream starts behind the first RMSNorm + modulate, or with the forward
+// (block_forward)
 constexpr int kEarlySideRows = 4096;
 
 void set_thread_error(const std::string& e);

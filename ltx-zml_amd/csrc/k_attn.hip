@@ -6,7 +6,7 @@
 //   tiles, K and V^T streamed global -> LDS by DMA; the block's self- and
 //   cross-attention take it. Keys past lkv are masked in the last tile, and
 //   V^T's rows are padded with zeros to whole tiles (0 * p stays 0): 2,970
-//   queries and keys 154 us with the padding's launch, 278-308 us on the w8
+//   queries and keys 161 us with the padding's launch, 278-308 us on the w8
 //   kernel, which took every ragged key count before;
 // - ltx_attn_{f16,bf16}_w8[_full] (any key count, V^T rows of any stride): 8
 //   waves of 32 queries, K and V^T staged through registers into LDS, keys

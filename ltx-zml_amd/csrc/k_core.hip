@@ -1,6 +1,7 @@
 // Kernels of the parts around the blocks (ltx/core_parts.zig) and of the
-// distilled scheduler (ltx/scheduler.zig). All f32; the linear layers of a few
-// rows run here, the others on the f32 GEMM (k_f32.hip).
+// distilled scheduler (ltx/scheduler.zig). All f32: patchify and the output tail
+// at every token count, the conditioning MLPs up to 32 rows (more on the f32 GEMM,
+// k_f32.hip).
 #include "ltx_device.h"
 
 // DDPM/PixArt sinusoid of t * 1000, cos half first, divisor HALF = 128

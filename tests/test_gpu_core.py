@@ -151,8 +151,9 @@ def test_patchify_and_tail(ctx, core_np, core_dev, T):
 
 @pytest.mark.parametrize("T", [1, 17, 4100])
 def test_patchify_and_tail_edges(ctx, core_np, core_dev, T):
-    """One token, one past a 16-token tile, and enough ragged 32-token tiles to
-    share out the columns over fewer workgroups."""
+    """One token, one past a 16-token block, and a ragged last tile behind many whole
+    ones in both kernels (64 and 32 tokens), some of whose tokens are of two
+    timestep rows."""
     test_patchify_and_tail(ctx, core_np, core_dev, T)
 
 
