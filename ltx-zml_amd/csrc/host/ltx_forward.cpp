@@ -229,7 +229,7 @@ static void carve32(Carve& c, Ws32& w, size_t T, size_t S, const ltx_ctx* ctx) {
     const int shapes[4][3] = {{(int)T, LTX_D, LTX_D}, {(int)S, LTX_D, LTX_D}, {(int)T, LTX_FF, LTX_D},
                               {(int)T, LTX_D, LTX_FF}};
     for (const auto& sh : shapes) {
-        if (!f3_shape(ctx, sh[0], sh[1], sh[2])) continue;
+        if (!ctx->ws_planes || !f3_shape(ctx, sh[0], sh[1], sh[2])) continue;
         planes = std::max(planes, f3_planes_bytes(sh[0], sh[2]));
         part = std::max(part, f3_part_bytes(ctx, sh[0], sh[1], sh[2]));
     }
@@ -238,21 +238,35 @@ static void carve32(Carve& c, Ws32& w, size_t T, size_t S, const ltx_ctx* ctx) {
     if (part) w.part = c.take(part);
 }
 
-static void ensure_ws(ltx_ctx* c, size_t T, size_t S, int mode) {
-    Carve cv{nullptr, 0, 0, true};
-    if (mode == LTX_MODE_F32) {
-        Ws32 w;
-        carve32(cv, w, T, S, c);
-    } else {
-        Ws16 w;
-        carve16(cv, w, T, S, c, mode);
+// Room for a forward. Mode F32's planes only where there is room for them too: a
+// forward without runs its GEMMs on the f32 MFMA kernel, as before they had any.
+// grow: may allocate for them (not in a capture).
+static void ensure_ws(ltx_ctx* c, size_t T, size_t S, int mode, bool grow = true) {
+    auto need = [&]() {
+        Carve cv{nullptr, 0, 0, true};
+        if (mode == LTX_MODE_F32) {
+            Ws32 w;
+            carve32(cv, w, T, S, c);
+        } else {
+            Ws16 w;
+            carve16(cv, w, T, S, c, mode);
+        }
+        return cv.off;
+    };
+    c->ws_planes = true;
+    size_t n = need();
+    if (mode == LTX_MODE_F32 && c->ws.bytes < n) {
+        c->ws_planes = false;
+        const size_t least = need();
+        c->ws_planes = n > least && grow && !c->ws_pins && hipDeviceSynchronize() == hipSuccess && c->ws.try_grow(n);
+        if (!c->ws_planes) n = least;
     }
-    if (c->ws.bytes < cv.off) {
+    if (c->ws.bytes < n) {
         if (c->ws_pins)
             throw Error("the workspace is bound by " + std::to_string(c->ws_pins) +
                         " live block graph(s) and this forward needs a larger one; destroy them first");
         HIPC(hipDeviceSynchronize());
-        c->ws.alloc(cv.off);
+        c->ws.alloc(n);
     }
 }
 
@@ -673,7 +687,7 @@ void block_forward(ltx_ctx* c, const ltx_block_weights* w, const float* x, const
     if ((const void*)x == (const void*)y) throw Error("y may not alias x");
     if (mode != LTX_MODE_F16 && mode != LTX_MODE_BF16 && mode != LTX_MODE_F32) throw Error("unknown mode");
     HIPC(hipSetDevice(c->device));
-    ensure_ws(c, (size_t)T, (size_t)S, mode);
+    ensure_ws(c, (size_t)T, (size_t)S, mode, !is_capturing(st));
     std::memset(c->stage_ptr, 0, sizeof(c->stage_ptr));
     c->stage_v = StageV{};
     const size_t TD = (size_t)T * LTX_D, SD = (size_t)S * LTX_D;

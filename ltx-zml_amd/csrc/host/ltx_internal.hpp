@@ -198,6 +198,7 @@ struct ltx_ctx {
     ltx::DevBuf dn_ws;     // the denoising loop's activations
     size_t ws_T = 0, ws_S = 0;
     int ws_mode = -1;
+    bool ws_planes = true;  // the current mode F32 forward's workspace has room for planes
     int ws_pins = 0;  // live block graphs: their kernels hold workspace addresses
     void* stage_ptr[LTX_ST_COUNT] = {};
     uint64_t stage_bytes[LTX_ST_COUNT] = {};

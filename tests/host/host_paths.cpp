@@ -311,6 +311,34 @@ static void linear_warmed() {
     }
 }
 
+// A mode F32 forward whose planes find no memory, or no room in a workspace that a
+// graph holds, runs on the f32 MFMA kernel; with room again, on the planes.
+static void f32_workspace() {
+    for (bool pinned : {false, true}) {
+        ltx_ctx* c = make_ctx();
+        ltx_block_weights w;
+        fill(w, true);
+        const int T = 20000;
+        // what the forward took before its GEMMs had planes: 13 tensors of T x 4,096,
+        // the FFN's hidden values, the gate logits and the context's, with some air
+        const uint64_t plain = (uint64_t)T * (13 * LTX_D + LTX_FF + 64) * 4 + (64 << 20);
+        if (pinned) {
+            c->ws.alloc(plain);
+            c->ws_pins = 1;
+        } else {
+            fake::limit = fake::in_use + plain;
+        }
+        fake::log.clear();
+        forward(c, w, T, 128, LTX_MODE_F32);
+        CHECK(!launches("ltx_split3") && launches("ltx_gemm_f32"), "planes without room");
+        fake::limit = ~0ull;
+        c->ws_pins = 0;
+        fake::log.clear();
+        forward(c, w, T, 128, LTX_MODE_F32);
+        CHECK(launches("ltx_split3") && !launches("ltx_gemm_f32"), "no planes with room");
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string cmd = argc > 1 ? argv[1] : "";
     auto arg = [&](int i) { return argc > i ? std::atoi(argv[i]) : 0; };
@@ -343,6 +371,8 @@ int main(int argc, char** argv) {
         }
     } else if (cmd == "linear_warmed")
         linear_warmed();
+    else if (cmd == "f32_workspace")
+        f32_workspace();
     else if (cmd == "stage_v")
         stage_v(arg(2), arg(3), arg(4), arg(5));
     else if (cmd == "attn_padded") {  // prints whether V^T is padded, for pairs lq lkv

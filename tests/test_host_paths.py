@@ -33,6 +33,10 @@ def test_f32_block_planes_fit_their_room(host_paths, T, S):
     host_paths("f32_planes", T, S)
 
 
+def test_f32_block_without_room_for_planes(host_paths):
+    host_paths("f32_workspace")
+
+
 @pytest.mark.parametrize("scratch", ["planes", "vt"])
 def test_operator_scratch_is_ordered(host_paths, scratch):
     """Calls that share a context's operator scratch (mode F32's planes, the
