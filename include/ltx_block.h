@@ -211,7 +211,8 @@ int ltx_range_count(ltx_ctx* ctx, void* stream, uint64_t* count, int reset);
  * odd multiple of 128) the weights as bytes q + 128. Two calls of one context on
  * different streams may overwrite that scratch, so keep one context's calls on
  * one stream. Mode F32 with N a multiple of 128 splits a into three bf16 planes
- * in context scratch of at most 512 MiB (as many rows at a time as fit); calls on different streams are ordered behind each other's
+ * in context scratch of at most 512 MiB (as many rows at a time as fit; values of
+ * a below 2^-110 keep what of them is at least 2^-133); calls on different streams are ordered behind each other's
  * use of it. A call being captured, or one that finds no memory for it, takes no
  * scratch for planes or partial sums. In the 16-bit modes it then sums the same
  * products in another order (no split of K); in mode F32 it runs the f32 MFMA
