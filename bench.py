@@ -28,7 +28,7 @@ sys.path.insert(0, str(ROOT))
 
 D, H, HD, FF = 4096, 32, 128, 16384
 PEAK_TFLOPS = 2500.0  # MI355X dense bf16/fp16 MFMA
-PEAK_F32_TFLOPS = 157.3  # MI355X fp32 (the f32 mode's kernels are SIMT f32)
+PEAK_F32_TFLOPS = 157.3  # MI355X fp32 (mode f32's attention; its GEMMs, on bf16 MFMAs over planes, pass it)
 # HBM bytes per self-attention launch, by (tokens, operand type): rocprofv3
 # FETCH_SIZE x 2.0 (the factor a 1 GiB copy calibrates) + WRITE_SIZE x 1.0,
 # measured on this kernel (profiles/block_t28672_hbm_bytes.md); None for a
